@@ -1,0 +1,337 @@
+"""Workloads of the ILU0-BiCGSTAB solver, for timing.
+
+A simulator's Newton step hands the solver new matrix values on a fixed
+pattern, factorises and solves once; an adjoint run solves with the transposed
+system and takes the gradient on the block pattern.  The cases are these calls
+through the public Python entry points, from a grid of a few hundred cells,
+where launches and latencies count, to the 128x128x64 grids, where memory
+bandwidth does, with 3x3 and 4x4 blocks, in FP64 and in the precision form,
+with the greedy colouring and with level scheduling, on device and on host
+arrays.  Every system comes from the package's own grid generator.
+
+Kinds of a case:
+  newton  new values, factorisation, one solve
+  solve   one more right-hand side on a factored system
+  train   DifferentiableSolver: forward solve, backward solve, gradients
+  spmv    one matrix-vector product on device vectors
+"""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import torch
+
+from fpga_amd.solver import BicgstabSolver, GridSpec, generate
+
+MAXIT = 1000
+
+
+def _case(name, kind, nx, ny, nz, bs=3, form="fp64", tol=1e-6, hard=True, host=False, level=False, warm=False):
+    """hard: wide permeability contrast, inactive cells and non-neighbour
+    connections (the generator settings of the 128x128x64 workload); else a
+    regular grid (those of the 32x32x16 one).  form: fp64, or mixed (the
+    precision form).  host: values, right-hand side and solution are host
+    arrays.  warm: the solve starts from a non-zero vector."""
+    c = dict(kind=kind, nx=nx, ny=ny, nz=nz, bs=bs, form=form, tol=tol, hard=hard, host=host, level=level, warm=warm)
+    if name:
+        c["name"] = name
+    return c
+
+
+def listed():
+    return [
+        # a sector model or a well test: the whole step is launches and latency
+        _case("newton-tiny", "newton", 12, 11, 5, tol=1e-2),
+        # the CPU-runnable parity workload, at a simulator's usual linear tolerance
+        _case("newton-small", "newton", 32, 32, 16, tol=1e-2, hard=False),
+        # the same grid in the precision form, to a tight tolerance
+        _case("newton-small-mixed", "newton", 32, 32, 16, form="mixed", hard=False),
+        # a ragged mid-size field model driven as the reference's caller drives it: host arrays in and out
+        _case("newton-host-ragged", "newton", 61, 53, 27, tol=1e-2, host=True),
+        # the headline single-GPU workload in FP64: one more right-hand side
+        _case("solve-large", "solve", 128, 128, 64),
+        # the headline workload as a simulator runs it, in the precision form
+        _case("newton-large-mixed", "newton", 128, 128, 64, form="mixed"),
+        # four equations per cell (thermal, polymer, solvent runs): the 256x256x64 workload
+        _case("newton-bs4-largest", "newton", 256, 256, 64, bs=4, form="mixed"),
+        # four equations per cell, ragged, FP64, started from the last step's solution
+        _case("newton-bs4-warm", "newton", 75, 66, 41, bs=4, warm=True),
+        # the adjoint workload: history matching, forward and backward to 1e-10
+        _case("train-mid", "train", 64, 64, 32, tol=1e-10, hard=False),
+        # the same with 4x4 blocks on a ragged grid in the precision form
+        _case("train-bs4-mixed", "train", 37, 41, 19, bs=4, form="mixed", tol=1e-8),
+        # level scheduling: fewer iterations, one small launch per level
+        _case("newton-level", "newton", 48, 48, 24, level=True),
+        # the bare operator, FP64
+        _case("spmv-mid", "spmv", 96, 96, 48),
+    ]
+
+
+def draw(rng):
+    def size(lo, hi):
+        return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+    kind = rng.choice(["newton"] * 5 + ["solve", "train", "spmv"])
+    nx, ny, nz = size(8, 128), size(8, 128), size(4, 64)
+    bs = rng.choice([3, 3, 4])
+    form = rng.choice(["fp64", "mixed"])
+    tol = rng.choice([1e-8, 1e-10]) if kind == "train" else rng.choice([1e-2, 1e-4, 1e-6])
+    level = kind == "newton" and rng.random() < 0.15
+    if kind == "train" or level:
+        nx, ny, nz = min(nx, 64), min(ny, 64), min(nz, 32)
+    return _case(None, kind, nx, ny, nz, bs, form, tol, hard=rng.random() < 0.6,
+                 host=kind == "newton" and rng.random() < 0.25, level=level,
+                 warm=kind in ("newton", "solve") and rng.random() < 0.3)
+
+
+def _system(case, seed):
+    """The case's grid (the same for every seed) with the values and the
+    right-hand side of one time step: every row scaled, as a time step scales
+    it, and the couplings a little weaker than the generator's."""
+    wide = dict(perm_sigma=2.0, layer_corr=0.5, inactive_frac=0.10, nnc_frac=0.01, nnc_dist=3) if case["hard"] else {}
+    s = generate(GridSpec(case["nx"], case["ny"], case["nz"], bs=case["bs"], seed=0, **wide))
+    gen = torch.Generator().manual_seed(seed)
+    counts = torch.from_numpy(np.diff(s.rowptr).astype(np.int64))
+    rows = torch.repeat_interleave(torch.arange(s.n), counts)
+    f = 1.0 - 0.02 * torch.rand(s.nnzb, generator=gen, dtype=torch.float64)
+    f[torch.from_numpy(s.colidx).long() == rows] = 1.0
+    f *= torch.exp2(2.0 * torch.rand(s.n, generator=gen, dtype=torch.float64) - 1.0)[rows]
+    torch.from_numpy(s.values).mul_(f[:, None, None])
+    torch.from_numpy(s.b).uniform_(-1.0, 1.0, generator=gen)
+    return s
+
+
+class _State:
+    pass
+
+
+def prepare(case, seed):
+    """The handle with its pattern analysed, and the step's inputs."""
+    s = _system(case, seed)
+    rng = np.random.default_rng(seed)
+    st = _State()
+    st.case, st.N = case, s.N
+    dev = torch.device("cuda:0")
+    if case["kind"] == "train":
+        from fpga_amd.autograd import DifferentiableSolver
+        st.solver = DifferentiableSolver(s.bs, s.rowptr, s.colidx, s.values)
+        st.values = torch.from_numpy(s.values).to(dev).requires_grad_(True)
+        st.b = torch.from_numpy(s.b).to(dev).requires_grad_(True)
+        st.w = torch.from_numpy(rng.standard_normal(s.N)).to(dev)
+        return st
+    st.solver = BicgstabSolver(s.bs, s.n, s.nnzb)
+    st.solver.upload_system(s)
+    st.solver.analyse(case["level"])
+    if case["kind"] == "spmv":
+        st.fp32 = case["form"] == "mixed"
+        st.solver.factor()  # the FP32 copies of the matrix belong to a factored system
+        if st.fp32:
+            st.solver.prepare_mixed()
+        # the operator works in the solver's own row order
+        dt = np.float32 if st.fp32 else np.float64
+        st.x = torch.from_numpy(_spmv_input(case, seed, s.N).astype(dt)).to(dev)
+        st.y = torch.empty_like(st.x)
+        return st
+    if case["kind"] == "solve":
+        st.solver.factor()
+        if case["form"] == "mixed":
+            st.solver.prepare_mixed()
+    x0 = 0.1 * rng.standard_normal(s.N) if case["warm"] else np.zeros(s.N)
+    if case["host"]:
+        st.values, st.b, st.x0 = s.values, s.b, x0
+    else:
+        st.values = torch.from_numpy(s.values).to(dev)
+        st.b = torch.from_numpy(s.b).to(dev)
+        st.x0 = torch.from_numpy(x0).to(dev)
+        st.x = torch.empty_like(st.b)
+    return st
+
+
+def run(st):
+    case, g = st.case, st.solver
+    tol, mixed = case["tol"], case["form"] == "mixed"
+    if case["kind"] == "train":
+        st.values.grad = st.b.grad = None
+        x = g(st.values, st.b, tol=tol, maxit=MAXIT, adj_tol=tol, adj_maxit=MAXIT, precision_form=mixed)
+        (x * st.w).sum().backward()
+        return {"x": x.detach(), "grad_values": st.values.grad, "grad_b": st.b.grad}
+    if case["kind"] == "spmv":
+        g.spmv_dev(st.x.data_ptr(), st.y.data_ptr(), prec=1 if st.fp32 else 0)
+        return st.y
+    if case["host"]:
+        g.update_values(st.values)
+        g.factor()
+        x, _ = g.solve_mixed(st.b, st.x0, tol=tol, inner_maxit=MAXIT) if mixed else g.solve(st.b, st.x0, tol, MAXIT)
+        return x
+    if case["kind"] == "newton":
+        g.update_values_dev(st.values.data_ptr())
+        g.factor()
+    st.x.copy_(st.x0)
+    if mixed:
+        g.solve_mixed_dev(st.b.data_ptr(), st.x.data_ptr(), tol, inner_maxit=MAXIT)
+    else:
+        g.solve_dev(st.b.data_ptr(), st.x.data_ptr(), tol, MAXIT)
+    return st.x
+
+
+def _sizes(case):
+    """Block rows and blocks of the case's system, nearly."""
+    nx, ny, nz = case["nx"], case["ny"], case["nz"]
+    keep = 0.9 if case["hard"] else 1.0
+    n = keep * nx * ny * nz
+    faces = (nx - 1) * ny * nz + nx * (ny - 1) * nz + nx * ny * (nz - 1)
+    return n, n + 2 * faces * keep * keep
+
+
+def _iterations(case):
+    """Iterations of a typical solve of the case's size and tolerance."""
+    digits = -math.log10(case["tol"])
+    side = (case["nx"] * case["ny"] * case["nz"]) ** (1 / 3)
+    return max(1.0, digits * ((2.3 + 0.025 * side) if case["hard"] else (0.8 + 0.022 * side)))
+
+
+def work(case):
+    """A solve reads, in each half-iteration, the matrix once for the product
+    and once more what the preconditioner adds to it: the lower factor (half
+    of the off-diagonal blocks) and the diagonal's inverses; the upper factor
+    of a first colour's rows is the matrix's own.  11 vector passes go with it.
+    The step around the solve reads the values and writes the factors once."""
+    n, nnzb = _sizes(case)
+    bb, bs = case["bs"] ** 2, case["bs"]
+    N = n * bs
+    f = 4 if case["form"] == "mixed" else 8
+    off = nnzb - n
+    if case["kind"] == "spmv":
+        return {"bytes": nnzb * (bb * f + 4) + 4 * n + 2 * N * f, "flops": 2 * nnzb * bb}
+    half_bytes = (nnzb + 0.5 * off) * (bb * f + 4) + n * bb * 8 + 11 * N * f
+    half_flops = 2 * bb * (nnzb + off + n) + 20 * N
+    solve = 2 * _iterations(case)
+    total_b, total_f = solve * half_bytes + 2 * N * 8, solve * half_flops
+    if case["kind"] == "train":
+        total_b, total_f = 2 * total_b + nnzb * bb * 8, 2 * total_f + nnzb * bb
+    if case["kind"] != "solve":
+        total_b += (nnzb + off + n) * bb * 8
+        total_f += off * bb * bs * 4 + n * bb * bs * 4
+    return {"bytes": total_b, "flops": total_f}
+
+
+def _spmv_input(case, seed, N):
+    return np.random.default_rng(seed + 1).standard_normal(N)
+
+
+def _colour_order(s):
+    """First-fit greedy colouring in row order on the symmetrised pattern; the
+    rows of a colour keep their order."""
+    n = s.n
+    rows = np.repeat(np.arange(n), np.diff(s.rowptr))
+    i = np.concatenate([rows, s.colidx])
+    j = np.concatenate([s.colidx, rows])
+    m = j < i
+    order = np.argsort(i[m], kind="stable")
+    i, j = i[m][order], j[m][order]
+    ptr = np.searchsorted(i, np.arange(n + 1)).tolist()
+    j = j.tolist()
+    colour = [0] * n
+    for r in range(n):
+        used = {colour[k] for k in j[ptr[r]:ptr[r + 1]]}
+        c = 0
+        while c in used:
+            c += 1
+        colour[r] = c
+    return np.argsort(np.array(colour), kind="stable")
+
+
+def _product(s, x):
+    """A x in the generator's row order, 64 bits."""
+    bs = s.bs
+    y = np.zeros((s.n, bs))
+    x = x.reshape(s.n, bs)
+    for k0 in range(0, s.n, 65536):
+        k1 = min(k0 + 65536, s.n)
+        q0, q1 = s.rowptr[k0], s.rowptr[k1]
+        p = np.einsum("qrc,qc->qr", s.values[q0:q1], x[s.colidx[q0:q1]])
+        y[k0:k1] = np.add.reduceat(p, s.rowptr[k0:k1] - q0, axis=0)
+    return y.reshape(-1)
+
+
+def _scalar_rows(s, transpose):
+    """The matrix as a torch CSR tensor of scalars, and its inverse block diagonal."""
+    bs = s.bs
+    rows = np.repeat(np.arange(s.n), np.diff(s.rowptr))
+    cols = s.colidx.astype(np.int64)
+    vals = s.values
+    diag = np.linalg.inv(vals[cols == rows])
+    if transpose:
+        rows, cols, vals, diag = cols, rows, vals.transpose(0, 2, 1), diag.transpose(0, 2, 1)
+        order = np.argsort(rows, kind="stable")
+        rows, cols, vals = rows[order], cols[order], vals[order]
+    k = np.arange(bs)
+    i = np.broadcast_to((rows * bs)[:, None, None] + k[:, None], vals.shape).reshape(-1)
+    j = np.broadcast_to((cols * bs)[:, None, None] + k, vals.shape).reshape(-1)
+    a = torch.sparse_coo_tensor(torch.from_numpy(np.stack([i, j])), torch.from_numpy(vals.reshape(-1).copy()),
+                                (s.N, s.N)).to_sparse_csr()
+    return a, torch.from_numpy(np.ascontiguousarray(diag))
+
+
+def _solution(s, rhs, transpose=False):
+    """A x = rhs to rounding, by plain BiCGSTAB with the inverse block diagonal
+    on the CPU, restarted from its own residual; None if it gets stuck."""
+    a, d = _scalar_rows(s, transpose)
+    n, bs = s.n, s.bs
+    b = torch.from_numpy(rhs)
+
+    def m(v):
+        return torch.bmm(d, v.view(n, bs, 1)).view(-1)
+
+    x, nb = torch.zeros_like(b), torch.linalg.vector_norm(b)
+    for _ in range(4):
+        r0 = b - a @ x
+        if torch.linalg.vector_norm(r0) <= 1e-14 * nb:
+            break
+        r, p, e, rho = r0, r0, torch.zeros_like(b), r0 @ r0
+        goal = 1e-8 * torch.linalg.vector_norm(r0)
+        for _ in range(500):
+            ph = m(p)
+            v = a @ ph
+            alpha = rho / (r0 @ v)
+            t0 = r - alpha * v
+            sh = m(t0)
+            t = a @ sh
+            om = (t @ t0) / (t @ t)
+            e = e + alpha * ph + om * sh
+            r = t0 - om * t
+            if not torch.linalg.vector_norm(r) > goal:
+                break
+            rho, old = r0 @ r, rho
+            p = r + (rho / old) * (alpha / om) * (p - om * v)
+        x = x + e
+    done = torch.linalg.vector_norm(b - a @ x) <= 1e-12 * nb
+    return x.numpy() if done else None
+
+
+def exact(case, seed):
+    """The product in 64 bits; a solution to rounding where the system is
+    small enough for a solver this plain: None for the larger ones."""
+    n, nnzb = _sizes(case)
+    if case["kind"] == "spmv":
+        s = _system(case, seed)
+        perm = _colour_order(s)
+        x = _spmv_input(case, seed, s.N)
+        if case["form"] == "mixed":
+            x = x.astype(np.float32).astype(np.float64)
+        xo = np.empty((s.n, s.bs))
+        xo[perm] = x.reshape(s.n, s.bs)
+        return _product(s, xo.reshape(-1)).reshape(s.n, s.bs)[perm].reshape(-1)
+    if nnzb * case["bs"] ** 2 > 3e7:
+        return None
+    s = _system(case, seed)
+    x = _solution(s, s.b)
+    if case["kind"] != "train":
+        return x
+    lam = _solution(s, np.random.default_rng(seed).standard_normal(s.N), transpose=True)
+    if x is None or lam is None:
+        return None
+    rows = np.repeat(np.arange(s.n), np.diff(s.rowptr))
+    grad = -lam.reshape(s.n, s.bs)[rows][:, :, None] * x.reshape(s.n, s.bs)[s.colidx][:, None, :]
+    return {"x": x, "grad_values": grad, "grad_b": lam}
