@@ -188,7 +188,7 @@ def _iterations(case):
     """Iterations of a typical solve of the case's size and tolerance."""
     digits = -math.log10(case["tol"])
     side = (case["nx"] * case["ny"] * case["nz"]) ** (1 / 3)
-    return max(1.0, digits * ((2.3 + 0.025 * side) if case["hard"] else (0.8 + 0.022 * side)))
+    return max(1.0, digits * ((2.6 + 0.009 * side) if case["hard"] else (0.8 + 0.022 * side)))
 
 
 def work(case):
