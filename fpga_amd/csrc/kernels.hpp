@@ -21,6 +21,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include <type_traits>
@@ -573,7 +574,27 @@ __global__ __launch_bounds__(256) void k_copy_check_finite(int64_t n, const doub
 // merged tail (k_tail3) follows: rows without blocks in the second sweep
 // also get z = D^-1 y there, computed from y as stored (rounded to the
 // vector type), which is what the second sweep would compute for them.
-enum StreamMode : int { SM_SPMV = 0, SM_SUB = 1, SM_SUB_DINV = 2, SM_SUB_Z = 3 };
+//
+// SM_SUB_SPMV is the second sweep of colour 0 and the product v = A z of the
+// same rows in one pass, for factors whose colour-0 rows of U are A's own
+// blocks (block ILU0 changes nothing in a row without earlier neighbours).
+// In A such a row holds its diagonal block first (every other column belongs
+// to a later colour), so the row partials q of the streamed U blocks serve
+// both sums:
+//   z_i = D_i^-1 (rhs_i - (((0 + q_1) + q_2) + ..)),
+//   v_i = ((0 + A_ii z_i) + q_1) + q_2 + ..,
+// each in the order, and with the roundings, of the separate launches: z, v
+// and the fused dots are the same bit for bit.  Its tiles are the product's
+// (the same rows, so the same reduction slots) with U's blocks; A_ii comes
+// from a packed copy (adiag), since streaming A's rows and reading their
+// diagonal blocks a second time fetched 100 MB more (the blocks no longer in
+// the L2; 66 instead of 50 us).  It is HBM-bound like the launches it stands
+// for, and saves the second read of half of A's off-diagonal blocks.  On a
+// 128x128x64 3x3 grid a half-iteration's colour-0 sweep and product took 41.4
+// + 93.0 us (FP32: 22.7 + 50.7) and take 50.2 + 52.0 us (26.8 + 29.0) as this
+// launch and the other colours' product; the FP64 solve 12.6 -> 11.0 ms, a
+// 4x4 256x256x64 precision-form step 44.6 -> 40.2 ms.
+enum StreamMode : int { SM_SPMV = 0, SM_SUB = 1, SM_SUB_DINV = 2, SM_SUB_Z = 3, SM_SUB_SPMV = 4 };
 
 template <typename TV, typename TX>
 struct StreamArgs {
@@ -596,6 +617,8 @@ struct StreamArgs {
     const int32_t *rowptr2 = nullptr;  // SUB_Z: the second sweep's row pointers
     TX *zout = nullptr;                // SUB_Z: z of the rows without second-sweep blocks
     const int32_t *rowmap = nullptr;   // dependency tiles (k_lower2): matrix row of each packed row
+    const TV *adiag = nullptr;         // SUB_SPMV: A's diagonal blocks of colour 0
+    TX *vout = nullptr;                // SUB_SPMV: v = A out of the tile's rows
 };
 
 template <typename TV, typename TX>
@@ -657,11 +680,12 @@ template <> struct TileCap<3, true> { static constexpr int value = 336; };   // 
 template <> struct TileCap<4, true> { static constexpr int value = 256; };
 
 // Which tiling a kernel instance uses: the wide one in the modes whose bit is
-// set in BDA_WIDE_MODES (the SpMV, in both precisions), the narrow one
+// set in BDA_WIDE_MODES (the SpMV and SUB_SPMV, whose rows share their
+// reduction slots, in both precisions), the narrow one
 // otherwise (the sweeps: with wide tiles their register and LDS use cuts the
 // resident workgroups, and the FP32 sweeps lose more than they gain).
 #ifndef BDA_WIDE_MODES
-#define BDA_WIDE_MODES 1
+#define BDA_WIDE_MODES 17
 #endif
 template <int MODE> constexpr bool wide_tiles() { return ((BDA_WIDE_MODES >> MODE) & 1) != 0; }
 template <int BS, int MODE> constexpr int stream_cap() { return TileCap<BS, wide_tiles<MODE>()>::value; }
@@ -781,8 +805,17 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
     int32_t *scol = lds.scol;
     int32_t *srow = lds.srow;
     double *tv = tile_tv<(MODE == SM_SUB_DINV || MODE == SM_SUB_Z) ? RS * NT : 1>();
+    if constexpr (MODE == SM_SUB_SPMV) {
+        // its 2 * NT row values take the place of the x entries, which every
+        // lane has read by the barrier before the row sums
+        static_assert(sizeof(lds.sx) >= 2 * NT * sizeof(double) && offsetof(std::decay_t<decltype(lds)>, sx) % 8 == 0,
+                      "row values fit the x entries' place");
+        tv = reinterpret_cast<double *>(lds.sx);
+    }
 
     static_assert(!KEEP || ROWS == 64, "kept outputs: one row per thread");
+    static_assert(MODE != SM_SUB_SPMV || (ROWS == 64 && !KEEP && V == 0 && wide_tiles<SM_SPMV>() == wide_tiles<MODE>()),
+                  "sweep and product: the product's tiles, one row per thread");
     const int r0 = d.x, r1 = d.z, b0 = d.y;
     const int nblk = d.w - b0;
     const int nrow = r1 - r0;
@@ -844,6 +877,7 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
     size_t gi[RS];
     double rhs_v[RS], w_v[RS];
     double dv[RS][BS];
+    TV dg[BS];  // SUB_SPMV: row r of the row's diagonal block
     bool zrow[RS];
 #pragma unroll
     for (int s = 0; s < RS; ++s) {
@@ -861,7 +895,11 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
             rhs_v[s] = (double)a.rhs[gi[s]];
         }
         if constexpr ((RED & SR_W0) != 0) w_v[s] = (double)a.w0[gi[s]];
-        if constexpr (MODE == SM_SUB_DINV || MODE == SM_SUB_Z) {
+        if constexpr (MODE == SM_SUB_SPMV) {
+#pragma unroll
+            for (int c = 0; c < BS; ++c) dg[c] = a.adiag[gi[s] * BS + c];
+        }
+        if constexpr (MODE == SM_SUB_DINV || MODE == SM_SUB_Z || MODE == SM_SUB_SPMV) {
             const double *D = a.dinv + gi[s] * BS;
 #pragma unroll
             for (int c = 0; c < BS; ++c) dv[s][c] = D[c];
@@ -932,38 +970,47 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
             if (ok) part[j] = sm;
         }
     } else if constexpr (LAY == LAY_PAIR) {
-#pragma unroll
-        for (int u = 0; u < NS; ++u) {
-            const int q = (u * NW + wave) * PPW + lane;
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                const int en = 2 * q + c;
-                xs[u][c] = sx[min(en / BB, CAP - 1) * BS + en % BS];
-            }
-        }
         // 3x3: lanes 3k, 3k+1, 3k+2 hold entries 6k'..6k'+5, two block rows;
         // lane 3k adds row 2k' (its two products, then the next lane's
         // first), lane 3k+1 row 2k'+1 (its second product, then the next
         // lane's two).  4x4: lane 2k adds its two products, then the next
         // lane's two.  Each is ((p0 + p1) + p2) [+ p3], the entry lanes' order.
+        // SUB_SPMV goes through the slots in two steps, so that only half the
+        // x entries are held beside its values and row operands (90 instead
+        // of 106 VGPRs, 5 instead of 4 waves per SIMD); the product, at 5
+        // waves with all of them, is 1-2 us slower in steps.
+        constexpr int kPairStep = MODE == SM_SUB_SPMV ? (NS + 1) / 2 : NS;
 #pragma unroll
-        for (int u = 0; u < NS; ++u) {
-            const int q = (u * NW + wave) * PPW + lane;
-            const double pa = prod<TV, TX>(av[u][0], xs[u][0]);
-            const double pb = prod<TV, TX>(av[u][1], xs[u][1]);
-            const double na = lane_down1(pa);
-            const double nb = lane_down1(pb);
-            int row;
-            double sm;
-            if constexpr (BS == 3) {
-                const int m = lane % 3;
-                row = m == 0 ? 2 * q / 3 : m == 1 ? (2 * q + 1) / 3 : -1;
-                sm = m == 0 ? (pa + pb) + na : (pb + na) + nb;
-            } else {
-                row = (lane & 1) == 0 ? q / 2 : -1;
-                sm = ((pa + pb) + na) + nb;
+        for (int u0 = 0; u0 < NS; u0 += kPairStep) {
+#pragma unroll
+            for (int u = u0; u < NS && u < u0 + kPairStep; ++u) {
+                const int q = (u * NW + wave) * PPW + lane;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const int en = 2 * q + c;
+                    xs[u][c] = sx[min(en / BB, CAP - 1) * BS + en % BS];
+                }
             }
-            if (lane < PPW && row >= 0 && row < nblk * BS) part[row] = sm;
+#pragma unroll
+            for (int u = u0; u < NS && u < u0 + kPairStep; ++u) {
+                const int q = (u * NW + wave) * PPW + lane;
+                const double pa = prod<TV, TX>(av[u][0], xs[u][0]);
+                const double pb = prod<TV, TX>(av[u][1], xs[u][1]);
+                const double na = lane_down1(pa);
+                const double nb = lane_down1(pb);
+                int row;
+                double sm;
+                if constexpr (BS == 3) {
+                    const int m = lane % 3;
+                    row = m == 0 ? 2 * q / 3 : m == 1 ? (2 * q + 1) / 3 : -1;
+                    sm = m == 0 ? (pa + pb) + na : (pb + na) + nb;
+                } else {
+                    row = (lane & 1) == 0 ? q / 2 : -1;
+                    sm = ((pa + pb) + na) + nb;
+                }
+                if (lane < PPW && row >= 0 && row < nblk * BS) part[row] = sm;
+            }
+            if constexpr (kPairStep < NS) __builtin_amdgcn_sched_barrier(0);
         }
     } else {
 #pragma unroll
@@ -1029,13 +1076,36 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
             }
         }
     }
+    if constexpr (MODE == SM_SUB_SPMV) {
+        tv[t] = res[0];
+        __syncthreads();
+        double z = 0.0;
+#pragma unroll
+        for (int c = 0; c < BS; ++c) z += dv[0][c] * tv[k0 * BS + c];
+        const TX zo = from_double<TX>(z);
+        tv[NT + t] = (double)zo;
+        if (has_row[0]) a.out[gi[0]] = zo;
+        __syncthreads();
+        if (has_row[0]) {
+            TX zr[BS];
+#pragma unroll
+            for (int c = 0; c < BS; ++c) zr[c] = (TX)tv[NT + k0 * BS + c];
+            double sm = prod<TV, TX>(dg[0], zr[0]);
+#pragma unroll
+            for (int c = 1; c < BS; ++c) sm = sm + prod<TV, TX>(dg[c], zr[c]);
+            double sum = 0.0 + sm;
+            for (int q = srow[k0]; q < srow[k0 + 1]; ++q) sum += part[q * BS + r];
+            res[0] = sum;
+        }
+    }
     double red[2] = {0.0, 0.0};
 #pragma unroll
     for (int s = 0; s < RS; ++s) {
         if (!has_row[s]) continue;
         const TX o = from_double<TX>(res[s]);
         if constexpr (KEEP) keep[t] = o;
-        if constexpr (V != 1) {
+        if constexpr (MODE == SM_SUB_SPMV) a.vout[gi[s]] = o;
+        else if constexpr (V != 1) {
             a.out[gi[s]] = o;
             if (a.out2) a.out2[gi[s]] = o;
             if (a.out3) a.out3[gi[s]] = o;

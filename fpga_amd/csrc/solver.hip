@@ -72,6 +72,13 @@ struct DevMat {
     DBuf<int32_t> slot, slot_sp, slot_wide, slot_wide_sp, slot_tall;
     std::vector<int32_t> colour_tile, colour_tile_wide, colour_tile_tall;
     int ntiles_wide = 0;
+    // the whole-matrix wide list without colour 0's tiles (the rest of a
+    // product whose colour-0 rows the second sweep's launch has computed),
+    // and colour 0's wide tiles, in tile_wide's order, with the block ranges
+    // of the second sweep's pattern (that launch)
+    DBuf<int4> tile_wide_rest, tile_wide_sweep;
+    DBuf<int32_t> slot_wide_rest;
+    int ntiles_wide_rest = 0;
     // rows of colour C-2 that carry blocks (for the merged tail launch of a
     // second sweep), when there are at most kTailRows of them; else -1
     DBuf<int32_t> tail_dep;
@@ -145,7 +152,9 @@ struct DevMat {
     static void upload_tiles(const MatPattern &p, const std::vector<int32_t> &tile_row,
                              const std::vector<int32_t> &colour_tile, const std::vector<int32_t> *orig_row,
                              int64_t L, DBuf<int4> &out, DBuf<int32_t> &out_slot, DBuf<int4> *out_sp,
-                             DBuf<int32_t> *out_sp_slot, hipStream_t s) {
+                             DBuf<int32_t> *out_sp_slot, hipStream_t s, DBuf<int4> *out_rest = nullptr,
+                             DBuf<int32_t> *out_rest_slot = nullptr, const MatPattern *sweep = nullptr,
+                             DBuf<int4> *out_sweep = nullptr) {
         const int nt = (int)tile_row.size() - 1;
         std::vector<int4> d(std::max(nt, 1), make_int4(0, 0, 0, 0));
         for (int t = 0; t < nt; ++t)
@@ -193,13 +202,36 @@ struct DevMat {
             HIP_CHECK(hipMemcpyAsync(out_sp->p, ds.data(), ds.size() * sizeof(int4), hipMemcpyHostToDevice, s));
             HIP_CHECK(hipMemcpyAsync(out_sp_slot->p, sls.data(), sls.size() * 4, hipMemcpyHostToDevice, s));
         }
+        std::vector<int4> dr, dw;
+        std::vector<int32_t> slr;
+        if (out_sweep) {
+            for (int t = 0; t < colour_tile[1]; ++t)
+                dw.push_back(make_int4(d[t].x, sweep->rowptr[d[t].x], d[t].z, sweep->rowptr[d[t].z]));
+            out_sweep->ensure(std::max<size_t>(dw.size(), 1));
+            HIP_CHECK(hipMemcpyAsync(out_sweep->p, dw.data(), dw.size() * sizeof(int4), hipMemcpyHostToDevice, s));
+        }
+        if (out_rest) {
+            for (int t = 0; t < nt; ++t)
+                if (sls[t] >= colour_tile[1]) {
+                    dr.push_back(ds[t]);
+                    slr.push_back(sls[t]);
+                }
+            out_rest->ensure(std::max<size_t>(dr.size(), 1));
+            out_rest_slot->ensure(std::max<size_t>(slr.size(), 1));
+            if (!dr.empty()) {
+                HIP_CHECK(hipMemcpyAsync(out_rest->p, dr.data(), dr.size() * sizeof(int4), hipMemcpyHostToDevice, s));
+                HIP_CHECK(hipMemcpyAsync(out_rest_slot->p, slr.data(), slr.size() * 4, hipMemcpyHostToDevice, s));
+            }
+        }
         HIP_CHECK(hipStreamSynchronize(s));
     }
 
     // orig_row: original row of every (permuted) row, and span: the
     // matrix's coupling_span, for the launch order of the tiles
+    // sweep: the second sweep's pattern, where its colour 0 may run with the
+    // product's
     void upload(const MatPattern &p, hipStream_t s, const std::vector<int32_t> *orig_row = nullptr,
-                int64_t span = 0) {
+                int64_t span = 0, const MatPattern *sweep = nullptr) {
         n = p.n;
         nnzb = p.nnzb();
         ntiles = p.ntiles();
@@ -217,7 +249,9 @@ struct DevMat {
             HIP_CHECK(hipMemcpyAsync(src.p, p.src.data(), p.src.size() * 4, hipMemcpyHostToDevice, s));
         upload_tiles(p, p.tile_row, p.colour_tile, orig_row, span, tile, slot, &tile_sp, &slot_sp, s);
         upload_tiles(p, p.tile_row_wide, p.colour_tile_wide, orig_row, span, tile_wide, slot_wide, &tile_wide_sp,
-                     &slot_wide_sp, s);
+                     &slot_wide_sp, s, sweep ? &tile_wide_rest : nullptr, sweep ? &slot_wide_rest : nullptr, sweep,
+                     sweep ? &tile_wide_sweep : nullptr);
+        ntiles_wide_rest = sweep ? ntiles_wide - colour_tile_wide[1] : 0;
         upload_tiles(p, p.tile_row_tall, p.colour_tile_tall, orig_row, span, tile_tall, slot_tall, nullptr, nullptr,
                      s);
     }
@@ -470,7 +504,9 @@ struct DevMat {
         tile_wide.release();
         tile_wide_sp.release();
         tile_tall.release();
-        for (DBuf<int32_t> *b : {&slot, &slot_sp, &slot_wide, &slot_wide_sp, &slot_tall}) b->release();
+        for (DBuf<int32_t> *b : {&slot, &slot_sp, &slot_wide, &slot_wide_sp, &slot_tall, &slot_wide_rest}) b->release();
+        tile_wide_rest.release();
+        tile_wide_sweep.release();
         tail_dep.release();
         for (DBuf<int32_t> *b : {&tail3_row, &tail3_blk, &tail3_src}) b->release();
         tail3_tile.release();
@@ -507,6 +543,7 @@ struct OpSet {
     const TV *S2val;
     bool s2_dinv;
     const double *dinv;
+    const TV *adiag = nullptr;  // A's diagonal blocks of colour 0, packed
 };
 
 enum ProfKind { PK_SPMV = 0, PK_LOWER = 1, PK_UPPER = 2, PK_VEC = 3, PK_N = 4 };
@@ -524,6 +561,12 @@ enum ProfKind { PK_SPMV = 0, PK_LOWER = 1, PK_UPPER = 2, PK_VEC = 3, PK_N = 4 };
 #endif
 #ifndef BDA_LOW2
 #define BDA_LOW2 1
+#endif
+// 1 (default): the second sweep's colour 0 and the product's colour-0 rows in
+// one launch where the factors allow it; 0: the separate launches (the same
+// results, for A/B timing)
+#ifndef BDA_FUSE0
+#define BDA_FUSE0 1
 #endif
 // 1 (default): k_finalize_joint for 2,049 to 18,432 partials; 0: k_finalize
 // (the same sums, for A/B timing)
@@ -552,6 +595,8 @@ struct bda_handle_s {
     bda::DBuf<int32_t> d_nonfinite;  // set by the factorisation when a matrix value is infinite or NaN
     bda::DBuf<double> d_orig, A64, L64, U64, LU, Dinv, DinvT, At64, Ut64, Lt64;
     bda::DBuf<float> A32, L32, U32;
+    bda::DBuf<double> A0d64;  // A's diagonal blocks of colour 0, packed (SM_SUB_SPMV)
+    bda::DBuf<float> A0d32;
     bda::DBuf<double> low2_v64;  // values of L's packed dependency rows (k_lower2)
     bda::DBuf<float> low2_v32;
     bda::DBuf<float> At32, Ut32, Lt32;  // FP32 transposes (component access only)
@@ -561,6 +606,10 @@ struct bda_handle_s {
     // (k_lower2) where the colouring allows them
     bool tail3 = BDA_TAIL3 != 0;
     bool low2 = BDA_LOW2 != 0;
+    // U's colour-0 rows are A's own blocks: true of factors made by
+    // bda_factor, not known of a caller's own (bda_upload_factored)
+    bool u0_is_a = false;
+    bool fuse0 = BDA_FUSE0 != 0;  // the second sweep of colour 0 with the product's (SM_SUB_SPMV)
 
     // vectors
     bda::Krylov<double> k64;
@@ -751,6 +800,11 @@ int stream_dispatch(H &h, const StreamArgs<TV, TX> &a) {
 // finalize) is bracketed by an event pair of that kind.
 // ZX: a step-0 residual that takes the short path when k_mark_nonzero left
 // the state's full_residual clear (zero start vector, finite matrix).
+// colour kRestOfRows (the product only): every colour but the first, whose
+// rows' partial sums launch_sweep_spmv has left in their slots.
+constexpr int kRestOfRows = -2;
+static_assert(wide_tiles<SM_SPMV>(), "the list without colour 0 is built of wide tiles");
+
 template <int BS, int MODE, int RED, typename TV, typename TX, bool ZX = false>
 void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x, const TX *rhs, TX *out,
                    const double *dinv, const TX *w0, RedArgs ra, bool use_state, TX *out2 = nullptr,
@@ -762,7 +816,12 @@ void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x
     const std::vector<int32_t> &ct = wide ? m.colour_tile_wide : m.colour_tile;
     a.tile = colour < 0 ? (wide ? m.tile_wide_sp.p : m.tile_sp.p) : (wide ? m.tile_wide.p : m.tile.p);
     a.slot = colour < 0 ? (wide ? m.slot_wide_sp.p : m.slot_sp.p) : (wide ? m.slot_wide.p : m.slot.p);
-    if (colour < 0) {
+    if (MODE == SM_SPMV && colour == kRestOfRows) {
+        a.tile = m.tile_wide_rest.p;
+        a.slot = m.slot_wide_rest.p;
+        a.tile0 = 0;
+        a.ntiles = m.ntiles_wide_rest;
+    } else if (colour < 0) {
         a.tile0 = 0;
         a.ntiles = wide ? m.ntiles_wide : m.ntiles;
     } else {
@@ -824,7 +883,37 @@ void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x
         nparts = stream_dispatch<BS, MODE, RED, TV, TX, kTileRows, ZX>(h, a);
     }
     if (prof_kind >= 0) prof_end(h);
+    if (MODE == SM_SPMV && colour == kRestOfRows) nparts = m.ntiles_wide;
     if (nred > 0) launch_finalize(h, nred, a.ra, nparts);
+}
+
+// The second sweep of colour 0 and the product's colour-0 rows in one launch
+// (SM_SUB_SPMV): z of colour 0, v = A z there, and the fused dots' partial
+// sums of its tiles.
+template <int BS, int RED, typename TV, typename TX>
+void launch_sweep_spmv(H &h, const OpSet<TV> &op, const TX *rhs, TX *z, TX *v, const TX *w0, RedArgs ra) {
+    const DevMat &m = *op.A;
+    StreamArgs<TV, TX> a;
+    std::memset(&a, 0, sizeof(a));
+    a.tile = m.tile_wide_sweep.p;
+    a.slot = m.slot_wide.p;
+    a.tile0 = 0;
+    a.ntiles = m.colour_tile_wide[1] - m.colour_tile_wide[0];
+    a.rowptr = op.S2->rowptr.p;
+    a.colidx = op.S2->colidx.p;
+    a.val = op.S2val;
+    a.x = z;
+    a.x_lo = z;
+    a.rhs = rhs;
+    a.out = z;
+    a.vout = v;
+    a.dinv = op.dinv;
+    a.adiag = op.adiag;
+    a.w0 = w0;
+    a.ra = ra;
+    if (!a.adiag) throw std::runtime_error("no diagonal blocks for the merged sweep and product");
+    if (m.ntiles_wide > a.ra.cap) throw std::runtime_error("partials buffer too small");
+    stream_dispatch<BS, SM_SUB_SPMV, RED, TV, TX>(h, a);
 }
 
 template <int BS, typename TV, typename TX>
@@ -1063,8 +1152,10 @@ template <> const float *low2_values<float>(H &h) { return h.low2_v32.p; }
 // When the last colour is a single tile and few rows of colour C-2 have
 // second-sweep blocks, that launch and the second sweep's colour C-2 launch
 // are one (tail_launch).
+// skip_last: everything but the second sweep's colour 0 (launch_sweep_spmv
+// follows).
 template <int BS, typename TV, typename TX>
-void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, bool use_state) {
+void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, bool use_state, bool skip_last = false) {
     const int nc = h.an.ncolours;
     if (op.s1_dinv && op.s2_dinv) throw std::runtime_error("at most one sweep may carry the diagonal inverse");
     const bool skip0 = !op.s1_dinv && nc > 1;
@@ -1072,7 +1163,8 @@ void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, bool use_stat
     const int split = skip0 ? h.an.colour_ptr[1] : 0;
     const bool merge = nc >= 3 && op.S2->tail_ndep >= 0 &&
                        op.S1->colour_tile[nc] - op.S1->colour_tile[nc - 1] == 1;
-    const bool merge3 = merge && h.tail3 && !op.s1_dinv && op.s2_dinv && op.S2->tail3_n >= 0;
+    // (with three colours the extended tail would cover colour 0)
+    const bool merge3 = merge && h.tail3 && !op.s1_dinv && op.s2_dinv && op.S2->tail3_n >= 0 && !(skip_last && nc == 3);
     const bool low2 = h.low2 && skip0 && op.S1->low2_n >= 0 && nc >= 4 && op.S1 == &h.L;
     prof_begin(h, PK_LOWER);
     for (int c = skip0 ? 1 : 0; c < nc - 1; ++c) {
@@ -1093,7 +1185,7 @@ void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, bool use_stat
     prof_begin(h, PK_UPPER);
     if (merge3) tail3_launch<BS, TV, TX>(h, op, y, lo, split, p, z, (nc - 3 == 0 && skip0) ? p : y, use_state);
     else if (merge) tail_launch<BS, TV, TX>(h, op, y, lo, split, p, z, use_state);
-    for (int c = merge3 ? nc - 4 : merge ? nc - 3 : nc - 2; c >= 0; --c)
+    for (int c = merge3 ? nc - 4 : merge ? nc - 3 : nc - 2; c >= (skip_last ? 1 : 0); --c)
         sweep_launch<BS, TV, TX>(h, *op.S2, op.S2val, c, op.s2_dinv, z, nullptr, 0, (c == 0 && skip0) ? p : y, z,
                                  op.dinv, use_state);
     prof_end(h);
@@ -1117,6 +1209,21 @@ int precond_launches(const H &h, const OpSet<TV> &op) {
     if (merge || merge3) k += 1;
     for (int c = merge3 ? nc - 4 : merge ? nc - 3 : nc - 2; c >= 0; --c) k += nonempty(*op.S2, c);
     return k;
+}
+
+// Whether a solve runs the second sweep's colour 0 together with the
+// product's (SM_SUB_SPMV).  Not for the transposed operators (the second
+// sweep is L^T, whose colour-0 blocks are A's times D^-1) and not for a
+// caller's own factors.  Where the launches are latency-bound the longer
+// kernel costs what it saves: us per FP64 iteration, separate / merged, by
+// colour-0 tiles, 3x3: 72.5 / 73.8 (170), 87.4 / 88.8 (575), 120.8 / 115.4
+// (1365), 192 / 173 (2666); 4x4: 71.4 / 71.5, 95.9 / 93.7, 150.7 / 136.9,
+// 248 / 213.
+constexpr int kFuseFrom = 640;
+template <typename TV>
+bool fuse_sweep_spmv(const H &h, const OpSet<TV> &op) {
+    return h.fuse0 && h.u0_is_a && op.A == &h.A && op.S2 == &h.U && !op.s1_dinv && op.s2_dinv && h.an.ncolours > 1 &&
+           op.A->colour_tile_wide[1] >= kFuseFrom;
 }
 
 struct RunOut {
@@ -1237,6 +1344,24 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     // of one half at most (ahead = 1), while the device still has that
     // preconditioner queued whenever the host waits.
     bool stop = false;
+    const bool fuse = fuse_sweep_spmv(h, op);
+    // z = M^-1 p, and, fused, the colour-0 rows of v = A z with their dots
+    auto apply = [&](auto redc, const TX *p, TX *z, TX *v, const TX *w0, int fin) {
+        constexpr int RED = decltype(redc)::value;
+        precond<BS, TV, TX>(h, op, p, k.y.p, z, true, fuse);
+        if (fuse) {
+            prof_begin(h, PK_UPPER);
+            launch_sweep_spmv<BS, RED, TV, TX>(h, op, p, z, v, w0, red(h, 0, fin));
+            prof_end(h);
+        }
+    };
+    auto product = [&](auto redc, const TX *z, TX *v, const TX *w0, int fin) {
+        constexpr int RED = decltype(redc)::value;
+        launch_stream<BS, SM_SPMV, RED, TV, TX>(h, *op.A, op.Aval, fuse ? kRestOfRows : -1, z, nullptr, v, nullptr,
+                                                w0, red(h, 0, fin), true, nullptr, nullptr, nullptr, 0, PK_SPMV);
+    };
+    constexpr std::integral_constant<int, SR_W0> red_w0{};
+    constexpr std::integral_constant<int, SR_BOTH> red_both{};
     const int ahead = std::min(3, std::max(1, h.poll_iters));
     const int ahead_h = 2 * ahead - 1;
     auto throttle = [&](int half) {
@@ -1255,11 +1380,10 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     };
     for (int it = 1; it <= maxit + 1 && !stop; ++it) {
         h.prof_tag = 2 * (it - 1);
-        precond<BS, TV, TX>(h, op, k.p.p, k.y.p, k.phat.p, true);
+        apply(red_w0, k.p.p, k.phat.p, k.v.p, k.rt.p, FIN_ALPHA);
         throttle(2 * it - 1);
         if (stop) break;
-        launch_stream<BS, SM_SPMV, SR_W0, TV, TX>(h, *op.A, op.Aval, -1, k.phat.p, nullptr, k.v.p, nullptr, k.rt.p,
-                                                  red(h, 0, FIN_ALPHA), true, nullptr, nullptr, nullptr, 0, PK_SPMV);
+        product(red_w0, k.phat.p, k.v.p, k.rt.p, FIN_ALPHA);
         prof_begin(h, PK_VEC);
         hipLaunchKernelGGL((k_update_s<TX>), dim3(vb), dim3(kVecThreads), 0, h.stream, (int64_t)N, k.r.p, k.v.p,
                            k.s.p, red(h, 0, FIN_HALF1));
@@ -1267,11 +1391,10 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
         launch_finalize(h, 1, red(h, 0, FIN_HALF1), vb);
         prof_end(h);
         h.prof_tag = 2 * (it - 1) + 1;
-        precond<BS, TV, TX>(h, op, k.s.p, k.y.p, k.shat.p, true);
+        apply(red_both, k.s.p, k.shat.p, k.t.p, k.s.p, FIN_OMEGA);
         throttle(2 * it);
         if (stop) break;
-        launch_stream<BS, SM_SPMV, SR_BOTH, TV, TX>(h, *op.A, op.Aval, -1, k.shat.p, nullptr, k.t.p, nullptr, k.s.p,
-                                                    red(h, 0, FIN_OMEGA), true, nullptr, nullptr, nullptr, 0, PK_SPMV);
+        product(red_both, k.shat.p, k.t.p, k.s.p, FIN_OMEGA);
         prof_begin(h, PK_VEC);
         hipLaunchKernelGGL((k_update_xr<TX, TX>), dim3(vb), dim3(kVecThreads), 0, h.stream, (int64_t)N, k.x.p,
                            k.phat.p, k.shat.p, k.s.p, k.t.p, k.r.p, k.rt.p, red(h, 0, FIN_HALF2));
@@ -1350,7 +1473,7 @@ void log_analysis(H &h);
 void finish_analyse(H &h) {
     const Analysis &an = h.an;
     const int64_t span = DevMat::coupling_span(an.A, an.perm);
-    h.A.upload(an.A, h.stream, &an.perm, span);
+    h.A.upload(an.A, h.stream, &an.perm, span, &an.U);
     h.L.upload(an.L, h.stream, &an.perm, span);
     h.U.upload(an.U, h.stream, &an.perm, span);
     h.At.upload(an.At, h.stream, &an.perm, span);
@@ -1450,8 +1573,13 @@ void do_factor(H &h) {
     gather_blocks<BS, double>(h, h.U.nnzb, h.U.src.p, h.LU.p, h.U64.p, 0);
     gather_blocks<BS, double>(h, h.n, nullptr, h.Dinv.p, h.DinvT.p, 1);
     gather_low2<BS>(h);
+    if (h.an.ncolours > 1) {
+        h.A0d64.ensure((size_t)h.an.colour_ptr[1] * BB);
+        gather_blocks<BS, double>(h, h.an.colour_ptr[1], h.d_diag.p, h.A64.p, h.A0d64.p, 0);
+    }
     HIP_CHECK(hipStreamSynchronize(h.stream));
     h.factored = true;
+    h.u0_is_a = true;
     h.factor_gen++;
     h.values_gen++;
 }
@@ -1478,6 +1606,7 @@ void load_factors(H &h, const double *lu_values, const double *dinv) {
     gather_low2<BS>(h);
     HIP_CHECK(hipStreamSynchronize(h.stream));
     h.factored = true;
+    h.u0_is_a = false;
     h.factor_gen++;
     h.values_gen++;
 }
@@ -1496,6 +1625,10 @@ void ensure_mixed(H &h) {
     if (h.L.low2_n >= 0) {
         h.low2_v32.ensure((h.L.low2_nvblk + kPadBlocks) * bb);
         gather_blocks<BS, float>(h, h.L.low2_nvblk, nullptr, h.low2_v64.p, h.low2_v32.p, 0);
+    }
+    if (h.u0_is_a && h.an.ncolours > 1) {
+        h.A0d32.ensure((size_t)h.an.colour_ptr[1] * bb);
+        gather_blocks<BS, float>(h, h.an.colour_ptr[1], nullptr, h.A0d64.p, h.A0d32.p, 0);
     }
     HIP_CHECK(hipStreamSynchronize(h.stream));
     h.mixed_gen = h.factor_gen;
@@ -1535,10 +1668,10 @@ void ensure_adjoint32(H &h) {
 }
 
 OpSet<double> op_fwd64(H &h) {
-    return OpSet<double>{&h.A, h.A64.p, &h.L, h.L64.p, false, &h.U, h.U64.p, true, h.Dinv.p};
+    return OpSet<double>{&h.A, h.A64.p, &h.L, h.L64.p, false, &h.U, h.U64.p, true, h.Dinv.p, h.A0d64.p};
 }
 OpSet<float> op_fwd32(H &h) {
-    return OpSet<float>{&h.A, h.A32.p, &h.L, h.L32.p, false, &h.U, h.U32.p, true, h.Dinv.p};
+    return OpSet<float>{&h.A, h.A32.p, &h.L, h.L32.p, false, &h.U, h.U32.p, true, h.Dinv.p, h.A0d32.p};
 }
 OpSet<double> op_adj64(H &h) {
     return OpSet<double>{&h.At, h.At64.p, &h.Ut, h.Ut64.p, true, &h.Lt, h.Lt64.p, false, h.DinvT.p};
@@ -2060,10 +2193,10 @@ int bda_destroy(bda_handle h) {
     for (DevMat *m : {&h->A, &h->L, &h->U, &h->At, &h->Ut, &h->Lt}) m->release();
     for (DBuf<int32_t> *b : {&h->d_perm, &h->d_diag, &h->d_blkrow, &h->d_bad}) b->release();
     for (DBuf<double> *b : {&h->d_orig, &h->A64, &h->L64, &h->U64, &h->LU, &h->Dinv, &h->DinvT, &h->At64, &h->Ut64,
-                            &h->Lt64, &h->bp, &h->xo, &h->ro, &h->vin, &h->vout, &h->vw, &h->gl, &h->gx, &h->ggrad,
+                            &h->Lt64, &h->A0d64, &h->low2_v64, &h->bp, &h->xo, &h->ro, &h->vin, &h->vout, &h->vw, &h->gl, &h->gx, &h->ggrad,
                             &h->partials})
         b->release();
-    for (DBuf<float> *b : {&h->A32, &h->L32, &h->U32, &h->At32, &h->Ut32, &h->Lt32}) b->release();
+    for (DBuf<float> *b : {&h->A32, &h->L32, &h->U32, &h->A0d32, &h->low2_v32, &h->At32, &h->Ut32, &h->Lt32}) b->release();
     h->k64.release();
     h->k32.release();
     h->st.release();
