@@ -537,16 +537,12 @@ __global__ __launch_bounds__(kFinGroupThreads) void k_finalize_stage1(RedArgs ra
     }
 }
 
-// dst = src (n doubles); *nonfinite = 1 when a value is infinite or NaN.
-// Every writer stores the same value.
-__global__ __launch_bounds__(256) void k_copy_check_finite(int64_t n, const double *src, double *dst,
-                                                           int32_t *nonfinite) {
+// *nonfinite = 1 when one of n values is infinite or NaN.  Every writer stores
+// the same value.
+__global__ __launch_bounds__(256) void k_check_finite(int64_t n, const double *src, int32_t *nonfinite) {
     bool bad = false;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const double v = src[i];
-        dst[i] = v;
-        bad = bad || !finite(v);
-    }
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        bad = bad || !finite(src[i]);
     if (bad) __hip_atomic_store(nonfinite, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -1719,24 +1715,54 @@ __global__ void k_scatter_rows(int n, int bs, const int32_t *perm, const double 
 }
 
 // dst block k = src block idx[k] (idx null: identity), optionally transposed
-// and converted (K17 demotion when TD = float).
+// and converted (K17 demotion when TD = float).  A workgroup writes
+// kGatherUnroll * 256 consecutive entries, each thread entries 256 apart: all
+// its index loads are in flight together, then all its value loads.  With one
+// entry per thread and a 64-bit division for each, 6.0M 3x3 blocks took 211 us
+// (4.1 TB/s) and 24M 4x4 blocks 1520 us, the two dependent loads leaving too
+// few bytes in flight; now 171 (5.1 TB/s) and 1150 us (5.4 TB/s).
+constexpr int kGatherUnroll = 8;
 template <int BS, typename TD>
-__global__ void k_gather_blocks(int64_t nblk, const int32_t *idx, const double *src, TD *dst, int trans) {
+__global__ __launch_bounds__(256) void k_gather_blocks(int64_t nblk, const int32_t *idx, const double *src, TD *dst,
+                                                       int trans) {
+    constexpr int BB = BS * BS, U = kGatherUnroll;
+    const int64_t i0 = (int64_t)blockIdx.x * (256 * U);
+    const int64_t k0 = i0 / BB;
+    const int rem = (int)(i0 - k0 * BB) + threadIdx.x;
+    const int64_t left = (nblk - k0) * BB;      // entries from block k0 on
+    const int last = (int)(left < 256 * U + BB ? left : 256 * U + BB) - 1;
+    int64_t s[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int k = min(rem + u * 256, last) / BB;
+        s[u] = idx ? (int64_t)idx[k0 + k] : k0 + k;
+    }
+    double v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int l = min(rem + u * 256, last), e = l - l / BB * BB;
+        v[u] = src[s[u] * BB + (trans ? e % BS * BS + e / BS : e)];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (rem + u * 256 <= last) dst[k0 * BB + rem + u * 256] = (TD)v[u];
+}
+
+// dst block idx[k] = src block k (the inverse of k_gather_blocks' copy)
+template <int BS>
+__global__ __launch_bounds__(256) void k_scatter_blocks(int64_t nblk, const int32_t *idx, const double *src,
+                                                        double *dst) {
     constexpr int BB = BS * BS;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= nblk * BB) return;
     const int64_t k = i / BB;
-    const int e = (int)(i - k * BB);
-    const int er = e / BS, ec = e - er * BS;
-    const int se = trans ? ec * BS + er : e;
-    const int64_t s = idx ? (int64_t)idx[k] : k;
-    dst[i] = (TD)src[s * BB + se];
+    dst[(int64_t)idx[k] * BB + (i - k * BB)] = src[i];
 }
 
 // ---------------------------------------------------------------------------
-// Block ILU0, one thread per block row of one colour (rows of a colour are
-// not coupled, so they factorise independently once all earlier colours are
-// done).  IKJ order on the colour-ordered matrix:
+// Block ILU0 of one colour's rows (rows of a colour are not coupled, so they
+// factorise independently once all earlier colours are done).  IKJ order on
+// the colour-ordered matrix:
 //   for each L block (i,k), k ascending:  L_ik = A_ik * Dinv_k
 //       for each U block (k,j) of row k:   A_ij -= L_ik * U_kj   if (i,j) in pattern
 //   Dinv_i = inverse of the updated A_ii (Gauss-Jordan, partial pivoting)
@@ -1795,59 +1821,213 @@ __device__ inline bool invert_block(const double *a, double *inv) {
     return true;
 }
 
-// out = a * b for BS x BS row-major blocks, entries summed over m ascending
-template <int BS>
-__device__ inline void block_mul(const double *a, const double *b, double *out) {
-#pragma unroll
-    for (int r = 0; r < BS; ++r)
-#pragma unroll
-        for (int c = 0; c < BS; ++c) {
-            double s = a[r * BS + 0] * b[0 * BS + c];
-#pragma unroll
-            for (int m = 1; m < BS; ++m) s = s + a[r * BS + m] * b[m * BS + c];
-            out[r * BS + c] = s;
+// What an L block of the pattern updates, by A's block index: the U block of
+// row k whose column is the row itself (the usual case, one block: the
+// diagonal), kUpdNone when nothing in the row is updated, kUpdRow when other
+// blocks are (the row of U is then searched).  A blocks outside L: kUpdNone.
+constexpr int32_t kUpdNone = -1, kUpdRow = -2;
+__global__ __launch_bounds__(256) void k_ilu0_updates(int64_t nnzb, const int32_t *blkrow, const int32_t *rowptr,
+                                                      const int32_t *colidx, const int32_t *u_rowptr,
+                                                      const int32_t *u_colidx, int32_t *upd) {
+    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (q >= nnzb) return;
+    const int i = blkrow[q], k = colidx[q];
+    int32_t v = kUpdNone;
+    if (k < i) {
+        const int rend = rowptr[i + 1];
+        int qi = (int)q + 1;
+        for (int p = u_rowptr[k]; p < u_rowptr[k + 1] && v != kUpdRow; ++p) {
+            const int j = u_colidx[p];
+            if (j == i) {
+                v = p;
+                continue;
+            }
+            while (qi < rend && colidx[qi] < j) ++qi;
+            if (qi < rend && colidx[qi] == j) v = kUpdRow;
         }
+    }
+    upd[q] = v;
 }
 
+// One workgroup (BS lanes per row) factorises the rows of one wide tile of A:
+// the tile's blocks are read once, in order, into LDS; lane (row, r) owns
+// component row r of every block of its row, so the whole elimination needs
+// no exchange between lanes; one lane per row inverts the diagonal block; and
+// L, U, D^-1, and the FP32 copies where the precision form is in use (the
+// float pointers, else null), are written from LDS, again in order.  On the
+// way it records non-finite values of A and copies colour 0's diagonal
+// blocks (adiag).  One thread per row instead, in place on a copy of A that
+// was gathered into L and U afterwards, read and wrote each 72- or 128-byte
+// block from one lane (64 cache lines per load) with a chain of dependent
+// loads per block: on a 128x128x64 3x3 grid copy 147 us, elimination 766,
+// gathers 220, FP32 copies 250; now 420 us with the FP32 copies (colour 0, a
+// stream with an inversion, 5.1 TB/s; colour 1, bound by the latency of its
+// D^-1 and U block reads, 4.1 TB/s), and 2.4 instead of 7.4 ms on a 4x4
+// 256x256x64 grid.  The last colours' few tiles take 17-22 us each, a chain
+// of one load latency per L block, against 41-64.
 template <int BS>
-__global__ void k_bilu0_rows(int row0, int row1, const int32_t *rowptr, const int32_t *colidx,
-                             const int32_t *diag, double *LU, double *dinv, int32_t *bad_row) {
-    constexpr int BB = BS * BS;
-    const int i = row0 + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= row1) return;
-    const int rend = rowptr[i + 1], di = diag[i];
-    for (int q = rowptr[i]; q < di; ++q) {
-        const int kk = colidx[q];
-        double a[BB], d[BB], l[BB];
+struct IluArgs {
+    const int4 *tile;
+    int32_t tile0, ntiles;
+    const int32_t *rowptr, *colidx, *upd;    // A's pattern; update of each L block
+    const int32_t *l_rowptr, *u_rowptr, *u_colidx;
+    const double *val;                       // A
+    double *l, *u, *dinv, *adiag;
+    float *a32, *l32, *u32, *adiag32;
+    int32_t *bad_row, *nonfinite;
+};
+
+template <int BS>
+__global__ __launch_bounds__(64 * BS) void k_ilu0_tile(IluArgs<BS> a) {
+    constexpr int BB = BS * BS, NT = 64 * BS, CAP = TileCap<BS, true>::value;
+    constexpr int S = (CAP * BB + NT - 1) / NT;
+    __shared__ double sa[CAP * BB];
+    __shared__ int32_t scol[CAP], supd[CAP], sdst[CAP];
+    __shared__ int32_t srow[kTileRows + 1], slrow[kTileRows + 1], surow[kTileRows + 1];
+    const int4 d = a.tile[a.tile0 + xcd_tile(blockIdx.x, a.ntiles)];
+    const int r0 = d.x, b0 = d.y, nrow = d.z - d.x, nblk = d.w - d.y;
+    const int t = threadIdx.x;
+
+    // the tile's blocks (clamped loads, all in flight together)
+    const double *val = a.val + (size_t)b0 * BB;
+    const int nval = nblk * BB;
+    double v[S];
 #pragma unroll
-        for (int e = 0; e < BB; ++e) { a[e] = LU[(size_t)q * BB + e]; d[e] = dinv[(size_t)kk * BB + e]; }
-        block_mul<BS>(a, d, l);
+    for (int u = 0; u < S; ++u) v[u] = val[min(u * NT + t, nval - 1)];
+    for (int j = t; j < nblk; j += NT) {
+        scol[j] = a.colidx[b0 + j];
+        supd[j] = a.upd[b0 + j];
+    }
+    if (t <= nrow) {
+        srow[t] = a.rowptr[r0 + t] - b0;
+        slrow[t] = a.l_rowptr[r0 + t];
+        surow[t] = a.u_rowptr[r0 + t];
+    }
+    bool bad = false;
 #pragma unroll
-        for (int e = 0; e < BB; ++e) LU[(size_t)q * BB + e] = l[e];
-        int qi = q + 1;
-        for (int pk = diag[kk] + 1; pk < rowptr[kk + 1]; ++pk) {
-            const int j = colidx[pk];
-            while (qi < rend && colidx[qi] < j) ++qi;
-            if (qi >= rend) break;
-            if (colidx[qi] != j) continue;
-            double u[BB], t[BB];
-#pragma unroll
-            for (int e = 0; e < BB; ++e) u[e] = LU[(size_t)pk * BB + e];
-            block_mul<BS>(l, u, t);
-#pragma unroll
-            for (int e = 0; e < BB; ++e) LU[(size_t)qi * BB + e] = LU[(size_t)qi * BB + e] - t[e];
+    for (int u = 0; u < S; ++u) {
+        const int e = u * NT + t;
+        if (e < nval) {
+            sa[e] = v[u];
+            bad = bad || !finite(v[u]);
+            if (a.a32) a.a32[(size_t)b0 * BB + e] = (float)v[u];
         }
     }
-    double dd[BB], inv[BB];
+    if (bad) __hip_atomic_store(a.nonfinite, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+
+    // where each block goes: L block index, -2 - U block index, -1 the diagonal
+    if (t < nrow) {
+        const int s0 = srow[t], nl = slrow[t + 1] - slrow[t], n = srow[t + 1] - s0;
+        for (int m = 0; m < n; ++m)
+            sdst[s0 + m] = m < nl ? slrow[t] + m : m == nl ? -1 : -2 - (surow[t] + m - nl - 1);
+    }
+    const int k0 = t / BS, r = t - k0 * BS;
+    if (k0 < nrow) {
+        const int i = r0 + k0, s0 = srow[k0], nl = slrow[k0 + 1] - slrow[k0], sd = s0 + nl;
+        double dd[BS];
 #pragma unroll
-    for (int e = 0; e < BB; ++e) dd[e] = LU[(size_t)di * BB + e];
-    if (!invert_block<BS>(dd, inv)) {
-        atomicMin(bad_row, i);
+        for (int c = 0; c < BS; ++c) dd[c] = sa[sd * BB + r * BS + c];
+        if (a.adiag) {
 #pragma unroll
-        for (int e = 0; e < BB; ++e) inv[e] = 0.0;
+            for (int c = 0; c < BS; ++c) {
+                a.adiag[(size_t)i * BB + r * BS + c] = dd[c];
+                if (a.adiag32) a.adiag32[(size_t)i * BB + r * BS + c] = (float)dd[c];
+            }
+        }
+        for (int m = 0; m < nl; ++m) {
+            const int k = scol[s0 + m], up = supd[s0 + m];
+            double dk[BB], uk[BB];
+            const double *dp = a.dinv + (size_t)k * BB, *upp = a.u + (size_t)max(up, 0) * BB;
+#pragma unroll
+            for (int e = 0; e < BB; ++e) dk[e] = dp[e];
+            if (up >= 0) {
+#pragma unroll
+                for (int e = 0; e < BB; ++e) uk[e] = upp[e];
+            }
+            double *ar = &sa[(s0 + m) * BB + r * BS];
+            double av[BS], l[BS];
+#pragma unroll
+            for (int c = 0; c < BS; ++c) av[c] = ar[c];
+#pragma unroll
+            for (int c = 0; c < BS; ++c) {
+                double s = av[0] * dk[c];
+#pragma unroll
+                for (int q = 1; q < BS; ++q) s = s + av[q] * dk[q * BS + c];
+                l[c] = s;
+            }
+#pragma unroll
+            for (int c = 0; c < BS; ++c) ar[c] = l[c];
+            if (up >= 0) {
+#pragma unroll
+                for (int c = 0; c < BS; ++c) {
+                    double s = l[0] * uk[c];
+#pragma unroll
+                    for (int q = 1; q < BS; ++q) s = s + l[q] * uk[q * BS + c];
+                    dd[c] = dd[c] - s;
+                }
+            } else if (up == kUpdRow) {
+                int qi = s0 + m + 1;
+                const int rend = srow[k0 + 1];
+                for (int p = a.u_rowptr[k]; p < a.u_rowptr[k + 1]; ++p) {
+                    const int j = a.u_colidx[p];
+                    while (qi < rend && scol[qi] < j) ++qi;
+                    if (qi >= rend) break;
+                    if (scol[qi] != j) continue;
+                    double s[BS];
+#pragma unroll
+                    for (int c = 0; c < BS; ++c) {
+                        s[c] = l[0] * a.u[(size_t)p * BB + c];
+#pragma unroll
+                        for (int q = 1; q < BS; ++q) s[c] = s[c] + l[q] * a.u[(size_t)p * BB + q * BS + c];
+                    }
+                    if (qi == sd) {
+#pragma unroll
+                        for (int c = 0; c < BS; ++c) dd[c] = dd[c] - s[c];
+                    } else {
+                        double *tr = &sa[qi * BB + r * BS];
+#pragma unroll
+                        for (int c = 0; c < BS; ++c) tr[c] = tr[c] - s[c];
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < BS; ++c) sa[sd * BB + r * BS + c] = dd[c];
+    }
+    __syncthreads();
+    if (t < nrow) {
+        const int sd = srow[t] + slrow[t + 1] - slrow[t];
+        double dd[BB], inv[BB];
+#pragma unroll
+        for (int e = 0; e < BB; ++e) dd[e] = sa[sd * BB + e];
+        if (!invert_block<BS>(dd, inv)) {
+            atomicMin(a.bad_row, r0 + t);
+#pragma unroll
+            for (int e = 0; e < BB; ++e) inv[e] = 0.0;
+        }
+#pragma unroll
+        for (int e = 0; e < BB; ++e) sa[sd * BB + e] = inv[e];
+    }
+    __syncthreads();
+    for (int e = t; e < nrow * BB; e += NT) {
+        const int k = e / BB;
+        a.dinv[(size_t)r0 * BB + e] = sa[(srow[k] + slrow[k + 1] - slrow[k]) * BB + e - k * BB];
     }
 #pragma unroll
-    for (int e = 0; e < BB; ++e) dinv[(size_t)i * BB + e] = inv[e];
+    for (int u = 0; u < S; ++u) {
+        const int e = u * NT + t;
+        if (e >= nval) break;
+        const int j = e / BB, ent = e - j * BB, to = sdst[j];
+        const double x = sa[e];
+        if (to >= 0) {
+            a.l[(size_t)to * BB + ent] = x;
+            if (a.l32) a.l32[(size_t)to * BB + ent] = (float)x;
+        } else if (to < -1) {
+            a.u[(size_t)(-2 - to) * BB + ent] = x;
+            if (a.u32) a.u32[(size_t)(-2 - to) * BB + ent] = (float)x;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------

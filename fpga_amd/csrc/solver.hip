@@ -585,13 +585,15 @@ struct bda_handle_s {
 
     // host copies
     bda::Bcsr pattern;
+    bool orig_current = false;  // d_orig holds the current values (else only A64 does)
     bool have_pattern = false, analysed = false, factored = false, have_values = false;
     bda::Analysis an;
     std::vector<int32_t> blkrow;  // block row of every permuted A block
 
     // device matrices
     bda::DevMat A, L, U, At, Ut, Lt;
-    bda::DBuf<int32_t> d_perm, d_diag, d_blkrow, d_bad;
+    bda::DBuf<int32_t> d_perm, d_blkrow, d_bad;
+    bda::DBuf<int32_t> d_upd;  // what each L block updates in the factorisation (k_ilu0_updates)
     bda::DBuf<int32_t> d_nonfinite;  // set by the factorisation when a matrix value is infinite or NaN
     bda::DBuf<double> d_orig, A64, L64, U64, LU, Dinv, DinvT, At64, Ut64, Lt64;
     bda::DBuf<float> A32, L32, U32;
@@ -600,6 +602,11 @@ struct bda_handle_s {
     bda::DBuf<double> low2_v64;  // values of L's packed dependency rows (k_lower2)
     bda::DBuf<float> low2_v32;
     bda::DBuf<float> At32, Ut32, Lt32;  // FP32 transposes (component access only)
+    // the precision form has been used: the factorisation then writes its FP32
+    // copies beside the FP64 values (copies_gen: the factorisation whose
+    // values they hold; mixed_gen: the one they were last asked for)
+    bool mixed_used = false;
+    uint64_t copies_gen = UINT64_MAX;
     uint64_t factor_gen = 0, mixed_gen = UINT64_MAX, adj_gen = UINT64_MAX, adj32_gen = UINT64_MAX;
     uint64_t values_gen = 0;  // changes with every upload, value update and factorisation
     // the extended merged tail launch (k_tail3) and the merged lower launch
@@ -1455,15 +1462,41 @@ template <int BS, typename TD>
 void gather_blocks(H &h, int64_t nblk, const int32_t *idx, const double *src, TD *dst, int trans) {
     if (nblk <= 0) return;
     const int64_t work = nblk * BS * BS;
-    hipLaunchKernelGGL((k_gather_blocks<BS, TD>), dim3(blocks_for(work, 256)), dim3(256), 0, h.stream, nblk, idx,
+    hipLaunchKernelGGL((k_gather_blocks<BS, TD>), dim3(blocks_for(work, 256 * kGatherUnroll)), dim3(256), 0, h.stream, nblk, idx,
                        src, dst, trans);
     check_launch();
 }
 
+// A's values in colour order from d_values in the caller's block order
 template <int BS>
-void permute_values(H &h) {
-    gather_blocks<BS, double>(h, h.A.nnzb, h.A.src.p, h.d_orig.p, h.A64.p, 0);
+void permute_values(H &h, const double *d_values) {
+    gather_blocks<BS, double>(h, h.A.nnzb, h.A.src.p, d_values, h.A64.p, 0);
     HIP_CHECK(hipStreamSynchronize(h.stream));
+}
+
+// Whether a kernel may read bytes at p: memory of this device, within one
+// allocation.  (Other pointers go through a copy, which reports its own
+// errors and reaches other devices.)
+bool readable_here(const H &h, const void *p, size_t bytes) {
+    hipPointerAttribute_t at;
+    void *base = nullptr;
+    size_t size = 0;
+    if (!p || hipPointerGetAttributes(&at, p) != hipSuccess || at.type != hipMemoryTypeDevice || at.device != h.device ||
+        hipMemGetAddressRange((hipDeviceptr_t *)&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return (size_t)((const char *)p - (const char *)base) + bytes <= size;
+}
+
+// d_orig from A's values, before the analysis that gave their order goes
+template <int BS>
+void restore_values(H &h) {
+    hipLaunchKernelGGL((k_scatter_blocks<BS>), dim3(blocks_for(h.A.nnzb * BS * BS, 256)), dim3(256), 0, h.stream,
+                       h.A.nnzb, h.A.src.p, (const double *)h.A64.p, h.d_orig.p);
+    check_launch();
+    HIP_CHECK(hipStreamSynchronize(h.stream));
+    h.orig_current = true;
 }
 
 // Device side of an analysis held in h.an: patterns, tilings, permutation
@@ -1472,6 +1505,10 @@ void log_analysis(H &h);
 
 void finish_analyse(H &h) {
     const Analysis &an = h.an;
+    if (h.analysed && h.have_values && !h.orig_current) {
+        if (h.bs == 3) restore_values<3>(h);
+        else restore_values<4>(h);
+    }
     const int64_t span = DevMat::coupling_span(an.A, an.perm);
     h.A.upload(an.A, h.stream, &an.perm, span, &an.U);
     h.L.upload(an.L, h.stream, &an.perm, span);
@@ -1484,23 +1521,24 @@ void finish_analyse(H &h) {
     h.L.set_low2(an.L, an.colour_ptr, an.perm, span, h.bs, h.stream);
     h.Lt.set_tail(an.Lt, an.colour_ptr, h.stream);
     h.d_perm.ensure(h.n);
-    h.d_diag.ensure(h.n);
     copy_sync(h, h.d_perm.p, an.perm.data(), h.n * 4, hipMemcpyHostToDevice);
-    copy_sync(h, h.d_diag.p, an.diag.data(), h.n * 4, hipMemcpyHostToDevice);
     h.blkrow.resize(an.A.nnzb());
     for (int k = 0; k < h.n; ++k)
         for (int32_t q = an.A.rowptr[k]; q < an.A.rowptr[k + 1]; ++q) h.blkrow[q] = k;
     h.d_blkrow.ensure(h.blkrow.size());
     copy_sync(h, h.d_blkrow.p, h.blkrow.data(), h.blkrow.size() * 4, hipMemcpyHostToDevice);
+    h.d_upd.ensure(h.blkrow.size());
+    hipLaunchKernelGGL(k_ilu0_updates, dim3(blocks_for((int64_t)h.blkrow.size(), 256)), dim3(256), 0, h.stream,
+                       (int64_t)h.blkrow.size(), h.d_blkrow.p, h.A.rowptr.p, h.A.colidx.p, h.U.rowptr.p,
+                       h.U.colidx.p, h.d_upd.p);
+    check_launch();
 
     const size_t bb = (size_t)h.bs * h.bs;
     const int64_t nnzb = an.A.nnzb();
     h.A64.ensure((nnzb + kPadBlocks) * bb);
-    h.LU.ensure(nnzb * bb);
     h.L64.ensure((an.L.nnzb() + kPadBlocks) * bb);
     h.U64.ensure((an.U.nnzb() + kPadBlocks) * bb);
     h.Dinv.ensure((size_t)h.n * bb);
-    h.DinvT.ensure((size_t)h.n * bb);
     h.d_bad.ensure(1);
     h.d_nonfinite.ensure(1);
     // reduction partials: one slot pair per workgroup of the largest reducing
@@ -1518,8 +1556,8 @@ void finish_analyse(H &h) {
     h.analysed = true;
     h.factored = false;
     if (h.have_values) {
-        if (h.bs == 3) permute_values<3>(h);
-        else permute_values<4>(h);
+        if (h.bs == 3) permute_values<3>(h, h.d_orig.p);
+        else permute_values<4>(h, h.d_orig.p);
     }
     log_analysis(h);
 }
@@ -1528,6 +1566,23 @@ void do_analyse(H &h, bool level) {
     if (!h.have_pattern) throw std::runtime_error("bda_upload_bcsr has not been called");
     analyse(h.pattern, level, h.an);
     finish_analyse(h);
+}
+
+// The precision form's FP32 copies: their buffers, and those of L's packed
+// dependency rows (k_lower2) from the FP64 ones.
+template <int BS>
+void mixed_buffers(H &h) {
+    const size_t bb = (size_t)BS * BS;
+    h.A32.ensure((h.A.nnzb + kPadBlocks) * bb);
+    h.L32.ensure((h.L.nnzb + kPadBlocks) * bb);
+    h.U32.ensure((h.U.nnzb + kPadBlocks) * bb);
+    if (h.an.ncolours > 1) h.A0d32.ensure((size_t)h.an.colour_ptr[1] * bb);
+    if (h.L.low2_n >= 0) h.low2_v32.ensure((h.L.low2_nvblk + kPadBlocks) * bb);
+}
+template <int BS>
+void gather_low2_32(H &h) {
+    if (h.L.low2_n < 0) return;
+    gather_blocks<BS, float>(h, h.L.low2_nvblk, nullptr, h.low2_v64.p, h.low2_v32.p, 0);
 }
 
 // Values of L's packed dependency rows (k_lower2) from L64.
@@ -1548,17 +1603,32 @@ void do_factor(H &h) {
     const auto t0 = std::chrono::steady_clock::now();
     HIP_CHECK(hipMemcpyAsync(h.d_bad.p, &big, 4, hipMemcpyHostToDevice, h.stream));
     HIP_CHECK(hipMemcpyAsync(h.d_nonfinite.p, &zero, 4, hipMemcpyHostToDevice, h.stream));
-    {   // LU = A, recording whether A holds a non-finite value (for the step-0 residual's short path)
-        const int64_t nval = (int64_t)h.A.nnzb * BB;
-        const int grid = (int)std::min<int64_t>(std::max<int64_t>(blocks_for(nval, 256), 1), 8192);
-        hipLaunchKernelGGL(k_copy_check_finite, dim3(grid), dim3(256), 0, h.stream, nval, (const double *)h.A64.p,
-                           h.LU.p, h.d_nonfinite.p);
-        check_launch();
-    }
+    const bool f32 = h.mixed_used;
+    if (f32) mixed_buffers<BS>(h);
+    if (an.ncolours > 1) h.A0d64.ensure((size_t)an.colour_ptr[1] * BB);
+    IluArgs<BS> a;
+    a.tile = h.A.tile_wide.p;
+    a.rowptr = h.A.rowptr.p;
+    a.colidx = h.A.colidx.p;
+    a.upd = h.d_upd.p;
+    a.l_rowptr = h.L.rowptr.p;
+    a.u_rowptr = h.U.rowptr.p;
+    a.u_colidx = h.U.colidx.p;
+    a.val = h.A64.p;
+    a.l = h.L64.p;
+    a.u = h.U64.p;
+    a.dinv = h.Dinv.p;
+    a.a32 = f32 ? h.A32.p : nullptr;
+    a.l32 = f32 ? h.L32.p : nullptr;
+    a.u32 = f32 ? h.U32.p : nullptr;
+    a.bad_row = h.d_bad.p;
+    a.nonfinite = h.d_nonfinite.p;
     for (int c = 0; c < an.ncolours; ++c) {
-        const int r0 = an.colour_ptr[c], r1 = an.colour_ptr[c + 1];
-        hipLaunchKernelGGL((k_bilu0_rows<BS>), dim3(blocks_for(r1 - r0, 128)), dim3(128), 0, h.stream, r0, r1,
-                           h.A.rowptr.p, h.A.colidx.p, h.d_diag.p, h.LU.p, h.Dinv.p, h.d_bad.p);
+        a.tile0 = h.A.colour_tile_wide[c];
+        a.ntiles = h.A.colour_tile_wide[c + 1] - a.tile0;
+        a.adiag = c == 0 && an.ncolours > 1 ? h.A0d64.p : nullptr;
+        a.adiag32 = a.adiag && f32 ? h.A0d32.p : nullptr;
+        hipLaunchKernelGGL((k_ilu0_tile<BS>), dim3(a.ntiles), dim3(64 * BS), 0, h.stream, a);
         check_launch();
     }
     int32_t bad = 0;
@@ -1569,13 +1639,10 @@ void do_factor(H &h) {
                                  " (original row " + std::to_string(an.perm[bad]) + ")");
     bda::info(1, "INFO: factor: block ILU0 of %d block rows over %d colours, %.3f ms", h.n, an.ncolours,
               std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count());
-    gather_blocks<BS, double>(h, h.L.nnzb, h.L.src.p, h.LU.p, h.L64.p, 0);
-    gather_blocks<BS, double>(h, h.U.nnzb, h.U.src.p, h.LU.p, h.U64.p, 0);
-    gather_blocks<BS, double>(h, h.n, nullptr, h.Dinv.p, h.DinvT.p, 1);
     gather_low2<BS>(h);
-    if (h.an.ncolours > 1) {
-        h.A0d64.ensure((size_t)h.an.colour_ptr[1] * BB);
-        gather_blocks<BS, double>(h, h.an.colour_ptr[1], h.d_diag.p, h.A64.p, h.A0d64.p, 0);
+    if (f32) {
+        gather_low2_32<BS>(h);
+        h.copies_gen = h.factor_gen + 1;
     }
     HIP_CHECK(hipStreamSynchronize(h.stream));
     h.factored = true;
@@ -1595,14 +1662,14 @@ void load_factors(H &h, const double *lu_values, const double *dinv) {
     HIP_CHECK(hipMemcpyAsync(h.d_nonfinite.p, &zero, 4, hipMemcpyHostToDevice, h.stream));
     const int64_t nval = (int64_t)h.A.nnzb * BB;
     const int grid = (int)std::min<int64_t>(std::max<int64_t>(blocks_for(nval, 256), 1), 8192);
-    hipLaunchKernelGGL(k_copy_check_finite, dim3(grid), dim3(256), 0, h.stream, nval, (const double *)h.A64.p, h.LU.p,
+    hipLaunchKernelGGL(k_check_finite, dim3(grid), dim3(256), 0, h.stream, nval, (const double *)h.A64.p,
                        h.d_nonfinite.p);
     check_launch();
+    h.LU.ensure((size_t)nval);
     HIP_CHECK(hipMemcpyAsync(h.LU.p, lu_values, (size_t)nval * 8, hipMemcpyHostToDevice, h.stream));
     HIP_CHECK(hipMemcpyAsync(h.Dinv.p, dinv, (size_t)h.n * BB * 8, hipMemcpyHostToDevice, h.stream));
     gather_blocks<BS, double>(h, h.L.nnzb, h.L.src.p, h.LU.p, h.L64.p, 0);
     gather_blocks<BS, double>(h, h.U.nnzb, h.U.src.p, h.LU.p, h.U64.p, 0);
-    gather_blocks<BS, double>(h, h.n, nullptr, h.Dinv.p, h.DinvT.p, 1);
     gather_low2<BS>(h);
     HIP_CHECK(hipStreamSynchronize(h.stream));
     h.factored = true;
@@ -1615,23 +1682,20 @@ template <int BS>
 void ensure_mixed(H &h) {
     require_factored(h);
     if (h.mixed_gen == h.factor_gen) return;
-    const size_t bb = (size_t)BS * BS;
-    h.A32.ensure((h.A.nnzb + kPadBlocks) * bb);
-    h.L32.ensure((h.L.nnzb + kPadBlocks) * bb);
-    h.U32.ensure((h.U.nnzb + kPadBlocks) * bb);
+    h.mixed_used = true;
+    if (h.copies_gen == h.factor_gen) {  // written by the factorisation
+        h.mixed_gen = h.factor_gen;
+        return;
+    }
+    mixed_buffers<BS>(h);
     gather_blocks<BS, float>(h, h.A.nnzb, nullptr, h.A64.p, h.A32.p, 0);
     gather_blocks<BS, float>(h, h.L.nnzb, nullptr, h.L64.p, h.L32.p, 0);
     gather_blocks<BS, float>(h, h.U.nnzb, nullptr, h.U64.p, h.U32.p, 0);
-    if (h.L.low2_n >= 0) {
-        h.low2_v32.ensure((h.L.low2_nvblk + kPadBlocks) * bb);
-        gather_blocks<BS, float>(h, h.L.low2_nvblk, nullptr, h.low2_v64.p, h.low2_v32.p, 0);
-    }
-    if (h.u0_is_a && h.an.ncolours > 1) {
-        h.A0d32.ensure((size_t)h.an.colour_ptr[1] * bb);
+    gather_low2_32<BS>(h);
+    if (h.u0_is_a && h.an.ncolours > 1)
         gather_blocks<BS, float>(h, h.an.colour_ptr[1], nullptr, h.A0d64.p, h.A0d32.p, 0);
-    }
     HIP_CHECK(hipStreamSynchronize(h.stream));
-    h.mixed_gen = h.factor_gen;
+    h.copies_gen = h.mixed_gen = h.factor_gen;
 }
 
 template <int BS>
@@ -1645,6 +1709,8 @@ void ensure_adjoint(H &h) {
     gather_blocks<BS, double>(h, h.At.nnzb, h.At.src.p, h.A64.p, h.At64.p, 1);
     gather_blocks<BS, double>(h, h.Ut.nnzb, h.Ut.src.p, h.U64.p, h.Ut64.p, 1);
     gather_blocks<BS, double>(h, h.Lt.nnzb, h.Lt.src.p, h.L64.p, h.Lt64.p, 1);
+    h.DinvT.ensure((size_t)h.n * bb);
+    gather_blocks<BS, double>(h, h.n, nullptr, h.Dinv.p, h.DinvT.p, 1);
     HIP_CHECK(hipStreamSynchronize(h.stream));
     h.adj_gen = h.factor_gen;
 }
@@ -2191,7 +2257,7 @@ int bda_destroy(bda_handle h) {
     (void)hipSetDevice(h->device);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     for (DevMat *m : {&h->A, &h->L, &h->U, &h->At, &h->Ut, &h->Lt}) m->release();
-    for (DBuf<int32_t> *b : {&h->d_perm, &h->d_diag, &h->d_blkrow, &h->d_bad}) b->release();
+    for (DBuf<int32_t> *b : {&h->d_perm, &h->d_blkrow, &h->d_upd, &h->d_bad, &h->d_nonfinite}) b->release();
     for (DBuf<double> *b : {&h->d_orig, &h->A64, &h->L64, &h->U64, &h->LU, &h->Dinv, &h->DinvT, &h->At64, &h->Ut64,
                             &h->Lt64, &h->A0d64, &h->low2_v64, &h->bp, &h->xo, &h->ro, &h->vin, &h->vout, &h->vw, &h->gl, &h->gx, &h->ggrad,
                             &h->partials})
@@ -2252,6 +2318,7 @@ int bda_upload_bcsr(bda_handle h, const int32_t *rowptr, const int32_t *colidx, 
         h->analysed = false;
         h->factored = false;
         copy_sync(*h, h->d_orig.p, values, (size_t)nnzb * h->bs * h->bs * 8, hipMemcpyHostToDevice);
+        h->orig_current = true;
         h->have_values = true;
         h->values_gen++;
     });
@@ -2262,10 +2329,11 @@ int bda_update_values(bda_handle h, const double *values) {
         if (!h->have_pattern) throw std::runtime_error("bda_upload_bcsr has not been called");
         const int64_t nnzb = h->pattern.nnzb();
         copy_sync(*h, h->d_orig.p, values, (size_t)nnzb * h->bs * h->bs * 8, hipMemcpyHostToDevice);
+        h->orig_current = true;
         h->have_values = true;
         h->factored = false;
         h->values_gen++;
-        if (h->analysed) BS_CALL(h, permute_values, *h);
+        if (h->analysed) BS_CALL(h, permute_values, *h, h->d_orig.p);
     });
 }
 
@@ -2273,11 +2341,17 @@ int bda_update_values_dev(bda_handle h, const double *d_values) {
     return guarded(h, [&] {
         if (!h->have_pattern) throw std::runtime_error("bda_upload_bcsr has not been called");
         const int64_t nnzb = h->pattern.nnzb();
-        copy_sync(*h, h->d_orig.p, d_values, (size_t)nnzb * h->bs * h->bs * 8, hipMemcpyDeviceToDevice);
+        // (an analysed handle keeps them in colour order alone: a copy in the
+        // caller's order is made again only for another analysis)
+        const size_t bytes = (size_t)nnzb * h->bs * h->bs * 8;
+        if (!d_values) throw std::runtime_error("null array");
+        const bool direct = h->analysed && (uintptr_t)d_values % 8 == 0 && readable_here(*h, d_values, bytes);
+        if (!direct) copy_sync(*h, h->d_orig.p, d_values, bytes, hipMemcpyDeviceToDevice);
+        h->orig_current = !direct;
+        if (h->analysed) BS_CALL(h, permute_values, *h, direct ? d_values : h->d_orig.p);
         h->have_values = true;
         h->factored = false;
         h->values_gen++;
-        if (h->analysed) BS_CALL(h, permute_values, *h);
     });
 }
 
@@ -2304,6 +2378,7 @@ int bda_upload_factored(bda_handle h, int32_t ncolours, const int32_t *colour_pt
         h->have_pattern = true;
         h->an = std::move(an);
         copy_sync(*h, h->d_orig.p, values, (size_t)nnzb * h->bs * h->bs * 8, hipMemcpyHostToDevice);
+        h->orig_current = true;
         h->have_values = true;
         h->values_gen++;
         finish_analyse(*h);   // identity permutation: A's values are copied as given
