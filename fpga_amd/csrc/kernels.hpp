@@ -93,13 +93,15 @@ struct RedArgs {
     int32_t fin;
 };
 
-__device__ inline void record_norm(SolverState *st, double nrm) {
-    if (st->hist != nullptr && st->nhist < st->hist_cap) st->hist[st->nhist] = nrm;
+// lead: the one workgroup whose scalar step reaches the host and the history
+// (where every workgroup runs the step on a copy of the state, see below)
+__device__ inline void record_norm(SolverState *st, double nrm, bool lead) {
+    if (lead && st->hist != nullptr && st->nhist < st->hist_cap) st->hist[st->nhist] = nrm;
     st->nhist += 1;
 }
 
-__device__ inline void push_norm(SolverState *st, double nrm) {
-    record_norm(st, nrm);
+__device__ inline void push_norm(SolverState *st, double nrm, bool lead) {
+    record_norm(st, nrm, lead);
     const int slot = st->norm_slot;
     st->norms[slot] = nrm;
     st->last_norm_idx = slot;
@@ -111,29 +113,26 @@ __device__ inline bool finite(double v) { return !__builtin_isnan(v) && !__built
 
 // The flag receives the run's id, so the host never has to clear it between
 // runs (a clear could race a late write of the previous run).
-__device__ inline void signal_done(SolverState *st) {
+__device__ inline void signal_done(SolverState *st, bool lead = true) {
     st->done = 1;
-    if (st->host_done) __hip_atomic_store(st->host_done, st->run_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (lead && st->host_done) __hip_atomic_store(st->host_done, st->run_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Progress for the host's throttling (it keeps a bounded number of
 // half-iterations queued ahead of the device): a mapped word, so no event
 // has to be recorded in the stream.
-__device__ inline void signal_progress(SolverState *st, int32_t count) {
-    if (st->host_prog)
+__device__ inline void signal_progress(SolverState *st, int32_t count, bool lead = true) {
+    if (lead && st->host_prog)
         __hip_atomic_store(st->host_prog, ((uint64_t)(uint32_t)st->run_id << 32) | (uint32_t)count, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Scalar epilogues; run by one thread after a grid-wide reduction.  The
-// watchdog is checked first: a run past its deadline stops here, and every
-// launch queued after it returns at once.
-__device__ inline void finalize(SolverState *st, int fin, double t0, double t1) {
-    if (fin != FIN_STORE && st->deadline != 0 && wall_clock64() > st->deadline) {
-        st->aborted = 1;
-        signal_done(st);
-        return;
-    }
+__device__ inline bool past_deadline(const SolverState *st) {
+    return st->deadline != 0 && wall_clock64() > st->deadline;
+}
+
+// Scalar epilogues; run by one thread after a grid-wide reduction.
+__device__ inline void scalar_step(SolverState *st, int fin, double t0, double t1, bool lead) {
     switch (fin) {
     case FIN_STORE:
         st->tot[0] = t0;
@@ -142,7 +141,7 @@ __device__ inline void finalize(SolverState *st, int fin, double t0, double t1) 
     case FIN_INIT: {   // solver.vhd:867-936 with dot_res = rho_new
         const double nrm = sqrt(t0);
         st->nhist = 0;
-        record_norm(st, nrm);
+        record_norm(st, nrm, lead);
         st->rho = t0;
         st->norms[0] = nrm;
         st->norm_slot = 1;
@@ -154,7 +153,7 @@ __device__ inline void finalize(SolverState *st, int fin, double t0, double t1) 
         if (!(nrm > precision)) {
             st->no_results = 1;
             if (!finite(nrm)) st->nan_flag = 1;
-            signal_done(st);
+            signal_done(st, lead);
         } else {
             st->thr = st->abs_mode ? st->tol : st->tol * nrm;
         }
@@ -163,46 +162,46 @@ __device__ inline void finalize(SolverState *st, int fin, double t0, double t1) 
     case FIN_ALPHA:    // step 5: divide rho_new by the dot result
         if (t0 == 0.0 || !finite(t0)) {
             if (t0 == 0.0) st->breakdown = 1; else st->nan_flag = 1;
-            signal_done(st);
+            signal_done(st, lead);
         } else {
             st->alpha = st->rho / t0;
         }
         break;
     case FIN_HALF1: {  // steps 7/8
         const double nrm = sqrt(t0);
-        push_norm(st, nrm);
+        push_norm(st, nrm, lead);
         st->last_half = 1;
-        if (!finite(nrm)) { st->nan_flag = 1; signal_done(st); }
-        else if (!(nrm > st->thr)) { st->converged = 1; signal_done(st); }
-        else if ((st->h >> 1) == st->maxit) { st->max_iter = 1; signal_done(st); }
+        if (!finite(nrm)) { st->nan_flag = 1; signal_done(st, lead); }
+        else if (!(nrm > st->thr)) { st->converged = 1; signal_done(st, lead); }
+        else if ((st->h >> 1) == st->maxit) { st->max_iter = 1; signal_done(st, lead); }
         else {
             st->h += 1;
-            signal_progress(st, st->h);
+            signal_progress(st, st->h, lead);
         }
         break;
     }
     case FIN_OMEGA:    // step 10
         if (t1 == 0.0 || !finite(t0) || !finite(t1)) {
             if (t1 == 0.0) st->breakdown = 1; else st->nan_flag = 1;
-            signal_done(st);
+            signal_done(st, lead);
         } else {
             st->omega = t0 / t1;
         }
         break;
     case FIN_HALF2: {  // step 12, then steps 13/14
         const double nrm = sqrt(t0);
-        push_norm(st, nrm);
+        push_norm(st, nrm, lead);
         st->last_half = 2;
-        if (!finite(nrm)) { st->nan_flag = 1; signal_done(st); }
-        else if (!(nrm > st->thr)) { st->converged = 1; signal_done(st); }
+        if (!finite(nrm)) { st->nan_flag = 1; signal_done(st, lead); }
+        else if (!(nrm > st->thr)) { st->converged = 1; signal_done(st, lead); }
         else {
             st->h += 1;
             st->rho_prev = st->rho;
             st->rho = t1;
-            if (t1 == 0.0 || st->omega == 0.0) { st->breakdown = 1; signal_done(st); }
+            if (t1 == 0.0 || st->omega == 0.0) { st->breakdown = 1; signal_done(st, lead); }
             else {
                 st->beta = (st->rho / st->rho_prev) * (st->alpha / st->omega);
-                signal_progress(st, st->h);
+                signal_progress(st, st->h, lead);
             }
         }
         break;
@@ -216,17 +215,17 @@ __device__ inline void finalize(SolverState *st, int fin, double t0, double t1) 
             if (!(nrm > precision)) {
                 st->no_results = 1;
                 if (__builtin_isnan(nrm)) st->nan_flag = 1;
-                signal_done(st);
+                signal_done(st, lead);
                 break;
             }
             st->thr = st->abs_mode ? st->tol : st->tol * nrm;
             st->last_norm = nrm;
         } else {
-            push_norm(st, nrm);
+            push_norm(st, nrm, lead);
         }
-        if (!finite(nrm)) { st->nan_flag = 1; signal_done(st); }
-        else if (st->outer > 0 && !(nrm > st->thr)) { st->converged = 1; signal_done(st); }
-        else if (st->outer == st->max_outer) { st->max_iter = 1; signal_done(st); }
+        if (!finite(nrm)) { st->nan_flag = 1; signal_done(st, lead); }
+        else if (st->outer > 0 && !(nrm > st->thr)) { st->converged = 1; signal_done(st, lead); }
+        else if (st->outer == st->max_outer) { st->max_iter = 1; signal_done(st, lead); }
         else if (st->adaptive) {
             const double want = st->eta * st->thr / nrm;
             const double m = st->inner_tol < want ? want : st->inner_tol;
@@ -234,12 +233,23 @@ __device__ inline void finalize(SolverState *st, int fin, double t0, double t1) 
         } else {
             st->itol = st->inner_tol;
         }
-        signal_progress(st, st->outer + 1);
+        signal_progress(st, st->outer + 1, lead);
         break;
     }
     default:
         break;
     }
+}
+
+// The watchdog is checked first: a run past its deadline stops here, and every
+// launch queued after it returns at once.
+__device__ inline void finalize(SolverState *st, int fin, double t0, double t1) {
+    if (fin != FIN_STORE && past_deadline(st)) {
+        st->aborted = 1;
+        signal_done(st);
+        return;
+    }
+    scalar_step(st, fin, t0, t1, true);
 }
 
 // Solver state set-up on the stream (no host copy, no synchronisation); the
@@ -1517,20 +1527,126 @@ __global__ __launch_bounds__(kVecThreads) void k_mark_nonzero(int64_t N, const T
     if (nz) __hip_atomic_store(&st->full_residual, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A vector update that forms the reduction results it needs itself ("folded"),
+// in place of a k_finalize launch before it.  Every workgroup adds up the
+// partials (in k_finalize's order, so to the same bits) and runs the scalar
+// step on its own copy of the state; workgroup 0 alone writes the new state,
+// to another slot than the one all of them read, and tells the host.  Up to
+// kFoldMax partials: a launch of its own takes one workgroup 3 us and a
+// launch (3.6 us of host time; 2.3 us in a graph); folded, the sums run
+// beside the update's own loads.  Above that the sums every workgroup repeats
+// cost more than the launch saves.
+struct FoldArgs {
+    const double *part;      // the product's partials: reduction j at part + j * cap
+    int32_t cap, n;
+    const double *vpart;     // those of the vector update before it
+    int32_t vcap, vn;
+    const SolverState *in;
+    SolverState *out;
+};
+constexpr int kFoldMax = 4 * kFinThreads;
+constexpr int kStateWords = sizeof(SolverState) / 8;
+static_assert(sizeof(SolverState) % 8 == 0 && kStateWords <= kVecThreads, "a state word per thread");
+
+template <int NRED, int U>
+__device__ inline void fold_waves(const double *part, int cap, int n, double (*sred)[2]) {
+    constexpr int VW = kFinThreads / kVecThreads;   // waves of k_finalize one wave stands for
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double v[VW][NRED][U];
+#pragma unroll
+    for (int w = 0; w < VW; ++w)
+#pragma unroll
+        for (int j = 0; j < NRED; ++j)
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = u * kFinThreads + (wave * VW + w) * 64 + lane;
+                v[w][j][u] = part[(size_t)j * cap + min(i, n - 1)];
+            }
+#pragma unroll
+    for (int w = 0; w < VW; ++w)
+#pragma unroll
+        for (int j = 0; j < NRED; ++j) {
+            double t = 0.0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = u * kFinThreads + (wave * VW + w) * 64 + lane;
+                t += 0.0 + (i < n ? v[w][j][u] : 0.0);
+            }
+            t = wave_sum(t);
+            if (lane == 0) sred[wave * VW + w][j] = t;
+        }
+}
+// the wave sums of NRED reductions over n <= kFoldMax partials, for fold_total
+// after a barrier
+template <int NRED>
+__device__ inline void fold_sums(const double *part, int cap, int n, double (*sred)[2]) {
+    if (n <= kFinThreads) fold_waves<NRED, 1>(part, cap, n, sred);
+    else fold_waves<NRED, kFoldMax / kFinThreads>(part, cap, n, sred);
+}
+__device__ inline double fold_total(const double (*sred)[2], int j) {
+    double t = sred[0][j];
+    for (int w = 1; w < kFinThreads / 64; ++w) t += sred[w][j];
+    return t;
+}
+// Whether a folded run is past its deadline (thread 0 of workgroup 0, whose
+// clock decides for all): it then stops with the launch after this one, whose
+// update is still complete.
+__device__ inline int fold_late(const SolverState *ss) {
+    return blockIdx.x == 0 && !ss->done && past_deadline(ss) ? 1 : 0;
+}
+// End of a folded scalar step (all threads, after the barrier that follows
+// it): the new state.
+__device__ inline void fold_store(const FoldArgs &f, const SolverState *ss, int late) {
+    if (blockIdx.x != 0) return;
+    const int t = threadIdx.x;
+    if (t < kStateWords) {
+        uint64_t w = reinterpret_cast<const uint64_t *>(ss)[t];
+        constexpr size_t od = offsetof(SolverState, done), oa = offsetof(SolverState, aborted);
+        if (late && t == (int)(od / 8)) w |= (uint64_t)1 << (od % 8 * 8);
+        if (late && t == (int)(oa / 8)) w |= (uint64_t)1 << (oa % 8 * 8);
+        reinterpret_cast<uint64_t *>(f.out)[t] = w;
+    }
+    if (t == 0 && late && ss->host_done)
+        __hip_atomic_store(ss->host_done, ss->run_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // steps 6-8 without the x update: s = r - alpha v; ||s||^2.  Step 6,
 // x += alpha phat, is deferred: k_update_xr applies it together with step 11
 // (the same two roundings, one read and one write of x fewer), and
 // k_finish_x applies it alone when a run ends after a first half-iteration.
-template <typename TX>
-__global__ __launch_bounds__(kVecThreads) void k_update_s(int64_t N, const TX *r, const TX *v, TX *s, RedArgs ra) {
-    if (ra.st->done) return;
-    const double malpha = -ra.st->alpha;
+// FOLD: with step 5 (alpha) before it; the ||s|| test is then left to the
+// folded k_update_xr, and the launches between run whether s is small or not.
+template <typename TX, bool FOLD>
+__global__ __launch_bounds__(kVecThreads) void k_update_s(int64_t N, const TX *r, const TX *v, TX *s, RedArgs ra,
+                                                         FoldArgs f) {
+    if constexpr (!FOLD)
+        if (ra.st->done) return;
     const VecIdx ix = vec_index(N);
     double r0[kVecPairsPerThread], r1[kVecPairsPerThread], v0[kVecPairsPerThread], v1[kVecPairsPerThread];
 #pragma unroll
     for (int j = 0; j < kVecPairsPerThread; ++j) {
         ld2(r, ix.pi[j], r0[j], r1[j]);
         ld2(v, ix.pi[j], v0[j], v1[j]);
+    }
+    double malpha;
+    if constexpr (FOLD) {
+        __shared__ SolverState ss;
+        __shared__ double sred[kFinThreads / 64][2];
+        __shared__ int late;
+        if (threadIdx.x < kStateWords)
+            reinterpret_cast<uint64_t *>(&ss)[threadIdx.x] = reinterpret_cast<const uint64_t *>(f.in)[threadIdx.x];
+        fold_sums<1>(f.part, f.cap, f.n, sred);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            if (!ss.done) scalar_step(&ss, FIN_ALPHA, fold_total(sred, 0), 0.0, blockIdx.x == 0);
+            late = fold_late(&ss);
+        }
+        __syncthreads();
+        fold_store(f, &ss, late);
+        if (ss.done) return;
+        malpha = -ss.alpha;
+    } else {
+        malpha = -ra.st->alpha;
     }
     double acc = 0.0;
 #pragma unroll
@@ -1547,11 +1663,13 @@ __global__ __launch_bounds__(kVecThreads) void k_update_s(int64_t N, const TX *r
 // steps 6 and 11-14: x = (x + alpha phat) + omega shat, rounded to the type
 // of x after each addition as two separate updates would be; r = s - omega
 // t; ||r||^2 and rt.r
-template <typename TX, typename TXX>
+// FOLD: with the ||s|| test (steps 7/8) and step 10 (omega) before it
+template <typename TX, typename TXX, bool FOLD>
 __global__ __launch_bounds__(kVecThreads) void k_update_xr(int64_t N, TXX *x, const TX *phat, const TX *shat,
-                                                          const TX *s, const TX *t, TX *r, const TX *rt, RedArgs ra) {
-    if (ra.st->done) return;
-    const double alpha = ra.st->alpha, omega = ra.st->omega, momega = -omega;
+                                                          const TX *s, const TX *t, TX *r, const TX *rt, RedArgs ra,
+                                                          FoldArgs f) {
+    if constexpr (!FOLD)
+        if (ra.st->done) return;
     const VecIdx ix = vec_index(N);
     double x0[kVecPairsPerThread], x1[kVecPairsPerThread], h0[kVecPairsPerThread], h1[kVecPairsPerThread];
     double s0[kVecPairsPerThread], s1[kVecPairsPerThread], t0[kVecPairsPerThread], t1[kVecPairsPerThread];
@@ -1565,6 +1683,29 @@ __global__ __launch_bounds__(kVecThreads) void k_update_xr(int64_t N, TXX *x, co
         ld2(t, ix.pi[j], t0[j], t1[j]);
         ld2(rt, ix.pi[j], q0[j], q1[j]);
     }
+    double alpha, omega;
+    if constexpr (FOLD) {
+        __shared__ SolverState ss;
+        __shared__ double sred1[kFinThreads / 64][2], sred2[kFinThreads / 64][2];
+        if (threadIdx.x < kStateWords)
+            reinterpret_cast<uint64_t *>(&ss)[threadIdx.x] = reinterpret_cast<const uint64_t *>(f.in)[threadIdx.x];
+        fold_sums<1>(f.vpart, f.vcap, f.vn, sred1);
+        fold_sums<2>(f.part, f.cap, f.n, sred2);
+        __syncthreads();
+        if (threadIdx.x == 0 && !ss.done) {
+            scalar_step(&ss, FIN_HALF1, fold_total(sred1, 0), 0.0, blockIdx.x == 0);
+            if (!ss.done) scalar_step(&ss, FIN_OMEGA, fold_total(sred2, 0), fold_total(sred2, 1), blockIdx.x == 0);
+        }
+        __syncthreads();
+        fold_store(f, &ss, 0);  // (no deadline here: the run would stop with ||r|| unknown)
+        if (ss.done) return;
+        alpha = ss.alpha;
+        omega = ss.omega;
+    } else {
+        alpha = ra.st->alpha;
+        omega = ra.st->omega;
+    }
+    const double momega = -omega;
     double acc[2] = {0.0, 0.0};
 #pragma unroll
     for (int j = 0; j < kVecPairsPerThread; ++j) {
@@ -1599,11 +1740,12 @@ __global__ __launch_bounds__(kVecThreads) void k_finish_x(int64_t N, TXX *x, con
 }
 
 // steps 15-17: p = r + beta (p - omega v), as tmp = (-omega) v + p; p = beta tmp + r
-template <typename TX>
+// FOLD: with step 12 (the ||r|| test, beta) before it
+template <typename TX, bool FOLD>
 __global__ __launch_bounds__(kVecThreads) void k_update_p(int64_t N, TX *p, const TX *r, const TX *v,
-                                                         const SolverState *st) {
-    if (st->done) return;
-    const double beta = st->beta, momega = -st->omega;
+                                                         const SolverState *st, FoldArgs f) {
+    if constexpr (!FOLD)
+        if (st->done) return;
     const VecIdx ix = vec_index(N);
     double p0[kVecPairsPerThread], p1[kVecPairsPerThread], r0[kVecPairsPerThread], r1[kVecPairsPerThread];
     double v0[kVecPairsPerThread], v1[kVecPairsPerThread];
@@ -1612,6 +1754,28 @@ __global__ __launch_bounds__(kVecThreads) void k_update_p(int64_t N, TX *p, cons
         ld2(p, ix.pi[j], p0[j], p1[j]);
         ld2(r, ix.pi[j], r0[j], r1[j]);
         ld2(v, ix.pi[j], v0[j], v1[j]);
+    }
+    double beta, momega;
+    if constexpr (FOLD) {
+        __shared__ SolverState ss;
+        __shared__ double sred[kFinThreads / 64][2];
+        __shared__ int late;
+        if (threadIdx.x < kStateWords)
+            reinterpret_cast<uint64_t *>(&ss)[threadIdx.x] = reinterpret_cast<const uint64_t *>(f.in)[threadIdx.x];
+        fold_sums<2>(f.vpart, f.vcap, f.vn, sred);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            if (!ss.done) scalar_step(&ss, FIN_HALF2, fold_total(sred, 0), fold_total(sred, 1), blockIdx.x == 0);
+            late = fold_late(&ss);
+        }
+        __syncthreads();
+        fold_store(f, &ss, late);
+        if (ss.done) return;
+        beta = ss.beta;
+        momega = -ss.omega;
+    } else {
+        beta = st->beta;
+        momega = -st->omega;
     }
 #pragma unroll
     for (int j = 0; j < kVecPairsPerThread; ++j) {

@@ -568,6 +568,12 @@ enum ProfKind { PK_SPMV = 0, PK_LOWER = 1, PK_UPPER = 2, PK_VEC = 3, PK_N = 4 };
 #ifndef BDA_FUSE0
 #define BDA_FUSE0 1
 #endif
+// 1 (default): reductions of up to kFoldMax partials are added up by the vector
+// update that needs them; 0: always by a launch of their own (the same sums,
+// for A/B timing)
+#ifndef BDA_FOLD
+#define BDA_FOLD 1
+#endif
 // 1 (default): k_finalize_joint for 2,049 to 18,432 partials; 0: k_finalize
 // (the same sums, for A/B timing)
 #ifndef BDA_FIN_JOINT
@@ -616,6 +622,7 @@ struct bda_handle_s {
     // U's colour-0 rows are A's own blocks: true of factors made by
     // bda_factor, not known of a caller's own (bda_upload_factored)
     bool u0_is_a = false;
+    bool fold = BDA_FOLD != 0;    // scalar steps folded into the vector updates (small systems)
     bool fuse0 = BDA_FUSE0 != 0;  // the second sweep of colour 0 with the product's (SM_SUB_SPMV)
 
     // vectors
@@ -627,6 +634,7 @@ struct bda_handle_s {
 
     // reductions and scalar state (0 = solve, 1 = outer loop or auxiliary, 2 = idle)
     bda::DBuf<double> partials;
+    bda::DBuf<double> vparts;  // folded runs: those of k_update_s, then the two of k_update_xr
     int32_t partial_cap = 0;
     bda::DBuf<bda::SolverState> st;
     bda::SolverState *h_st = nullptr;  // pinned
@@ -753,8 +761,10 @@ void check_launch() { HIP_CHECK(hipGetLastError()); }
 
 // State slots: 0 = the running BiCGSTAB, 1 = the outer refinement loop (or a
 // standalone reduction), kIdleState = a state that is never stopped, for
-// launches outside a solve (the streaming kernel always reads a state).
-constexpr int kIdleState = 2;
+// launches outside a solve (the streaming kernel always reads a state).  A run
+// with folded scalar steps takes its state around slots 0, kStateB (after
+// alpha), kStateC (after omega) and back to 0 (after beta).
+constexpr int kIdleState = 2, kStateB = 3, kStateC = 4, kStates = 5;
 
 RedArgs red(H &h, int state_idx, int fin) {
     RedArgs ra;
@@ -891,7 +901,7 @@ void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x
     }
     if (prof_kind >= 0) prof_end(h);
     if (MODE == SM_SPMV && colour == kRestOfRows) nparts = m.ntiles_wide;
-    if (nred > 0) launch_finalize(h, nred, a.ra, nparts);
+    if (nred > 0 && a.ra.fin != FIN_NONE) launch_finalize(h, nred, a.ra, nparts);
 }
 
 // The second sweep of colour 0 and the product's colour-0 rows in one launch
@@ -949,13 +959,13 @@ int vec_blocks(size_t N) { return (int)((N + kVecElemsPerBlock - 1) / kVecElemsP
 
 template <int BS, typename TV, typename TX>
 void sweep_launch(H &h, const DevMat &m, const TV *val, int c, bool dinv_mode, const TX *x, const TX *x_lo, int split,
-                  const TX *rhs, TX *out, const double *dinv, bool use_state) {
-    RedArgs ra = red(h, 0, FIN_NONE);
+                  const TX *rhs, TX *out, const double *dinv, int si) {
+    RedArgs ra = red(h, si, FIN_NONE);
     if (dinv_mode)
-        launch_stream<BS, SM_SUB_DINV, SR_NONE, TV, TX>(h, m, val, c, x, rhs, out, dinv, nullptr, ra, use_state,
+        launch_stream<BS, SM_SUB_DINV, SR_NONE, TV, TX>(h, m, val, c, x, rhs, out, dinv, nullptr, ra, true,
                                                         nullptr, nullptr, x_lo, split);
     else
-        launch_stream<BS, SM_SUB, SR_NONE, TV, TX>(h, m, val, c, x, rhs, out, nullptr, nullptr, ra, use_state, nullptr,
+        launch_stream<BS, SM_SUB, SR_NONE, TV, TX>(h, m, val, c, x, rhs, out, nullptr, nullptr, ra, true, nullptr,
                                                    nullptr, x_lo, split);
 }
 
@@ -973,7 +983,7 @@ void tail_dispatch(H &h, const StreamArgs<TV, TX> &a, const TailArgs<TV, TX> &b)
 
 template <int BS, typename TV, typename TX>
 void tail_launch(H &h, const OpSet<TV> &op, const TX *y, const TX *lo, int split, const TX *p, TX *z,
-                 bool use_state) {
+                 int si) {
     const int nc = h.an.ncolours;
     const DevMat &m1 = *op.S1, &m2 = *op.S2;
     StreamArgs<TV, TX> a;
@@ -991,8 +1001,7 @@ void tail_launch(H &h, const OpSet<TV> &op, const TX *y, const TX *lo, int split
     a.rhs = p;
     a.out = z;
     a.dinv = op.dinv;
-    a.ra = red(h, 0, FIN_NONE);
-    if (!use_state) a.ra.st = h.st.p + kIdleState;
+    a.ra = red(h, si, FIN_NONE);
     TailArgs<TV, TX> b;
     b.rowptr = m2.rowptr.p;
     b.colidx = m2.colidx.p;
@@ -1024,7 +1033,7 @@ void tail3_dispatch(H &h, const StreamArgs<TV, TX> &a, const Tail3Args<TV, TX> &
 // and the first sweep skipped it.
 template <int BS, typename TV, typename TX>
 void tail3_launch(H &h, const OpSet<TV> &op, const TX *y, const TX *lo, int split, const TX *p, TX *z,
-                  const TX *rhs3, bool use_state) {
+                  const TX *rhs3, int si) {
     const int nc = h.an.ncolours;
     const DevMat &m1 = *op.S1, &m2 = *op.S2;
     if (op.s1_dinv || !op.s2_dinv || m2.tail3_n < 0 || m2.tail_ndep < 0 || nc < 3 ||
@@ -1045,8 +1054,7 @@ void tail3_launch(H &h, const OpSet<TV> &op, const TX *y, const TX *lo, int spli
     a.rhs = p;
     a.out = z;
     a.dinv = op.dinv;
-    a.ra = red(h, 0, FIN_NONE);
-    if (!use_state) a.ra.st = h.st.p + kIdleState;
+    a.ra = red(h, si, FIN_NONE);
     Tail3Args<TV, TX> b;
     b.val = op.S2val;
     b.rhs2 = y;
@@ -1090,7 +1098,7 @@ void lower2_dispatch(H &h, const StreamArgs<TV, TX> &a, const StreamArgs<TV, TX>
 // also z of colour C-2's rows without second-sweep blocks.
 template <int BS, typename TV, typename TX>
 void lower2_launch(H &h, const OpSet<TV> &op, const TV *vval, const TX *p, TX *y, const TX *lo, int split, TX *zout,
-                   bool use_state) {
+                   int si) {
     const int nc = h.an.ncolours;
     const DevMat &m = *op.S1;
     const int c = nc - 3;
@@ -1105,8 +1113,7 @@ void lower2_launch(H &h, const OpSet<TV> &op, const TV *vval, const TX *p, TX *y
     a.split = lo ? split : 0;
     a.rhs = p;
     a.out = y;
-    a.ra = red(h, 0, FIN_NONE);
-    if (!use_state) a.ra.st = h.st.p + kIdleState;
+    a.ra = red(h, si, FIN_NONE);
     StreamArgs<TV, TX> v = a, g = a;
     // colour c's own tiles, tall when that saves a quarter of the workgroups
     a.tile0 = m.colour_tile[c];
@@ -1162,7 +1169,7 @@ template <> const float *low2_values<float>(H &h) { return h.low2_v32.p; }
 // skip_last: everything but the second sweep's colour 0 (launch_sweep_spmv
 // follows).
 template <int BS, typename TV, typename TX>
-void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, bool use_state, bool skip_last = false) {
+void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si, bool skip_last = false) {
     const int nc = h.an.ncolours;
     if (op.s1_dinv && op.s2_dinv) throw std::runtime_error("at most one sweep may carry the diagonal inverse");
     const bool skip0 = !op.s1_dinv && nc > 1;
@@ -1176,25 +1183,25 @@ void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, bool use_stat
     prof_begin(h, PK_LOWER);
     for (int c = skip0 ? 1 : 0; c < nc - 1; ++c) {
         if (low2 && c == nc - 3) {
-            lower2_launch<BS, TV, TX>(h, op, low2_values<TV>(h), p, y, lo, split, merge3 ? z : nullptr, use_state);
+            lower2_launch<BS, TV, TX>(h, op, low2_values<TV>(h), p, y, lo, split, merge3 ? z : nullptr, si);
             ++c;  // colour C-2 is done too
         } else if (merge3 && c == nc - 2)
             launch_stream<BS, SM_SUB_Z, SR_NONE, TV, TX>(h, *op.S1, op.S1val, c, y, p, y, op.dinv, nullptr,
-                                                         red(h, 0, FIN_NONE), use_state, nullptr, nullptr, lo, split,
+                                                         red(h, si, FIN_NONE), true, nullptr, nullptr, lo, split,
                                                          -1, op.S2->rowptr.p, z);
         else
-            sweep_launch<BS, TV, TX>(h, *op.S1, op.S1val, c, op.s1_dinv, y, lo, split, p, y, op.dinv, use_state);
+            sweep_launch<BS, TV, TX>(h, *op.S1, op.S1val, c, op.s1_dinv, y, lo, split, p, y, op.dinv, si);
     }
     if (!merge)
         sweep_launch<BS, TV, TX>(h, *op.S1, op.S1val, nc - 1, op.s1_dinv || op.s2_dinv, y, lo, split, p, z, op.dinv,
-                                 use_state);
+                                 si);
     prof_end(h);
     prof_begin(h, PK_UPPER);
-    if (merge3) tail3_launch<BS, TV, TX>(h, op, y, lo, split, p, z, (nc - 3 == 0 && skip0) ? p : y, use_state);
-    else if (merge) tail_launch<BS, TV, TX>(h, op, y, lo, split, p, z, use_state);
+    if (merge3) tail3_launch<BS, TV, TX>(h, op, y, lo, split, p, z, (nc - 3 == 0 && skip0) ? p : y, si);
+    else if (merge) tail_launch<BS, TV, TX>(h, op, y, lo, split, p, z, si);
     for (int c = merge3 ? nc - 4 : merge ? nc - 3 : nc - 2; c >= (skip_last ? 1 : 0); --c)
         sweep_launch<BS, TV, TX>(h, *op.S2, op.S2val, c, op.s2_dinv, z, nullptr, 0, (c == 0 && skip0) ? p : y, z,
-                                 op.dinv, use_state);
+                                 op.dinv, si);
     prof_end(h);
 }
 
@@ -1352,20 +1359,37 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     // preconditioner queued whenever the host waits.
     bool stop = false;
     const bool fuse = fuse_sweep_spmv(h, op);
+    const int nparts = op.A->ntiles_wide;  // of the product
+    const bool fold = h.fold && nparts <= kFoldMax && vb <= kFoldMax;
+    const int st2 = fold ? kStateB : 0;    // the second half's state
+    auto fin_of = [&](int fin) { return fold ? (int)FIN_NONE : fin; };
+    auto fold_args = [&](int in, int out, const double *vpart) {
+        return FoldArgs{h.partials.p, h.partial_cap, nparts, vpart, vb, vb, h.st.p + in, h.st.p + out};
+    };
+    auto vec_red = [&](int fin, double *part) {
+        RedArgs ra = red(h, 0, fin);
+        if (fold) {
+            ra.partials = part;
+            ra.cap = vb;
+        }
+        return ra;
+    };
+    double *spart = h.vparts.p, *xrpart = h.vparts.p + vb;
     // z = M^-1 p, and, fused, the colour-0 rows of v = A z with their dots
-    auto apply = [&](auto redc, const TX *p, TX *z, TX *v, const TX *w0, int fin) {
+    auto apply = [&](auto redc, int si, const TX *p, TX *z, TX *v, const TX *w0) {
         constexpr int RED = decltype(redc)::value;
-        precond<BS, TV, TX>(h, op, p, k.y.p, z, true, fuse);
+        precond<BS, TV, TX>(h, op, p, k.y.p, z, si, fuse);
         if (fuse) {
             prof_begin(h, PK_UPPER);
-            launch_sweep_spmv<BS, RED, TV, TX>(h, op, p, z, v, w0, red(h, 0, fin));
+            launch_sweep_spmv<BS, RED, TV, TX>(h, op, p, z, v, w0, red(h, si, FIN_NONE));
             prof_end(h);
         }
     };
-    auto product = [&](auto redc, const TX *z, TX *v, const TX *w0, int fin) {
+    auto product = [&](auto redc, int si, const TX *z, TX *v, const TX *w0, int fin) {
         constexpr int RED = decltype(redc)::value;
         launch_stream<BS, SM_SPMV, RED, TV, TX>(h, *op.A, op.Aval, fuse ? kRestOfRows : -1, z, nullptr, v, nullptr,
-                                                w0, red(h, 0, fin), true, nullptr, nullptr, nullptr, 0, PK_SPMV);
+                                                w0, red(h, si, fin_of(fin)), true, nullptr, nullptr, nullptr, 0,
+                                                PK_SPMV);
     };
     constexpr std::integral_constant<int, SR_W0> red_w0{};
     constexpr std::integral_constant<int, SR_BOTH> red_both{};
@@ -1385,31 +1409,52 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
             }
         }
     };
+    const dim3 vg(vb), vt(kVecThreads);
     for (int it = 1; it <= maxit + 1 && !stop; ++it) {
         h.prof_tag = 2 * (it - 1);
-        apply(red_w0, k.p.p, k.phat.p, k.v.p, k.rt.p, FIN_ALPHA);
+        apply(red_w0, 0, k.p.p, k.phat.p, k.v.p, k.rt.p);
         throttle(2 * it - 1);
         if (stop) break;
-        product(red_w0, k.phat.p, k.v.p, k.rt.p, FIN_ALPHA);
+        product(red_w0, 0, k.phat.p, k.v.p, k.rt.p, FIN_ALPHA);
         prof_begin(h, PK_VEC);
-        hipLaunchKernelGGL((k_update_s<TX>), dim3(vb), dim3(kVecThreads), 0, h.stream, (int64_t)N, k.r.p, k.v.p,
-                           k.s.p, red(h, 0, FIN_HALF1));
-        check_launch();
-        launch_finalize(h, 1, red(h, 0, FIN_HALF1), vb);
+        if (fold) {
+            hipLaunchKernelGGL((k_update_s<TX, true>), vg, vt, 0, h.stream, (int64_t)N, k.r.p, k.v.p, k.s.p,
+                               vec_red(FIN_NONE, spart), fold_args(0, kStateB, nullptr));
+            check_launch();
+        } else {
+            hipLaunchKernelGGL((k_update_s<TX, false>), vg, vt, 0, h.stream, (int64_t)N, k.r.p, k.v.p, k.s.p,
+                               red(h, 0, FIN_HALF1), FoldArgs{});
+            check_launch();
+            launch_finalize(h, 1, red(h, 0, FIN_HALF1), vb);
+        }
         prof_end(h);
         h.prof_tag = 2 * (it - 1) + 1;
-        apply(red_both, k.s.p, k.shat.p, k.t.p, k.s.p, FIN_OMEGA);
-        throttle(2 * it);
-        if (stop) break;
-        product(red_both, k.shat.p, k.t.p, k.s.p, FIN_OMEGA);
+        apply(red_both, st2, k.s.p, k.shat.p, k.t.p, k.s.p);
+        // (a folded run reports the first half's end with the second's, so
+        // the host checks its lead once per iteration)
+        if (!fold) {
+            throttle(2 * it);
+            if (stop) break;
+        }
+        product(red_both, st2, k.shat.p, k.t.p, k.s.p, FIN_OMEGA);
         prof_begin(h, PK_VEC);
-        hipLaunchKernelGGL((k_update_xr<TX, TX>), dim3(vb), dim3(kVecThreads), 0, h.stream, (int64_t)N, k.x.p,
-                           k.phat.p, k.shat.p, k.s.p, k.t.p, k.r.p, k.rt.p, red(h, 0, FIN_HALF2));
-        check_launch();
-        launch_finalize(h, 2, red(h, 0, FIN_HALF2), vb);
-        hipLaunchKernelGGL((k_update_p<TX>), dim3(vb), dim3(kVecThreads), 0, h.stream, (int64_t)N, k.p.p, k.r.p,
-                           k.v.p, (const SolverState *)(h.st.p));
-        check_launch();
+        if (fold) {
+            hipLaunchKernelGGL((k_update_xr<TX, TX, true>), vg, vt, 0, h.stream, (int64_t)N, k.x.p, k.phat.p,
+                               k.shat.p, k.s.p, k.t.p, k.r.p, k.rt.p, vec_red(FIN_NONE, xrpart),
+                               fold_args(kStateB, kStateC, spart));
+            check_launch();
+            hipLaunchKernelGGL((k_update_p<TX, true>), vg, vt, 0, h.stream, (int64_t)N, k.p.p, k.r.p, k.v.p,
+                               (const SolverState *)nullptr, fold_args(kStateC, 0, xrpart));
+            check_launch();
+        } else {
+            hipLaunchKernelGGL((k_update_xr<TX, TX, false>), vg, vt, 0, h.stream, (int64_t)N, k.x.p, k.phat.p,
+                               k.shat.p, k.s.p, k.t.p, k.r.p, k.rt.p, red(h, 0, FIN_HALF2), FoldArgs{});
+            check_launch();
+            launch_finalize(h, 2, red(h, 0, FIN_HALF2), vb);
+            hipLaunchKernelGGL((k_update_p<TX, false>), vg, vt, 0, h.stream, (int64_t)N, k.p.p, k.r.p, k.v.p,
+                               (const SolverState *)(h.st.p), FoldArgs{});
+            check_launch();
+        }
         prof_end(h);
     }
     // x += alpha phat of a run that ended after a first half-iteration (the
@@ -1546,6 +1591,7 @@ void finish_analyse(H &h) {
     const int cap = std::max({h.A.ntiles, h.At.ntiles, vec_blocks(h.N()), 1}) + kFinGroups;
     h.partial_cap = cap;
     h.partials.ensure((size_t)2 * cap);
+    h.vparts.ensure((size_t)3 * vec_blocks(h.N()));
     h.k64.ensure(h.Npad());
     h.bp.ensure(h.Npad());
     h.xo.ensure(h.Npad());
@@ -2095,13 +2141,13 @@ void precond_perm(H &h, int prec, const void *p, void *z, int transpose) {
     // the intermediate of the two sweeps goes to vw
     if (prec == PREC_F32) {
         OpSet<float> op = transpose ? op_adj32(h) : op_fwd32(h);
-        precond<BS, float, float>(h, op, (const float *)h.vin.p, (float *)h.vw.p, (float *)h.vout.p, false);
+        precond<BS, float, float>(h, op, (const float *)h.vin.p, (float *)h.vw.p, (float *)h.vout.p, kIdleState);
     } else if (prec == PREC_F32_X64) {
         OpSet<float> op = transpose ? op_adj32(h) : op_fwd32(h);
-        precond<BS, float, double>(h, op, h.vin.p, h.vw.p, h.vout.p, false);
+        precond<BS, float, double>(h, op, h.vin.p, h.vw.p, h.vout.p, kIdleState);
     } else {
         OpSet<double> op = transpose ? op_adj64(h) : op_fwd64(h);
-        precond<BS, double, double>(h, op, h.vin.p, h.vw.p, h.vout.p, false);
+        precond<BS, double, double>(h, op, h.vin.p, h.vw.p, h.vout.p, kIdleState);
     }
     HIP_CHECK(hipStreamSynchronize(h.stream));
     prof_collect(h);
@@ -2168,8 +2214,8 @@ double time_precond(H &h, int reps, int fp32) {
     HIP_CHECK(hipEventCreate(&e1));
     for (int rep = -1; rep < reps; ++rep) {
         if (rep == 0) HIP_CHECK(hipEventRecord(e0, h.stream));
-        if (fp32) precond<BS, float, float>(h, op_fwd32(h), h.k32.p.p, h.k32.y.p, h.k32.phat.p, false);
-        else precond<BS, double, double>(h, op_fwd64(h), h.k64.p.p, h.k64.y.p, h.k64.phat.p, false);
+        if (fp32) precond<BS, float, float>(h, op_fwd32(h), h.k32.p.p, h.k32.y.p, h.k32.phat.p, kIdleState);
+        else precond<BS, double, double>(h, op_fwd64(h), h.k64.p.p, h.k64.y.p, h.k64.phat.p, kIdleState);
     }
     HIP_CHECK(hipEventRecord(e1, h.stream));
     HIP_CHECK(hipEventSynchronize(e1));
@@ -2232,7 +2278,7 @@ int bda_create(int32_t bs, int32_t n, int32_t nnzb_max, bda_handle *out) {
         // the legacy default stream (torch's default), so device inputs
         // produced there are complete before the handle reads them
         HIP_CHECK(hipStreamCreate(&h->stream));
-        h->st.ensure(kIdleState + 1);  // DBuf zero-fills: the idle slot never has done set
+        h->st.ensure(kStates);  // DBuf zero-fills: the idle slot never has done set
         HIP_CHECK(hipHostMalloc((void **)&h->h_st, sizeof(SolverState), hipHostMallocDefault));
         HIP_CHECK(hipHostMalloc((void **)&h->h_done, 2 * sizeof(int32_t), hipHostMallocMapped));
         h->h_done[0] = h->h_done[1] = 0;
@@ -2260,7 +2306,7 @@ int bda_destroy(bda_handle h) {
     for (DBuf<int32_t> *b : {&h->d_perm, &h->d_blkrow, &h->d_upd, &h->d_bad, &h->d_nonfinite}) b->release();
     for (DBuf<double> *b : {&h->d_orig, &h->A64, &h->L64, &h->U64, &h->LU, &h->Dinv, &h->DinvT, &h->At64, &h->Ut64,
                             &h->Lt64, &h->A0d64, &h->low2_v64, &h->bp, &h->xo, &h->ro, &h->vin, &h->vout, &h->vw, &h->gl, &h->gx, &h->ggrad,
-                            &h->partials})
+                            &h->partials, &h->vparts})
         b->release();
     for (DBuf<float> *b : {&h->A32, &h->L32, &h->U32, &h->A0d32, &h->low2_v32, &h->At32, &h->Ut32, &h->Lt32}) b->release();
     h->k64.release();
