@@ -1532,10 +1532,12 @@ __global__ __launch_bounds__(kVecThreads) void k_mark_nonzero(int64_t N, const T
 // partials (in k_finalize's order, so to the same bits) and runs the scalar
 // step on its own copy of the state; workgroup 0 alone writes the new state,
 // to another slot than the one all of them read, and tells the host.  Up to
-// kFoldMax partials: a launch of its own takes one workgroup 3 us and a
-// launch (3.6 us of host time; 2.3 us in a graph); folded, the sums run
-// beside the update's own loads.  Above that the sums every workgroup repeats
-// cost more than the launch saves.
+// kFoldMax partials: a launch of its own takes about 3 us whatever it does;
+// folded, the sums run beside the update's own loads and add 1.0-1.5 us to
+// it.  A forward and backward solve of 64x64x32 to 1e-10 (20 iterations each)
+// 4.26 -> 3.96 ms, a 32x32x16 precision-form step 648 -> 608 us.  Every
+// workgroup repeats the sums, so their cost grows with the square of the
+// system: at 4,096 partials 288 workgroups read 19 MB from the L2.
 struct FoldArgs {
     const double *part;      // the product's partials: reduction j at part + j * cap
     int32_t cap, n;
@@ -1614,8 +1616,7 @@ __device__ inline void fold_store(const FoldArgs &f, const SolverState *ss, int 
 // x += alpha phat, is deferred: k_update_xr applies it together with step 11
 // (the same two roundings, one read and one write of x fewer), and
 // k_finish_x applies it alone when a run ends after a first half-iteration.
-// FOLD: with step 5 (alpha) before it; the ||s|| test is then left to the
-// folded k_update_xr, and the launches between run whether s is small or not.
+// FOLD: with step 5 (alpha) before it
 template <typename TX, bool FOLD>
 __global__ __launch_bounds__(kVecThreads) void k_update_s(int64_t N, const TX *r, const TX *v, TX *s, RedArgs ra,
                                                          FoldArgs f) {
@@ -1660,10 +1661,26 @@ __global__ __launch_bounds__(kVecThreads) void k_update_s(int64_t N, const TX *r
     block_partials<kVecThreads, 1>(vv, ra, blockIdx.x);
 }
 
+// The ||s|| test (steps 7/8) of a folded run, one workgroup.  Folded into the
+// second half's k_update_xr the run learns of a convergence in its first half
+// only after the second half's product: 2% faster over 20 iterations, 2-8%
+// slower over 2 to 5.
+__global__ __launch_bounds__(kVecThreads) void k_fold_half1(FoldArgs f) {
+    __shared__ SolverState ss;
+    __shared__ double sred[kFinThreads / 64][2];
+    if (threadIdx.x < kStateWords)
+        reinterpret_cast<uint64_t *>(&ss)[threadIdx.x] = reinterpret_cast<const uint64_t *>(f.in)[threadIdx.x];
+    fold_sums<1>(f.vpart, f.vcap, f.vn, sred);
+    __syncthreads();
+    if (threadIdx.x == 0 && !ss.done) scalar_step(&ss, FIN_HALF1, fold_total(sred, 0), 0.0, true);
+    __syncthreads();
+    fold_store(f, &ss, 0);
+}
+
 // steps 6 and 11-14: x = (x + alpha phat) + omega shat, rounded to the type
 // of x after each addition as two separate updates would be; r = s - omega
 // t; ||r||^2 and rt.r
-// FOLD: with the ||s|| test (steps 7/8) and step 10 (omega) before it
+// FOLD: with step 10 (omega) before it
 template <typename TX, typename TXX, bool FOLD>
 __global__ __launch_bounds__(kVecThreads) void k_update_xr(int64_t N, TXX *x, const TX *phat, const TX *shat,
                                                           const TX *s, const TX *t, TX *r, const TX *rt, RedArgs ra,
@@ -1686,16 +1703,13 @@ __global__ __launch_bounds__(kVecThreads) void k_update_xr(int64_t N, TXX *x, co
     double alpha, omega;
     if constexpr (FOLD) {
         __shared__ SolverState ss;
-        __shared__ double sred1[kFinThreads / 64][2], sred2[kFinThreads / 64][2];
+        __shared__ double sred2[kFinThreads / 64][2];
         if (threadIdx.x < kStateWords)
             reinterpret_cast<uint64_t *>(&ss)[threadIdx.x] = reinterpret_cast<const uint64_t *>(f.in)[threadIdx.x];
-        fold_sums<1>(f.vpart, f.vcap, f.vn, sred1);
         fold_sums<2>(f.part, f.cap, f.n, sred2);
         __syncthreads();
-        if (threadIdx.x == 0 && !ss.done) {
-            scalar_step(&ss, FIN_HALF1, fold_total(sred1, 0), 0.0, blockIdx.x == 0);
-            if (!ss.done) scalar_step(&ss, FIN_OMEGA, fold_total(sred2, 0), fold_total(sred2, 1), blockIdx.x == 0);
-        }
+        if (threadIdx.x == 0 && !ss.done)
+            scalar_step(&ss, FIN_OMEGA, fold_total(sred2, 0), fold_total(sred2, 1), blockIdx.x == 0);
         __syncthreads();
         fold_store(f, &ss, 0);  // (no deadline here: the run would stop with ||r|| unknown)
         if (ss.done) return;

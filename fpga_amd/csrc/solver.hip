@@ -762,9 +762,9 @@ void check_launch() { HIP_CHECK(hipGetLastError()); }
 // State slots: 0 = the running BiCGSTAB, 1 = the outer refinement loop (or a
 // standalone reduction), kIdleState = a state that is never stopped, for
 // launches outside a solve (the streaming kernel always reads a state).  A run
-// with folded scalar steps takes its state around slots 0, kStateB (after
-// alpha), kStateC (after omega) and back to 0 (after beta).
-constexpr int kIdleState = 2, kStateB = 3, kStateC = 4, kStates = 5;
+// with folded scalar steps takes its state to kStateB after alpha and after
+// omega, and back to slot 0 after the ||s|| test and after beta.
+constexpr int kIdleState = 2, kStateB = 3, kStates = 4;
 
 RedArgs red(H &h, int state_idx, int fin) {
     RedArgs ra;
@@ -1361,7 +1361,6 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     const bool fuse = fuse_sweep_spmv(h, op);
     const int nparts = op.A->ntiles_wide;  // of the product
     const bool fold = h.fold && nparts <= kFoldMax && vb <= kFoldMax;
-    const int st2 = fold ? kStateB : 0;    // the second half's state
     auto fin_of = [&](int fin) { return fold ? (int)FIN_NONE : fin; };
     auto fold_args = [&](int in, int out, const double *vpart) {
         return FoldArgs{h.partials.p, h.partial_cap, nparts, vpart, vb, vb, h.st.p + in, h.st.p + out};
@@ -1376,19 +1375,19 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     };
     double *spart = h.vparts.p, *xrpart = h.vparts.p + vb;
     // z = M^-1 p, and, fused, the colour-0 rows of v = A z with their dots
-    auto apply = [&](auto redc, int si, const TX *p, TX *z, TX *v, const TX *w0) {
+    auto apply = [&](auto redc, const TX *p, TX *z, TX *v, const TX *w0) {
         constexpr int RED = decltype(redc)::value;
-        precond<BS, TV, TX>(h, op, p, k.y.p, z, si, fuse);
+        precond<BS, TV, TX>(h, op, p, k.y.p, z, 0, fuse);
         if (fuse) {
             prof_begin(h, PK_UPPER);
-            launch_sweep_spmv<BS, RED, TV, TX>(h, op, p, z, v, w0, red(h, si, FIN_NONE));
+            launch_sweep_spmv<BS, RED, TV, TX>(h, op, p, z, v, w0, red(h, 0, FIN_NONE));
             prof_end(h);
         }
     };
-    auto product = [&](auto redc, int si, const TX *z, TX *v, const TX *w0, int fin) {
+    auto product = [&](auto redc, const TX *z, TX *v, const TX *w0, int fin) {
         constexpr int RED = decltype(redc)::value;
         launch_stream<BS, SM_SPMV, RED, TV, TX>(h, *op.A, op.Aval, fuse ? kRestOfRows : -1, z, nullptr, v, nullptr,
-                                                w0, red(h, si, fin_of(fin)), true, nullptr, nullptr, nullptr, 0,
+                                                w0, red(h, 0, fin_of(fin)), true, nullptr, nullptr, nullptr, 0,
                                                 PK_SPMV);
     };
     constexpr std::integral_constant<int, SR_W0> red_w0{};
@@ -1412,14 +1411,16 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     const dim3 vg(vb), vt(kVecThreads);
     for (int it = 1; it <= maxit + 1 && !stop; ++it) {
         h.prof_tag = 2 * (it - 1);
-        apply(red_w0, 0, k.p.p, k.phat.p, k.v.p, k.rt.p);
+        apply(red_w0, k.p.p, k.phat.p, k.v.p, k.rt.p);
         throttle(2 * it - 1);
         if (stop) break;
-        product(red_w0, 0, k.phat.p, k.v.p, k.rt.p, FIN_ALPHA);
+        product(red_w0, k.phat.p, k.v.p, k.rt.p, FIN_ALPHA);
         prof_begin(h, PK_VEC);
         if (fold) {
             hipLaunchKernelGGL((k_update_s<TX, true>), vg, vt, 0, h.stream, (int64_t)N, k.r.p, k.v.p, k.s.p,
                                vec_red(FIN_NONE, spart), fold_args(0, kStateB, nullptr));
+            check_launch();
+            hipLaunchKernelGGL(k_fold_half1, dim3(1), vt, 0, h.stream, fold_args(kStateB, 0, spart));
             check_launch();
         } else {
             hipLaunchKernelGGL((k_update_s<TX, false>), vg, vt, 0, h.stream, (int64_t)N, k.r.p, k.v.p, k.s.p,
@@ -1429,22 +1430,18 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
         }
         prof_end(h);
         h.prof_tag = 2 * (it - 1) + 1;
-        apply(red_both, st2, k.s.p, k.shat.p, k.t.p, k.s.p);
-        // (a folded run reports the first half's end with the second's, so
-        // the host checks its lead once per iteration)
-        if (!fold) {
-            throttle(2 * it);
-            if (stop) break;
-        }
-        product(red_both, st2, k.shat.p, k.t.p, k.s.p, FIN_OMEGA);
+        apply(red_both, k.s.p, k.shat.p, k.t.p, k.s.p);
+        throttle(2 * it);
+        if (stop) break;
+        product(red_both, k.shat.p, k.t.p, k.s.p, FIN_OMEGA);
         prof_begin(h, PK_VEC);
         if (fold) {
             hipLaunchKernelGGL((k_update_xr<TX, TX, true>), vg, vt, 0, h.stream, (int64_t)N, k.x.p, k.phat.p,
                                k.shat.p, k.s.p, k.t.p, k.r.p, k.rt.p, vec_red(FIN_NONE, xrpart),
-                               fold_args(kStateB, kStateC, spart));
+                               fold_args(0, kStateB, nullptr));
             check_launch();
             hipLaunchKernelGGL((k_update_p<TX, true>), vg, vt, 0, h.stream, (int64_t)N, k.p.p, k.r.p, k.v.p,
-                               (const SolverState *)nullptr, fold_args(kStateC, 0, xrpart));
+                               (const SolverState *)nullptr, fold_args(kStateB, 0, xrpart));
             check_launch();
         } else {
             hipLaunchKernelGGL((k_update_xr<TX, TX, false>), vg, vt, 0, h.stream, (int64_t)N, k.x.p, k.phat.p,

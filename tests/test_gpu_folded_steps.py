@@ -3,7 +3,7 @@ the CPU oracle and against themselves at the limits of the rule: one to a few
 hundred product tiles (one load per thread in the folded sums), above 1,024
 (four), and above 4,096 (launches of their own).  What has to hold on every
 side: the iteration counts, flags and norms of the oracle's solve, the same
-bits when a solve is repeated, and the stops that fall between two folded
+bits when a solve is repeated, and the stops around the folded
 steps: an iteration cap (which stops after a first half), a convergence in the
 first half, and the watchdog.
 """
