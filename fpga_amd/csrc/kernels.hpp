@@ -4,14 +4,14 @@
 //
 // Kernel map (reference op -> kernel):
 //   SpMV mode, sparstition.vhd:655-878 / spmvp.vhd:240-383  -> k_stream<SPMV>
-//   steps 0-1 (r = b - A x0, rho)  solver_pkg.vhd:122-123     -> k_mark_nonzero + k_stream<SUB, ZX> + FIN_INIT
+//   steps 0-1 (r = b - A x0, rho)  solver_pkg.vhd:122-123     -> k_gather_start + k_stream<SUB, ZX> + FIN_INIT
 //                                                                 (r = b without the product when x0 = 0)
 //   ILU0_L_fs, ilu0.vhd:412-416                               -> k_stream<SUB> per colour
 //   ILU0_U_bs, ilu0.vhd:385-410                               -> k_stream<SUB_DINV> per colour
 //   dot1 -> alpha, solver.vhd:793-798                         -> SpMV epilogue + FIN_ALPHA
 //   axpy1 + axpy2/norm, solver_pkg.vhd:128-130                -> k_update_s + FIN_HALF1 (axpy1,
 //                                                                 x += alpha phat, deferred into
-//                                                                 k_update_xr / k_finish_x)
+//                                                                 k_update_xr / k_scatter_end)
 //   dot2 -> omega, solver.vhd:831-842                         -> SpMV epilogue + FIN_OMEGA
 //   axpy1 + axpy2/norm + dot1 -> beta, solver_pkg.vhd:133-136 -> k_update_xr + FIN_HALF2
 //   calc_p, vector_ops.vhd:319-323,429-458                    -> k_update_p
@@ -61,7 +61,7 @@ struct SolverState {
     int32_t max_outer;
     int32_t adaptive;
     int32_t inner_h;        // sum of the inner runs' half iterations
-    int32_t full_residual;  // set by k_mark_nonzero: the step-0 residual needs the product
+    int32_t full_residual;  // set by k_gather_start: the step-0 residual needs the product
     // watchdog (the counterpart of the reference kernel's abort cycle count,
     // param0): timeout in ticks of the device's constant-rate wall clock
     // (0 = off); the run's deadline is set on the device when its state is
@@ -259,17 +259,16 @@ __global__ void k_set_state(SolverState *st, SolverState v) {
     *st = v;
 }
 
-// Start of an inner run of the precision form: tolerance and deadline from
+// State of an inner run of the precision form: tolerance and deadline from
 // the outer state; an outer state that has already stopped stops the inner
 // run.
-__global__ void k_inner_start(SolverState *in, const SolverState *out, SolverState v) {
+__device__ inline void inner_start(SolverState *in, const SolverState *out, SolverState v) {
     v.deadline = out->deadline;
+    if (!out->done) v.tol = out->itol;
     *in = v;
     if (out->done) {
         in->no_results = 1;
         signal_done(in);
-    } else {
-        in->tol = out->itol;
     }
 }
 
@@ -277,7 +276,7 @@ __global__ void k_inner_start(SolverState *in, const SolverState *out, SolverSta
 // run whose right-hand side was already zero ends the refinement, and so
 // does one that broke down or met a NaN before completing a half-iteration:
 // it changed nothing, so the next outer step would repeat it exactly.
-__global__ void k_refine_step(SolverState *out, const SolverState *in) {
+__device__ inline void refine_step(SolverState *out, const SolverState *in) {
     if (out->done) return;
     out->outer += 1;
     out->inner_h += in->h;
@@ -289,6 +288,16 @@ __global__ void k_refine_step(SolverState *out, const SolverState *in) {
     if (in->aborted) out->aborted = 1;
     if (in->no_results || in->aborted || ((in->breakdown || in->nan_flag) && in->h == 0 && in->last_half == 0))
         signal_done(out);
+}
+
+// The factorisation's flags: cleared before it, and the bad row (INT32_MAX:
+// none) to mapped host memory after it.
+__global__ void k_factor_begin(int32_t *bad, int32_t *nonfinite) {
+    *bad = INT32_MAX;
+    *nonfinite = 0;
+}
+__global__ void k_factor_end(const int32_t *bad, int32_t *host_bad) {
+    __hip_atomic_store(host_bad, *bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Sum over the 64 lanes of a wave as the butterfly v += v[lane ^ o] for
@@ -1509,24 +1518,6 @@ __device__ inline VecIdx vec_index(int64_t N) {
     return v;
 }
 
-// Check before a step-0 residual: sets st->full_residual when an entry of x
-// is not zero (a NaN counts as nonzero) or the matrix holds a non-finite
-// value (*nonfinite, recorded when the factorisation copied it).  Every
-// writer stores the same value.
-template <typename TX>
-__global__ __launch_bounds__(kVecThreads) void k_mark_nonzero(int64_t N, const TX *x, const int32_t *nonfinite,
-                                                              SolverState *st) {
-    const VecIdx ix = vec_index(N);
-    bool nz = *nonfinite != 0;
-#pragma unroll
-    for (int j = 0; j < kVecPairsPerThread; ++j) {
-        double a, b;
-        ld2(x, ix.pi[j], a, b);
-        nz = nz || (ix.ok[j] && !(a == 0.0)) || (ix.second[j] && !(b == 0.0));
-    }
-    if (nz) __hip_atomic_store(&st->full_residual, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // A vector update that forms the reduction results it needs itself ("folded"),
 // in place of a k_finalize launch before it.  Every workgroup adds up the
 // partials (in k_finalize's order, so to the same bits) and runs the scalar
@@ -1615,7 +1606,7 @@ __device__ inline void fold_store(const FoldArgs &f, const SolverState *ss, int 
 // steps 6-8 without the x update: s = r - alpha v; ||s||^2.  Step 6,
 // x += alpha phat, is deferred: k_update_xr applies it together with step 11
 // (the same two roundings, one read and one write of x fewer), and
-// k_finish_x applies it alone when a run ends after a first half-iteration.
+// finished_x applies it alone when a run ends after a first half-iteration.
 // FOLD: with step 5 (alpha) before it
 template <typename TX, bool FOLD>
 __global__ __launch_bounds__(kVecThreads) void k_update_s(int64_t N, const TX *r, const TX *v, TX *s, RedArgs ra,
@@ -1735,24 +1726,6 @@ __global__ __launch_bounds__(kVecThreads) void k_update_xr(int64_t N, TXX *x, co
     block_partials<kVecThreads, 2>(acc, ra, blockIdx.x);
 }
 
-// End of a run: the deferred step 6, x += alpha phat, when the last
-// half-iteration that ran was a first half (its ||s|| test stopped the run,
-// or the run ended there); it runs whether or not the run has stopped.
-template <typename TX, typename TXX>
-__global__ __launch_bounds__(kVecThreads) void k_finish_x(int64_t N, TXX *x, const TX *phat, const SolverState *st) {
-    if (st->last_half != 1) return;
-    const double alpha = st->alpha;
-    const VecIdx ix = vec_index(N);
-    double x0[kVecPairsPerThread], x1[kVecPairsPerThread], p0[kVecPairsPerThread], p1[kVecPairsPerThread];
-#pragma unroll
-    for (int j = 0; j < kVecPairsPerThread; ++j) {
-        ld2(x, ix.pi[j], x0[j], x1[j]);
-        ld2(phat, ix.pi[j], p0[j], p1[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < kVecPairsPerThread; ++j) st2(x, ix.pi[j], alpha * p0[j] + x0[j], alpha * p1[j] + x1[j]);
-}
-
 // steps 15-17: p = r + beta (p - omega v), as tmp = (-omega) v + p; p = beta tmp + r
 // FOLD: with step 12 (the ||r|| test, beta) before it
 template <typename TX, bool FOLD>
@@ -1799,11 +1772,14 @@ __global__ __launch_bounds__(kVecThreads) void k_update_p(int64_t N, TX *p, cons
 }
 
 // Steps 0-1 for x0 = 0 (A*0 = 0, so rt = b exactly): rt = r = p = rhs,
-// x = 0, rho = rt.rt.  Used by the inner solves of the precision form.
+// x = 0, rho = rt.rt, for the inner solves of the precision form, whose state
+// it also sets up (workgroup 0; all read the outer state instead).
 template <typename TX, typename TXX>
 __global__ __launch_bounds__(kVecThreads) void k_init_zero_x0(int64_t N, const double *rhs, TX *rt, TX *r, TX *p,
-                                                             TXX *x, RedArgs ra) {
-    if (ra.st->done) return;
+                                                             TXX *x, RedArgs ra, const SolverState *outer,
+                                                             SolverState start) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) inner_start(ra.st, outer, start);
+    if (outer->done) return;
     const VecIdx ix = vec_index(N);
     double b0[kVecPairsPerThread], b1[kVecPairsPerThread];
 #pragma unroll
@@ -1823,16 +1799,26 @@ __global__ __launch_bounds__(kVecThreads) void k_init_zero_x0(int64_t N, const d
     block_partials<kVecThreads, 1>(vv, ra, blockIdx.x);
 }
 
-// x64 += d (outer refinement update of the precision form), unless the inner
-// run produced no results: it then either never started (the outer loop had
-// already stopped when its start was queued) or had a zero right-hand side,
-// and d is not its output
+// The deferred step 6 of a run that ended after a first half-iteration (its
+// ||s|| test stopped it, or it ended there): x + alpha phat, else x.
+template <typename TX>
+__device__ inline double finished_x(const TX *x, const TX *phat, int64_t i, bool first_half, double alpha) {
+    const double v = (double)x[i];
+    return first_half ? rnd<TX>(alpha * (double)phat[i] + v) : v;
+}
+
+// End of an inner run: x64 += d, its finished result (the outer refinement
+// update of the precision form), unless it produced no results: it then
+// either never started (the outer loop had already stopped when its start was
+// queued) or had a zero right-hand side, and d is not its output.  Workgroup
+// 0 also takes the run's counters and flags to the outer state.
 template <typename TXX>
-__global__ __launch_bounds__(kVecThreads) void k_add_correction(int64_t N, double *x, const TXX *d,
-                                                                const SolverState *in) {
+__global__ __launch_bounds__(kVecThreads) void k_add_correction(int64_t N, double *x, const TXX *d, const TXX *phat,
+                                                                const SolverState *in, SolverState *outer) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) refine_step(outer, in);
     if (in->no_results) return;
     const int64_t i = (int64_t)blockIdx.x * kVecThreads + threadIdx.x;
-    if (i < N) x[i] = x[i] + (double)d[i];
+    if (i < N) x[i] = x[i] + finished_x(d, phat, i, in->last_half == 1, in->alpha);
 }
 
 // ---------------------------------------------------------------------------
@@ -1874,22 +1860,43 @@ __global__ void k_gather_rows(int n, int bs, const int32_t *perm, const double *
     const int64_t k = i / bs, c = i - k * bs;
     out[i] = in[(int64_t)perm[k] * bs + c];
 }
-// two vectors in one launch (the right-hand side and the start vector)
-__global__ void k_gather_rows2(int n, int bs, const int32_t *perm, const double *in1, double *out1,
-                               const double *in2, double *out2) {
+// Start of a solve: the right-hand side and the start vector in one launch,
+// with the check before the step-0 residual: sets st->full_residual when an
+// entry of the start vector is not zero (a NaN counts as nonzero) or the
+// matrix holds a non-finite value (*nonfinite, recorded when it was
+// factorised).  Every writer stores the same value.
+__global__ void k_gather_start(int n, int bs, const int32_t *perm, const double *b, double *bp, const double *x,
+                               double *xp, const int32_t *nonfinite, SolverState *st) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (int64_t)n * bs) return;
     const int64_t k = i / bs, c = i - k * bs;
     const int64_t j = (int64_t)perm[k] * bs + c;
-    const double a = in1[j], b = in2[j];
-    out1[i] = a;
-    out2[i] = b;
+    const double vb = b[j], vx = x[j];
+    bp[i] = vb;
+    xp[i] = vx;
+    if (!(vx == 0.0) || (i == 0 && *nonfinite != 0))
+        __hip_atomic_store(&st->full_residual, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __global__ void k_scatter_rows(int n, int bs, const int32_t *perm, const double *in, double *out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (int64_t)n * bs) return;
     const int64_t k = i / bs, c = i - k * bs;
     out[(int64_t)perm[k] * bs + c] = in[i];
+}
+// End of a solve: x (finished with phat, when given) to the caller's order,
+// and the state to mapped host memory, so that the host waits once, for this
+// launch (an 8-byte copy and its wait took 21 us).
+__global__ __launch_bounds__(256) void k_scatter_end(int n, int bs, const int32_t *perm, const double *x,
+                                                     const double *phat, double *out, const SolverState *st,
+                                                     SolverState *host) {
+    if (blockIdx.x == 0 && threadIdx.x < kStateWords)
+        __hip_atomic_store(reinterpret_cast<uint64_t *>(host) + threadIdx.x,
+                           reinterpret_cast<const uint64_t *>(st)[threadIdx.x], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (int64_t)n * bs) return;
+    const int64_t k = i / bs, c = i - k * bs;
+    out[(int64_t)perm[k] * bs + c] = finished_x(x, phat, i, phat && st->last_half == 1, st->alpha);
 }
 
 // dst block k = src block idx[k] (idx null: identity), optionally transposed

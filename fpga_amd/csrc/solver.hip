@@ -638,7 +638,9 @@ struct bda_handle_s {
     int32_t partial_cap = 0;
     bda::DBuf<bda::SolverState> st;
     bda::SolverState *h_st = nullptr;  // pinned
-    int32_t *h_done = nullptr;          // mapped host flags, one per state: the id of the run that stopped
+    bda::SolverState *d_host_st = nullptr;  // its device address
+    int32_t *h_done = nullptr;          // mapped host flags, one per state: the id of the run that stopped;
+                                        // then the factorisation's bad row (kBadRow)
     int32_t *d_done = nullptr;          // their device address
     uint64_t *h_prog = nullptr;         // mapped progress words, one per state (run id << 32 | count)
     uint64_t *d_prog = nullptr;
@@ -720,6 +722,13 @@ void copy_sync(H &h, void *dst, const void *src, size_t bytes, hipMemcpyKind kin
     HIP_CHECK(hipStreamSynchronize(h.stream));
 }
 
+// A host array to the device without a wait of its own: for calls that wait
+// for the stream before they return, also with an error (guarded), so the
+// array outlives the copy.
+void copy_in(H &h, void *dst, const void *src, size_t bytes) {
+    HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h.stream));
+}
+
 int blocks_for(int64_t work, int tpb) { return (int)((work + tpb - 1) / tpb); }
 
 void prof_begin(H &h, int kind) {
@@ -765,6 +774,7 @@ void check_launch() { HIP_CHECK(hipGetLastError()); }
 // with folded scalar steps takes its state to kStateB after alpha and after
 // omega, and back to slot 0 after the ||s|| test and after beta.
 constexpr int kIdleState = 2, kStateB = 3, kStates = 4;
+constexpr int kBadRow = 2;  // its place among the mapped flags
 
 RedArgs red(H &h, int state_idx, int fin) {
     RedArgs ra;
@@ -815,7 +825,7 @@ int stream_dispatch(H &h, const StreamArgs<TV, TX> &a) {
 // --- streaming kernel launch over the tiles of one colour (or all) ---------
 // prof_kind >= 0: with profiling on, the streaming kernel alone (not its
 // finalize) is bracketed by an event pair of that kind.
-// ZX: a step-0 residual that takes the short path when k_mark_nonzero left
+// ZX: a step-0 residual that takes the short path when k_gather_start left
 // the state's full_residual clear (zero start vector, finite matrix).
 // colour kRestOfRows (the product only): every colour but the first, whose
 // rows' partial sums launch_sweep_spmv has left in their slots.
@@ -1305,39 +1315,48 @@ int32_t init_state(H &h, int idx, double tol, int maxit, bool abs_mode) {
     return s.run_id;
 }
 
+// The start and the end of a solve on the caller's vectors.
+void gather_start(H &h, const double *d_b, double *bp, const double *d_x, double *xp, SolverState *st) {
+    hipLaunchKernelGGL(k_gather_start, dim3(blocks_for((int64_t)h.N(), 256)), dim3(256), 0, h.stream, h.n, h.bs,
+                       h.d_perm.p, d_b, bp, d_x, xp, (const int32_t *)h.d_nonfinite.p, st);
+    check_launch();
+}
+// x and the state (to h.h_st), complete on return
+void scatter_end(H &h, const double *x, const double *phat, double *d_x, const SolverState *st) {
+    hipLaunchKernelGGL(k_scatter_end, dim3(blocks_for((int64_t)h.N(), 256)), dim3(256), 0, h.stream, h.n, h.bs,
+                       h.d_perm.p, x, phat, d_x, st, h.d_host_st);
+    check_launch();
+    HIP_CHECK(hipStreamSynchronize(h.stream));
+}
+
 // One BiCGSTAB run following the reference microprogram (solver_pkg.vhd:120-141).
-// zero_x0: x0 = 0 and the initial residual is the right-hand side itself.
-// outer != nullptr: an inner run of the precision form; its tolerance comes
-// from the outer state on the device, and the run ends without reading its
-// state back (the outer state collects the counters).
+// outer == nullptr: a solve of the caller's d_b into d_x (also the start
+// vector); rhs is d_b in colour order.
+// outer != nullptr: an inner run of the precision form from x0 = 0, whose
+// initial residual is the right-hand side itself; its tolerance comes from
+// the outer state on the device, and the run ends without reading its state
+// back (the outer state collects the counters).
 template <int BS, typename TV, typename TX>
-RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs, bool zero_x0, double tol,
-                    int maxit, bool abs_mode, const SolverState *outer = nullptr) {
+RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs, const double *d_b, double *d_x,
+                    double tol, int maxit, bool abs_mode, const SolverState *outer = nullptr) {
     const size_t N = h.N();
     const int vb = vec_blocks(N);
+    RunOut out;
+    const auto t0 = std::chrono::steady_clock::now();
+    h.prof_tag = -1;
     int32_t run_id;
     if (outer) {
         const SolverState s = new_state(h, 0, 0.0, maxit, false);
         run_id = s.run_id;
-        hipLaunchKernelGGL(k_inner_start, dim3(1), dim3(1), 0, h.stream, h.st.p, outer, s);
-        check_launch();
-    } else {
-        run_id = init_state(h, 0, tol, maxit, abs_mode);
-    }
-    RunOut out;
-    const auto t0 = std::chrono::steady_clock::now();
-    h.prof_tag = -1;
-    if (zero_x0) {
         hipLaunchKernelGGL((k_init_zero_x0<TX, TX>), dim3(vb), dim3(kVecThreads), 0, h.stream, (int64_t)N, rhs,
-                           k.rt.p, k.r.p, k.p.p, k.x.p, red(h, 0, FIN_INIT));
+                           k.rt.p, k.r.p, k.p.p, k.x.p, red(h, 0, FIN_INIT), outer, s);
         check_launch();
         launch_finalize(h, 1, red(h, 0, FIN_INIT), vb);
     } else {
         if constexpr (std::is_same<TX, double>::value) {
             // r = b - A x0; with x0 = 0 (and a finite matrix) this is b, without the product
-            hipLaunchKernelGGL((k_mark_nonzero<TX>), dim3(vb), dim3(kVecThreads), 0, h.stream, (int64_t)N,
-                               (const TX *)k.x.p, (const int32_t *)h.d_nonfinite.p, h.st.p);
-            check_launch();
+            run_id = init_state(h, 0, tol, maxit, abs_mode);
+            gather_start(h, d_b, h.bp.p, d_x, k.x.p, h.st.p);
             launch_stream<BS, SM_SUB, SR_SELF, TV, TX, true>(h, *op.A, op.Aval, -1, k.x.p, rhs, k.rt.p, nullptr,
                                                              nullptr, red(h, 0, FIN_INIT), true, k.r.p, k.p.p,
                                                              nullptr, 0, PK_SPMV);
@@ -1454,19 +1473,17 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
         }
         prof_end(h);
     }
-    // x += alpha phat of a run that ended after a first half-iteration (the
-    // x update of a first half is otherwise applied by the next k_update_xr)
-    hipLaunchKernelGGL((k_finish_x<TX, TX>), dim3(vb), dim3(kVecThreads), 0, h.stream, (int64_t)N, k.x.p, k.phat.p,
-                       (const SolverState *)(h.st.p));
-    check_launch();
+    // (x += alpha phat of a run that ended after a first half-iteration, which
+    // the next k_update_xr otherwise applies, comes with the result's way out)
     if (outer) {
         h.prof_tag = -1;
         return out;
     }
-    HIP_CHECK(hipStreamSynchronize(h.stream));
-    out.ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-    copy_sync(h, h.h_st, h.st.p, sizeof(SolverState), hipMemcpyDeviceToHost);
-    out.st = *h.h_st;
+    if constexpr (std::is_same<TX, double>::value) {
+        scatter_end(h, k.x.p, k.phat.p, d_x, h.st.p);
+        out.ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+        out.st = *h.h_st;
+    }
     prof_collect(h, out.st.no_results ? -1 : out.st.h);
     h.prof_tag = -1;
     return out;
@@ -1642,10 +1659,9 @@ void do_factor(H &h) {
     if (!h.have_values) throw std::runtime_error("no matrix values uploaded");
     constexpr int BB = BS * BS;
     const Analysis &an = h.an;
-    const int32_t big = INT_MAX, zero = 0;
     const auto t0 = std::chrono::steady_clock::now();
-    HIP_CHECK(hipMemcpyAsync(h.d_bad.p, &big, 4, hipMemcpyHostToDevice, h.stream));
-    HIP_CHECK(hipMemcpyAsync(h.d_nonfinite.p, &zero, 4, hipMemcpyHostToDevice, h.stream));
+    hipLaunchKernelGGL(k_factor_begin, dim3(1), dim3(1), 0, h.stream, h.d_bad.p, h.d_nonfinite.p);
+    check_launch();
     const bool f32 = h.mixed_used;
     if (f32) mixed_buffers<BS>(h);
     if (an.ncolours > 1) h.A0d64.ensure((size_t)an.colour_ptr[1] * BB);
@@ -1674,20 +1690,18 @@ void do_factor(H &h) {
         hipLaunchKernelGGL((k_ilu0_tile<BS>), dim3(a.ntiles), dim3(64 * BS), 0, h.stream, a);
         check_launch();
     }
-    int32_t bad = 0;
-    HIP_CHECK(hipMemcpyAsync(&bad, h.d_bad.p, 4, hipMemcpyDeviceToHost, h.stream));
+    gather_low2<BS>(h);
+    if (f32) gather_low2_32<BS>(h);
+    hipLaunchKernelGGL(k_factor_end, dim3(1), dim3(1), 0, h.stream, (const int32_t *)h.d_bad.p, h.d_done + kBadRow);
+    check_launch();
     HIP_CHECK(hipStreamSynchronize(h.stream));
+    const int32_t bad = __atomic_load_n(h.h_done + kBadRow, __ATOMIC_ACQUIRE);
     if (bad != INT_MAX)
         throw std::runtime_error("singular diagonal block in ILU0 at colour-ordered row " + std::to_string(bad) +
                                  " (original row " + std::to_string(an.perm[bad]) + ")");
     bda::info(1, "INFO: factor: block ILU0 of %d block rows over %d colours, %.3f ms", h.n, an.ncolours,
               std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count());
-    gather_low2<BS>(h);
-    if (f32) {
-        gather_low2_32<BS>(h);
-        h.copies_gen = h.factor_gen + 1;
-    }
-    HIP_CHECK(hipStreamSynchronize(h.stream));
+    if (f32) h.copies_gen = h.factor_gen + 1;
     h.factored = true;
     h.u0_is_a = true;
     h.factor_gen++;
@@ -1822,12 +1836,6 @@ void log_result(const char *what, const bda_result &r) {
               r.norms[2], r.norms[3], r.last_norm_idx);
 }
 
-void gather_vec2(H &h, const double *in1, double *out1, const double *in2, double *out2) {
-    hipLaunchKernelGGL(k_gather_rows2, dim3(blocks_for((int64_t)h.N(), 256)), dim3(256), 0, h.stream, h.n, h.bs,
-                       h.d_perm.p, in1, out1, in2, out2);
-    check_launch();
-}
-
 void gather_vec(H &h, const double *in, double *out) {
     hipLaunchKernelGGL(k_gather_rows, dim3(blocks_for((int64_t)h.N(), 256)), dim3(256), 0, h.stream, h.n, h.bs,
                        h.d_perm.p, in, out);
@@ -1850,11 +1858,8 @@ void solve_dev(H &h, const double *d_b, double *d_x, double tol, int maxit, bda_
     require_factored(h);
     check_solve_args(tol, maxit);
     if (adjoint) ensure_adjoint<BS>(h);
-    gather_vec2(h, d_b, h.bp.p, d_x, h.k64.x.p);
     OpSet<double> op = adjoint ? op_adj64(h) : op_fwd64(h);
-    RunOut o = run_bicgstab<BS, double, double>(h, op, h.k64, h.bp.p, false, tol, maxit, h.abs_tol != 0);
-    scatter_vec(h, h.k64.x.p, d_x);
-    HIP_CHECK(hipStreamSynchronize(h.stream));
+    RunOut o = run_bicgstab<BS, double, double>(h, op, h.k64, h.bp.p, d_b, d_x, tol, maxit, h.abs_tol != 0);
     bda_result r;
     fill_result(o, &r);
     if (res) *res = r;
@@ -1865,18 +1870,18 @@ void solve_dev(H &h, const double *d_b, double *d_x, double tol, int maxit, bda_
 
 // precision form: FP64 refinement around FP32-value inner solves.  The outer
 // loop runs on the device: the FP64 residual's epilogue (FIN_REFINE) makes
-// the stop decisions and sets the next inner tolerance, k_inner_start and
-// k_refine_step link the inner runs to the outer state.  The host waits once
+// the stop decisions and sets the next inner tolerance, inner_start and
+// refine_step link the inner runs to the outer state.  The host waits once
 // per outer step, after the residual, to learn whether another inner run is
 // needed.
 template <int BS, typename TX>
 bool mixed_inner(H &h, Krylov<TX> &k, int inner_maxit, bool adjoint) {
     OpSet<float> op = adjoint ? op_adj32(h) : op_fwd32(h);
-    const RunOut o = run_bicgstab<BS, float, TX>(h, op, k, h.ro.p, true, 0.0, inner_maxit, false, h.st.p + 1);
+    const RunOut o = run_bicgstab<BS, float, TX>(h, op, k, h.ro.p, nullptr, nullptr, 0.0, inner_maxit, false,
+                                                 h.st.p + 1);
     hipLaunchKernelGGL((k_add_correction<TX>), dim3(blocks_for((int64_t)h.N(), kVecThreads)), dim3(kVecThreads), 0,
-                       h.stream, (int64_t)h.N(), h.xo.p, (const TX *)k.x.p, (const SolverState *)h.st.p);
-    check_launch();
-    hipLaunchKernelGGL(k_refine_step, dim3(1), dim3(1), 0, h.stream, h.st.p + 1, (const SolverState *)h.st.p);
+                       h.stream, (int64_t)h.N(), h.xo.p, (const TX *)k.x.p, (const TX *)k.phat.p,
+                       (const SolverState *)h.st.p, h.st.p + 1);
     check_launch();
     return o.aborted;
 }
@@ -1896,7 +1901,6 @@ void solve_mixed_dev(H &h, const double *d_b, double *d_x, double tol, int max_o
     const double *Mval = adjoint ? h.At64.p : h.A64.p;
     if (vec32) h.k32.ensure(h.Npad());
     const auto t0 = std::chrono::steady_clock::now();
-    gather_vec2(h, d_b, h.bp.p, d_x, h.xo.p);
     SolverState os = new_state(h, 1, tol, 0, h.abs_tol != 0);
     os.max_outer = max_outer;
     os.inner_tol = inner_tol;
@@ -1904,14 +1908,12 @@ void solve_mixed_dev(H &h, const double *d_b, double *d_x, double tol, int max_o
     os.adaptive = h.refine_adaptive;
     hipLaunchKernelGGL(k_set_state, dim3(1), dim3(1), 0, h.stream, h.st.p + 1, os);
     check_launch();
+    gather_start(h, d_b, h.bp.p, d_x, h.xo.p, h.st.p + 1);
     bool aborted = false;
     for (int outer = 0;; ++outer) {
         // FP64 true residual ro = b - A x and the outer step's decisions; the
         // first one is b without the product when x = 0 and A is finite
         if (outer == 0) {
-            hipLaunchKernelGGL((k_mark_nonzero<double>), dim3(vec_blocks(h.N())), dim3(kVecThreads), 0, h.stream,
-                               (int64_t)h.N(), (const double *)h.xo.p, (const int32_t *)h.d_nonfinite.p, h.st.p + 1);
-            check_launch();
             launch_stream<BS, SM_SUB, SR_SELF, double, double, true>(h, M, Mval, -1, h.xo.p, h.bp.p, h.ro.p,
                                                                      nullptr, nullptr, red(h, 1, FIN_REFINE), true);
         } else {
@@ -1943,10 +1945,8 @@ void solve_mixed_dev(H &h, const double *d_b, double *d_x, double tol, int max_o
             break;
         }
     }
-    scatter_vec(h, h.xo.p, d_x);
-    HIP_CHECK(hipStreamSynchronize(h.stream));
+    scatter_end(h, h.xo.p, nullptr, d_x, h.st.p + 1);
     prof_collect(h);  // inner runs are not filtered: their no-op launches count too
-    copy_sync(h, h.h_st, h.st.p + 1, sizeof(SolverState), hipMemcpyDeviceToHost);
     const SolverState s = *h.h_st;
     bda_result r;
     std::memset(&r, 0, sizeof(r));
@@ -2233,10 +2233,12 @@ int guarded(bda_handle h, F &&f) {
         f();
         return 0;
     } catch (const std::exception &e) {
+        (void)hipStreamSynchronize(h->stream);  // no copy of the caller's arrays outlives the call
         h->err = e.what();
         bda::info(1, "ERROR: %s", e.what());
         return 1;
     } catch (...) {
+        (void)hipStreamSynchronize(h->stream);
         h->err = "unknown error";
         bda::info(1, "ERROR: unknown error");
         return 1;
@@ -2276,8 +2278,9 @@ int bda_create(int32_t bs, int32_t n, int32_t nnzb_max, bda_handle *out) {
         // produced there are complete before the handle reads them
         HIP_CHECK(hipStreamCreate(&h->stream));
         h->st.ensure(kStates);  // DBuf zero-fills: the idle slot never has done set
-        HIP_CHECK(hipHostMalloc((void **)&h->h_st, sizeof(SolverState), hipHostMallocDefault));
-        HIP_CHECK(hipHostMalloc((void **)&h->h_done, 2 * sizeof(int32_t), hipHostMallocMapped));
+        HIP_CHECK(hipHostMalloc((void **)&h->h_st, sizeof(SolverState), hipHostMallocMapped));
+        HIP_CHECK(hipHostGetDevicePointer((void **)&h->d_host_st, h->h_st, 0));
+        HIP_CHECK(hipHostMalloc((void **)&h->h_done, (kBadRow + 1) * sizeof(int32_t), hipHostMallocMapped));
         h->h_done[0] = h->h_done[1] = 0;
         HIP_CHECK(hipHostGetDevicePointer((void **)&h->d_done, h->h_done, 0));
         HIP_CHECK(hipHostMalloc((void **)&h->h_prog, 2 * sizeof(uint64_t), hipHostMallocMapped));
@@ -2488,8 +2491,8 @@ int bda_solve(bda_handle h, const double *b, double *x, double tol, int32_t maxi
     return guarded(h, [&] {
         if (!b || !x) throw std::runtime_error("null vector");
         require_factored(*h);
-        copy_sync(*h, h->vin.p, b, h->N() * 8, hipMemcpyHostToDevice);
-        copy_sync(*h, h->vout.p, x, h->N() * 8, hipMemcpyHostToDevice);
+        copy_in(*h, h->vin.p, b, h->N() * 8);
+        copy_in(*h, h->vout.p, x, h->N() * 8);
         BS_CALL(h, solve_dev, *h, h->vin.p, h->vout.p, tol, maxit, res, false);
         copy_sync(*h, x, h->vout.p, h->N() * 8, hipMemcpyDeviceToHost);
     });
@@ -2524,8 +2527,8 @@ int bda_solve_mixed(bda_handle h, const double *b, double *x, double tol, int32_
     return guarded(h, [&] {
         if (!b || !x) throw std::runtime_error("null vector");
         require_factored(*h);
-        copy_sync(*h, h->vin.p, b, h->N() * 8, hipMemcpyHostToDevice);
-        copy_sync(*h, h->vout.p, x, h->N() * 8, hipMemcpyHostToDevice);
+        copy_in(*h, h->vin.p, b, h->N() * 8);
+        copy_in(*h, h->vout.p, x, h->N() * 8);
         BS_CALL(h, solve_mixed_dev, *h, h->vin.p, h->vout.p, tol, max_outer, inner_tol, inner_maxit, vec32, res);
         copy_sync(*h, x, h->vout.p, h->N() * 8, hipMemcpyDeviceToHost);
     });
@@ -2540,8 +2543,8 @@ int bda_adjoint_solve(bda_handle h, const double *w, double *lambda, double tol,
     return guarded(h, [&] {
         if (!w || !lambda) throw std::runtime_error("null vector");
         require_factored(*h);
-        copy_sync(*h, h->vin.p, w, h->N() * 8, hipMemcpyHostToDevice);
-        copy_sync(*h, h->vout.p, lambda, h->N() * 8, hipMemcpyHostToDevice);
+        copy_in(*h, h->vin.p, w, h->N() * 8);
+        copy_in(*h, h->vout.p, lambda, h->N() * 8);
         BS_CALL(h, solve_dev, *h, h->vin.p, h->vout.p, tol, maxit, res, true);
         copy_sync(*h, lambda, h->vout.p, h->N() * 8, hipMemcpyDeviceToHost);
     });
@@ -2559,8 +2562,8 @@ int bda_adjoint_solve_mixed(bda_handle h, const double *w, double *lambda, doubl
     return guarded(h, [&] {
         if (!w || !lambda) throw std::runtime_error("null vector");
         require_factored(*h);
-        copy_sync(*h, h->vin.p, w, h->N() * 8, hipMemcpyHostToDevice);
-        copy_sync(*h, h->vout.p, lambda, h->N() * 8, hipMemcpyHostToDevice);
+        copy_in(*h, h->vin.p, w, h->N() * 8);
+        copy_in(*h, h->vout.p, lambda, h->N() * 8);
         BS_CALL(h, solve_mixed_dev, *h, h->vin.p, h->vout.p, tol, max_outer, inner_tol, inner_maxit, vec32, res,
                 true);
         copy_sync(*h, lambda, h->vout.p, h->N() * 8, hipMemcpyDeviceToHost);
@@ -2577,8 +2580,8 @@ int bda_grad_values(bda_handle h, const double *lambda, const double *x, double 
         require_analysed(*h);
         const size_t nv = (size_t)h->A.nnzb * h->bs * h->bs;
         h->ggrad.ensure(nv);
-        copy_sync(*h, h->vin.p, lambda, h->N() * 8, hipMemcpyHostToDevice);
-        copy_sync(*h, h->vout.p, x, h->N() * 8, hipMemcpyHostToDevice);
+        copy_in(*h, h->vin.p, lambda, h->N() * 8);
+        copy_in(*h, h->vout.p, x, h->N() * 8);
         BS_CALL(h, grad_dev, *h, h->vin.p, h->vout.p, h->ggrad.p);
         copy_sync(*h, grad, h->ggrad.p, nv * 8, hipMemcpyDeviceToHost);
     });
