@@ -632,6 +632,9 @@ struct StreamArgs {
     const int32_t *rowptr2 = nullptr;  // SUB_Z: the second sweep's row pointers
     TX *zout = nullptr;                // SUB_Z: z of the rows without second-sweep blocks
     const int32_t *rowmap = nullptr;   // dependency tiles (k_lower2): matrix row of each packed row
+    TX *reset = nullptr;               // waiting tiles: entries to mark as not written (see k_sweep_wait)
+    int32_t *fail = nullptr;           // waiting tiles: a wait has run out; on the device, and for the host
+    int32_t *host_fail = nullptr;
     const TV *adiag = nullptr;         // SUB_SPMV: A's diagonal blocks of colour 0
     TX *vout = nullptr;                // SUB_SPMV: v = A out of the tile's rows
 };
@@ -648,6 +651,38 @@ __device__ inline double prod<float, double>(float a, double x) { return (double
 template <typename T> __device__ inline T from_double(double v);
 template <> __device__ inline double from_double<double>(double v) { return v; }
 template <> __device__ inline float from_double<float>(double v) { return (float)v; }
+
+// The waiting sweeps' vector entries (k_sweep_wait): an entry not yet written
+// holds a NaN of this one bit pattern; a result that happens to be that NaN is
+// stored as the ordinary one.  Entries are read and written with relaxed
+// agent-scope atomics, whole (so the entry is its own flag, and no other
+// ordering is needed).
+template <typename T> struct NotYet;
+template <> struct NotYet<double> {
+    using Bits = uint64_t;
+    static constexpr uint64_t mark = 0x7FF8BDA5BDA5BDA5ull, nan = 0x7FF8000000000000ull;
+};
+template <> struct NotYet<float> {
+    using Bits = uint32_t;
+    static constexpr uint32_t mark = 0x7FC0BDA5u, nan = 0x7FC00000u;
+};
+template <typename T> __device__ inline typename NotYet<T>::Bits load_entry(const T *p) {
+    return __hip_atomic_load(reinterpret_cast<const typename NotYet<T>::Bits *>(p), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T> __device__ inline void store_entry(T *p, T v) {
+    typename NotYet<T>::Bits b;
+    __builtin_memcpy(&b, &v, sizeof(T));
+    if (b == NotYet<T>::mark) b = NotYet<T>::nan;
+    __hip_atomic_store(reinterpret_cast<typename NotYet<T>::Bits *>(p), b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T> __device__ inline void mark_entry(T *p) {
+    *reinterpret_cast<typename NotYet<T>::Bits *>(p) = NotYet<T>::mark;
+}
+// Ticks of the wall clock (100 MHz) after which a wait is given up: 2 s, far
+// beyond any sweep.  Nothing waits that long (see k_sweep_wait); it bounds
+// the loop whatever happens.
+constexpr uint64_t kWaitTicks = 200000000;
 
 // Map workgroups to tiles so that each XCD (workgroups are dispatched to the
 // 8 XCDs round-robin) works on one contiguous range of tiles and the x
@@ -790,7 +825,9 @@ __device__ inline double *tile_tv() {
 // packed row's matrix row, for its right-hand side); its outputs only go to
 // keep[]; 2, a tile whose column indices below zero name a row of the
 // dependency tile: -1 - c is the row's place there, and its x comes from
-// ldsx[] (that tile's keep[]) instead of memory.
+// ldsx[] (that tile's keep[]) instead of memory.  3, a tile of a waiting sweep
+// (k_sweep_wait): its x entries are waited for, its outputs are stored for
+// tiles that wait.
 template <int BS, int MODE, int RED, typename TV, typename TX, int ROWS, bool KEEP, bool PLAIN = false, int V = 0>
 __device__ __attribute__((always_inline)) inline void stream_tile(const StreamArgs<TV, TX> &a, const int4 d, TX *keep,
                                                                    int slot, const TX *ldsx = nullptr) {
@@ -938,6 +975,51 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
     XVec<TX, BS> xg[XV];
     int xq[XV];
     int xl[XV];
+    if constexpr (V == 3) {
+        using Bits = typename NotYet<TX>::Bits;
+        const TX *src[XV];
+        bool ready[XV], free[XV], all = false;  // free: nothing to wait for
+#pragma unroll
+        for (int j = 0; j < XV; ++j) {
+            xq[j] = min(t + j * NT, nblk > 0 ? nblk - 1 : 0);
+            const int cb = nblk > 0 ? scol[xq[j]] : 0;
+            src[j] = (cb < a.split ? a.x_lo : a.x) + (size_t)cb * BS;
+            ready[j] = false;
+            free[j] = nblk == 0 || cb < a.split;
+        }
+        uint64_t since = 0;
+        for (uint32_t spin = 0; !all; ++spin) {
+            if (spin > 0) {
+                __builtin_amdgcn_s_sleep(1);
+                if ((spin & 255) == 0) {
+                    const uint64_t now = wall_clock64();
+                    if (since == 0) since = now;
+                    bool over = __hip_atomic_load(a.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+                    if (!over && now - since > kWaitTicks) {
+                        over = true;
+                        __hip_atomic_store(a.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        __hip_atomic_store(a.host_fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    }
+                    if (over) break;
+                }
+            }
+            all = true;
+            Bits w[XV][BS];
+#pragma unroll
+            for (int j = 0; j < XV; ++j)
+#pragma unroll
+                for (int c = 0; c < BS; ++c) w[j][c] = load_entry(src[j] + c);
+#pragma unroll
+            for (int j = 0; j < XV; ++j) {
+                bool r = true;
+#pragma unroll
+                for (int c = 0; c < BS; ++c) r = r && w[j][c] != NotYet<TX>::mark;
+                if (!ready[j]) __builtin_memcpy(&xg[j], w[j], sizeof(xg[j]));
+                ready[j] = ready[j] || r || free[j];
+                all = all && ready[j];
+            }
+        }
+    } else
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
         const int q = min(t + j * NT, nblk > 0 ? nblk - 1 : 0);
@@ -1120,7 +1202,10 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
         const TX o = from_double<TX>(res[s]);
         if constexpr (KEEP) keep[t] = o;
         if constexpr (MODE == SM_SUB_SPMV) a.vout[gi[s]] = o;
-        else if constexpr (V != 1) {
+        else if constexpr (V == 3) {
+            store_entry(&a.out[gi[s]], o);
+            if (a.reset) mark_entry(&a.reset[gi[s]]);
+        } else if constexpr (V != 1) {
             a.out[gi[s]] = o;
             if (a.out2) a.out2[gi[s]] = o;
             if (a.out3) a.out3[gi[s]] = o;
@@ -1465,6 +1550,65 @@ __global__ __launch_bounds__(64 * BS) void k_lower2(StreamArgs<TV, TX> a, Stream
     stream_tile<BS, SM_SUB, SR_NONE, TV, TX, 64, true, plain_small<TV>(), 1>(v, dv, ydep, 0);
     __syncthreads();
     stream_tile<BS, MODEB, SR_NONE, TV, TX, 64, false, plain_small<TV>(), 2>(g, dg, nullptr, 0, ydep);
+}
+
+// ---------------------------------------------------------------------------
+// A whole sweep in one launch, for orderings of many small levels.  Workgroups
+// take tiles in level order from a ticket counter; a tile loads what does not
+// depend on other tiles, then waits for the x entries it reads, entry by
+// entry (NotYet): the hop from one level to the next is one store and one
+// load instead of a launch.  Every tile waits only for tiles of earlier
+// tickets, each held by a workgroup that runs and itself waits only for
+// earlier ones, so the first unfinished tile never waits and the sweep ends
+// however few workgroups are resident; ticket numbers are bounded, so every
+// workgroup ends.
+//
+// The first sweep writes y, except that the last level (which has no blocks
+// in the second sweep) goes to z with the diagonal inverse, as when launched
+// by itself; it marks the other z entries as not written, the second sweep
+// the y entries, and each clears the other's ticket counter: y and the
+// counters only have to be prepared once per run (k_sweep_reset).  The
+// arithmetic is k_stream's.
+template <typename TX>
+struct WaitArgs {
+    int32_t *ticket, *other;   // this sweep's ticket counter and the other's
+    int32_t ntiles;
+    int32_t reverse;           // levels descending: the tiles from the last to the first
+    const TX *rhs_lo;          // right-hand side of the rows below rhs_split
+    int32_t rhs_split;
+    int32_t last_row0;         // rows from here on: z = D^-1 (rhs - S1 y) (first sweep)
+    TX *z;
+};
+
+template <int BS, int MODE, typename TV, typename TX>
+__global__ __launch_bounds__(64 * BS) void k_sweep_wait(StreamArgs<TV, TX> a, WaitArgs<TX> w) {
+    if (a.ra.st->done) return;
+    __shared__ int tk;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *w.other = 0;
+    for (;;) {
+        if (threadIdx.x == 0) tk = __hip_atomic_fetch_add(w.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        const int k = tk;
+        if (k >= w.ntiles) return;
+        const int4 d = a.tile[a.tile0 + (w.reverse ? w.ntiles - 1 - k : k)];
+        StreamArgs<TV, TX> b = a;
+        if (d.x < w.rhs_split) b.rhs = w.rhs_lo;
+        if (d.x >= w.last_row0) {
+            b.out = w.z;
+            b.reset = nullptr;
+            stream_tile<BS, SM_SUB_DINV, SR_NONE, TV, TX, 64, false, plain_small<TV>(), 3>(b, d, nullptr, 0);
+        } else {
+            stream_tile<BS, MODE, SR_NONE, TV, TX, 64, false, plain_small<TV>(), 3>(b, d, nullptr, 0);
+        }
+        __syncthreads();  // the tile's LDS, and tk
+    }
+}
+
+template <typename TX>
+__global__ __launch_bounds__(256) void k_sweep_reset(int64_t N, TX *y, int32_t *tickets) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < N) mark_entry(&y[i]);
+    if (i < 3) tickets[i] = 0;   // both counters and the fail flag
 }
 
 // ---------------------------------------------------------------------------

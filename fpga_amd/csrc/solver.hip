@@ -574,6 +574,11 @@ enum ProfKind { PK_SPMV = 0, PK_LOWER = 1, PK_UPPER = 2, PK_VEC = 3, PK_N = 4 };
 #ifndef BDA_FOLD
 #define BDA_FOLD 1
 #endif
+// 1 (default): a solve's sweeps over many levels in one launch each; 0: one
+// launch per level (the same results, for A/B timing)
+#ifndef BDA_WAIT
+#define BDA_WAIT 1
+#endif
 // 1 (default): k_finalize_joint for 2,049 to 18,432 partials; 0: k_finalize
 // (the same sums, for A/B timing)
 #ifndef BDA_FIN_JOINT
@@ -622,6 +627,7 @@ struct bda_handle_s {
     // U's colour-0 rows are A's own blocks: true of factors made by
     // bda_factor, not known of a caller's own (bda_upload_factored)
     bool u0_is_a = false;
+    bool wait = BDA_WAIT != 0;    // sweeps of many levels in one launch each (k_sweep_wait)
     bool fold = BDA_FOLD != 0;    // scalar steps folded into the vector updates (small systems)
     bool fuse0 = BDA_FUSE0 != 0;  // the second sweep of colour 0 with the product's (SM_SUB_SPMV)
 
@@ -640,7 +646,8 @@ struct bda_handle_s {
     bda::SolverState *h_st = nullptr;  // pinned
     bda::SolverState *d_host_st = nullptr;  // its device address
     int32_t *h_done = nullptr;          // mapped host flags, one per state: the id of the run that stopped;
-                                        // then the factorisation's bad row (kBadRow)
+                                        // then kBadRow and kSweepFail
+    bda::DBuf<int32_t> d_sweep;         // waiting sweeps: two ticket counters, and whether a wait ran out
     int32_t *d_done = nullptr;          // their device address
     uint64_t *h_prog = nullptr;         // mapped progress words, one per state (run id << 32 | count)
     uint64_t *d_prog = nullptr;
@@ -774,7 +781,7 @@ void check_launch() { HIP_CHECK(hipGetLastError()); }
 // with folded scalar steps takes its state to kStateB after alpha and after
 // omega, and back to slot 0 after the ||s|| test and after beta.
 constexpr int kIdleState = 2, kStateB = 3, kStates = 4;
-constexpr int kBadRow = 2;  // its place among the mapped flags
+constexpr int kBadRow = 2, kSweepFail = 3, kFlags = 4;  // places among the mapped flags
 
 RedArgs red(H &h, int state_idx, int fin) {
     RedArgs ra;
@@ -1215,6 +1222,85 @@ void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si, bool 
     prof_end(h);
 }
 
+// A solve runs its sweeps as two launches whose tiles wait for one another
+// (k_sweep_wait) where the launches per level would be latency-bound.
+constexpr int kWaitFromLevels = 16;
+constexpr int kWaitLevelsAhead = 6;
+bool sweeps_wait(const H &h) { return h.wait && h.an.ncolours >= kWaitFromLevels; }
+
+// Workgroups of a waiting sweep: enough for kWaitLevelsAhead of its widest
+// levels, so that a level's tiles have loaded their operands when their turn
+// comes, and few enough that those waiting do not crowd the memory system.
+int wait_grid(const DevMat &m, int c0, int c1) {
+    int widest = 1;
+    for (int c = c0; c < c1; ++c) widest = std::max(widest, m.colour_tile[c + 1] - m.colour_tile[c]);
+    return std::min({m.colour_tile[c1] - m.colour_tile[c0], std::max(64, kWaitLevelsAhead * widest), 2048});
+}
+
+template <int BS, typename TV, typename TX>
+void precond_wait(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si) {
+    const int nc = h.an.ncolours;
+    if (op.s1_dinv == op.s2_dinv) throw std::runtime_error("exactly one sweep carries the diagonal inverse");
+    const bool skip0 = !op.s1_dinv;
+    const int c0 = skip0 ? 1 : 0;
+    const DevMat &m1 = *op.S1, &m2 = *op.S2;
+    StreamArgs<TV, TX> a;
+    std::memset(&a, 0, sizeof(a));
+    a.tile = m1.tile.p;
+    a.tile0 = m1.colour_tile[c0];
+    a.rowptr = m1.rowptr.p;
+    a.colidx = m1.colidx.p;
+    a.val = op.S1val;
+    a.x = y;
+    a.x_lo = skip0 ? p : y;
+    a.split = skip0 ? h.an.colour_ptr[1] : 0;
+    a.rhs = p;
+    a.out = y;
+    a.reset = z;
+    a.dinv = op.dinv;
+    a.fail = h.d_sweep.p + 2;
+    a.host_fail = h.d_done + kSweepFail;
+    a.ra = red(h, si, FIN_NONE);
+    WaitArgs<TX> w;
+    w.ticket = h.d_sweep.p;
+    w.other = h.d_sweep.p + 1;
+    w.ntiles = m1.colour_tile[nc] - m1.colour_tile[c0];
+    w.reverse = 0;
+    w.rhs_lo = nullptr;
+    w.rhs_split = 0;
+    w.last_row0 = h.an.colour_ptr[nc - 1];
+    w.z = z;
+    prof_begin(h, PK_LOWER);
+    const dim3 g1(wait_grid(m1, c0, nc)), b(64 * BS);
+    if (op.s1_dinv) hipLaunchKernelGGL((k_sweep_wait<BS, SM_SUB_DINV, TV, TX>), g1, b, 0, h.stream, a, w);
+    else hipLaunchKernelGGL((k_sweep_wait<BS, SM_SUB, TV, TX>), g1, b, 0, h.stream, a, w);
+    check_launch();
+    prof_end(h);
+    a.tile = m2.tile.p;
+    a.tile0 = 0;
+    a.rowptr = m2.rowptr.p;
+    a.colidx = m2.colidx.p;
+    a.val = op.S2val;
+    a.x = a.x_lo = z;
+    a.split = 0;
+    a.rhs = y;
+    a.out = z;
+    a.reset = y;
+    w.ticket = h.d_sweep.p + 1;
+    w.other = h.d_sweep.p;
+    w.ntiles = m2.colour_tile[nc - 1];
+    w.reverse = 1;
+    w.rhs_lo = p;
+    w.rhs_split = skip0 ? h.an.colour_ptr[1] : 0;
+    w.last_row0 = INT_MAX;
+    prof_begin(h, PK_UPPER);
+    const dim3 g2(wait_grid(m2, 0, nc - 1));
+    if (op.s2_dinv) hipLaunchKernelGGL((k_sweep_wait<BS, SM_SUB_DINV, TV, TX>), g2, b, 0, h.stream, a, w);
+    else hipLaunchKernelGGL((k_sweep_wait<BS, SM_SUB, TV, TX>), g2, b, 0, h.stream, a, w);
+    check_launch();
+    prof_end(h);
+}
+
 // Kernel launches of one application of op's preconditioner (as precond
 // issues them).
 template <typename TV>
@@ -1327,6 +1413,8 @@ void scatter_end(H &h, const double *x, const double *phat, double *d_x, const S
                        h.d_perm.p, x, phat, d_x, st, h.d_host_st);
     check_launch();
     HIP_CHECK(hipStreamSynchronize(h.stream));
+    if (__atomic_exchange_n(h.h_done + kSweepFail, 0, __ATOMIC_ACQ_REL) != 0)
+        throw std::runtime_error("a sweep's wait did not end");
 }
 
 // One BiCGSTAB run following the reference microprogram (solver_pkg.vhd:120-141).
@@ -1377,7 +1465,13 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     // of one half at most (ahead = 1), while the device still has that
     // preconditioner queued whenever the host waits.
     bool stop = false;
-    const bool fuse = fuse_sweep_spmv(h, op);
+    const bool wait = sweeps_wait(h);
+    const bool fuse = !wait && fuse_sweep_spmv(h, op);
+    if (wait) {
+        hipLaunchKernelGGL((k_sweep_reset<TX>), dim3(blocks_for((int64_t)std::max<size_t>(N, 3), 256)), dim3(256), 0,
+                           h.stream, (int64_t)N, k.y.p, h.d_sweep.p);
+        check_launch();
+    }
     const int nparts = op.A->ntiles_wide;  // of the product
     const bool fold = h.fold && nparts <= kFoldMax && vb <= kFoldMax;
     auto fin_of = [&](int fin) { return fold ? (int)FIN_NONE : fin; };
@@ -1396,7 +1490,8 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     // z = M^-1 p, and, fused, the colour-0 rows of v = A z with their dots
     auto apply = [&](auto redc, const TX *p, TX *z, TX *v, const TX *w0) {
         constexpr int RED = decltype(redc)::value;
-        precond<BS, TV, TX>(h, op, p, k.y.p, z, 0, fuse);
+        if (wait) precond_wait<BS, TV, TX>(h, op, p, k.y.p, z, 0);
+        else precond<BS, TV, TX>(h, op, p, k.y.p, z, 0, fuse);
         if (fuse) {
             prof_begin(h, PK_UPPER);
             launch_sweep_spmv<BS, RED, TV, TX>(h, op, p, z, v, w0, red(h, 0, FIN_NONE));
@@ -2280,8 +2375,9 @@ int bda_create(int32_t bs, int32_t n, int32_t nnzb_max, bda_handle *out) {
         h->st.ensure(kStates);  // DBuf zero-fills: the idle slot never has done set
         HIP_CHECK(hipHostMalloc((void **)&h->h_st, sizeof(SolverState), hipHostMallocMapped));
         HIP_CHECK(hipHostGetDevicePointer((void **)&h->d_host_st, h->h_st, 0));
-        HIP_CHECK(hipHostMalloc((void **)&h->h_done, (kBadRow + 1) * sizeof(int32_t), hipHostMallocMapped));
-        h->h_done[0] = h->h_done[1] = 0;
+        HIP_CHECK(hipHostMalloc((void **)&h->h_done, kFlags * sizeof(int32_t), hipHostMallocMapped));
+        std::memset(h->h_done, 0, kFlags * sizeof(int32_t));
+        h->d_sweep.ensure(3);
         HIP_CHECK(hipHostGetDevicePointer((void **)&h->d_done, h->h_done, 0));
         HIP_CHECK(hipHostMalloc((void **)&h->h_prog, 2 * sizeof(uint64_t), hipHostMallocMapped));
         h->h_prog[0] = h->h_prog[1] = 0;
@@ -2303,7 +2399,7 @@ int bda_destroy(bda_handle h) {
     (void)hipSetDevice(h->device);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     for (DevMat *m : {&h->A, &h->L, &h->U, &h->At, &h->Ut, &h->Lt}) m->release();
-    for (DBuf<int32_t> *b : {&h->d_perm, &h->d_blkrow, &h->d_upd, &h->d_bad, &h->d_nonfinite}) b->release();
+    for (DBuf<int32_t> *b : {&h->d_perm, &h->d_blkrow, &h->d_upd, &h->d_bad, &h->d_nonfinite, &h->d_sweep}) b->release();
     for (DBuf<double> *b : {&h->d_orig, &h->A64, &h->L64, &h->U64, &h->LU, &h->Dinv, &h->DinvT, &h->At64, &h->Ut64,
                             &h->Lt64, &h->A0d64, &h->low2_v64, &h->bp, &h->xo, &h->ro, &h->vin, &h->vout, &h->vw, &h->gl, &h->gx, &h->ggrad,
                             &h->partials, &h->vparts})
