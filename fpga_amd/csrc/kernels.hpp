@@ -1553,7 +1553,8 @@ __global__ __launch_bounds__(64 * BS) void k_lower2(StreamArgs<TV, TX> a, Stream
 }
 
 // ---------------------------------------------------------------------------
-// A whole sweep in one launch, for orderings of many small levels.  Workgroups
+// A whole sweep in one launch, for orderings of many small levels (or several
+// small colours; the rule is at the launch).  Workgroups
 // take tiles in level order from a ticket counter; a tile loads what does not
 // depend on other tiles, then waits for the x entries it reads, entry by
 // entry (NotYet): the hop from one level to the next is one store and one
@@ -1568,7 +1569,10 @@ __global__ __launch_bounds__(64 * BS) void k_lower2(StreamArgs<TV, TX> a, Stream
 // by itself; it marks the other z entries as not written, the second sweep
 // the y entries, and each clears the other's ticket counter: y and the
 // counters only have to be prepared once per run (k_sweep_reset).  The
-// arithmetic is k_stream's.
+// arithmetic is k_stream's.  It is bound by the chain: 1.1 us from level to
+// level (store, poll, the tile's LDS exchanges) against 2.8 us for a launch
+// per level; the 48x48x24 level-scheduled FP64 step 33.6 -> 14.6 ms, 128x128x64
+// 150 -> 49 ms.
 template <typename TX>
 struct WaitArgs {
     int32_t *ticket, *other;   // this sweep's ticket counter and the other's

@@ -1222,19 +1222,16 @@ void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si, bool 
     prof_end(h);
 }
 
-// A solve runs its sweeps as two launches whose tiles wait for one another
-// (k_sweep_wait) where the launches per level would be latency-bound.
-constexpr int kWaitFromLevels = 16;
-constexpr int kWaitLevelsAhead = 6;
-bool sweeps_wait(const H &h) { return h.wait && h.an.ncolours >= kWaitFromLevels; }
-
 // Workgroups of a waiting sweep: enough for kWaitLevelsAhead of its widest
 // levels, so that a level's tiles have loaded their operands when their turn
-// comes, and few enough that those waiting do not crowd the memory system.
+// comes, and few enough that those waiting do not crowd the memory system
+// (128x128x64 by level sets, FP64 step by levels ahead: 1: 57.1 ms, 2: 49.0,
+// 4: 50.9, 6: 53.0, 12: 60.3; 48x48x24: 17.9, 14.6, 14.7, 14.7, 14.8).
+constexpr int kWaitLevelsAhead = 2;
 int wait_grid(const DevMat &m, int c0, int c1) {
     int widest = 1;
     for (int c = c0; c < c1; ++c) widest = std::max(widest, m.colour_tile[c + 1] - m.colour_tile[c]);
-    return std::min({m.colour_tile[c1] - m.colour_tile[c0], std::max(64, kWaitLevelsAhead * widest), 2048});
+    return std::min({m.colour_tile[c1] - m.colour_tile[c0], std::max(8, kWaitLevelsAhead * widest), 2048});
 }
 
 template <int BS, typename TV, typename TX>
@@ -1334,6 +1331,25 @@ template <typename TV>
 bool fuse_sweep_spmv(const H &h, const OpSet<TV> &op) {
     return h.fuse0 && h.u0_is_a && op.A == &h.A && op.S2 == &h.U && !op.s1_dinv && op.s2_dinv && h.an.ncolours > 1 &&
            op.A->colour_tile_wide[1] >= kFuseFrom;
+}
+
+// Whether a solve runs its sweeps as two launches whose tiles wait for one
+// another (k_sweep_wait).  A launch of a small colour or level costs 2.8 us, a
+// waiting sweep's about 4.2, and its tiles about 10 ns each more than
+// k_stream's (their gathers go past the L2): it pays from four launches on
+// and up to kWaitTilesPerLaunch tiles for each launch above three.  us per
+// FP64 iteration, launches / waiting: 4 colours of 110 to 3 rows, forward (3
+// launches) 59.8 / 58.8, adjoint (6) 74.3 / 61.4; of 811 to 15 rows (4) 68.6 /
+// 59.9; 5 colours of 12116 to 1 rows, 5 launches 87.3 / 97.1, 8 launches 108 /
+// 106; 2 colours of 8192 51.9 / 70.4; 16 levels of 2000 rows 295 / 156; of
+// 20000 rows 406 / 420.
+constexpr int kWaitTilesPerLaunch = 280;
+template <typename TV>
+bool sweeps_wait(const H &h, const OpSet<TV> &op) {
+    if (!h.wait) return false;
+    const int launches = precond_launches(h, op);
+    const int64_t tiles = (int64_t)op.S1->ntiles + op.S2->ntiles;
+    return launches >= 4 && tiles < (int64_t)kWaitTilesPerLaunch * (launches - 3);
 }
 
 struct RunOut {
@@ -1465,7 +1481,7 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     // of one half at most (ahead = 1), while the device still has that
     // preconditioner queued whenever the host waits.
     bool stop = false;
-    const bool wait = sweeps_wait(h);
+    const bool wait = sweeps_wait(h, op);
     const bool fuse = !wait && fuse_sweep_spmv(h, op);
     if (wait) {
         hipLaunchKernelGGL((k_sweep_reset<TX>), dim3(blocks_for((int64_t)std::max<size_t>(N, 3), 256)), dim3(256), 0,

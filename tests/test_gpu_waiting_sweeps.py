@@ -1,12 +1,13 @@
-"""Sweeps whose tiles wait for one another (a solve's sweeps over 16 levels or
-more) against the launches per level that apply the preconditioner by itself
+"""Sweeps whose tiles wait for one another (a solve's sweeps over many small
+levels, or several small colours) against the launches per level that apply the preconditioner by itself
 (which other tests hold to the oracle bit for bit).  A solve that stops after
 its first half-iteration returns x = alpha phat, each entry rounded once, so
 phat = M^-1 b shows in x up to the one number alpha: some double next to
 x_k / phat_k must give every entry.  FP64, the two precision forms, and the
 adjoint; level sets of grids, a chain (as many levels as rows), rows without
-lower blocks, 15 and 16 levels (either side of the rule).  Then whole solves:
-converged, and the same bits when repeated.
+lower blocks, colourings on either side of the rule (2 to 5 colours, forward
+and transposed launches differing).  Then whole solves: converged, and the same
+bits when repeated.
 """
 import numpy as np
 import pytest
@@ -35,13 +36,23 @@ def bands(bs):
     return random_system(bs, links(int(start[-1]), pairs), 4)
 
 
-CASES = {
-    "grid": grid_case(scaled(GRID_128x128x64, 17, 14, 9)),
-    "grid_wide": grid_case(fa.GridSpec(40, 36, 12, seed=3)),
-    "chain": path(700),
-    "bands": bands,
-    "levels_15": path(15),
-    "levels_16": path(16),
+def clique_rows(bs):
+    """Nine colours, most of one or two rows."""
+    return random_system(bs, links(300, [(i, i + 1) for i in range(299)] +
+                                   [(i, j) for i in range(100, 109) for j in range(100, i)]), 5)
+
+
+CASES = {  # system, level sets
+    "grid": (grid_case(scaled(GRID_128x128x64, 17, 14, 9)), True),
+    "grid_wide": (grid_case(fa.GridSpec(40, 36, 12, seed=3)), True),
+    "chain": (path(700), True),
+    "bands": (bands, True),
+    "levels_3": (path(3), True),
+    "levels_4": (path(4), True),
+    "colours_2": (grid_case(fa.GridSpec(9, 8, 7, seed=3)), False),
+    "colours_4": (grid_case(scaled(GRID_128x128x64, 16, 15, 8)), False),
+    "colours_wide": (grid_case(scaled(GRID_128x128x64, 37, 41, 19)), False),
+    "colours_9": (clique_rows, False),
 }
 
 
@@ -65,12 +76,13 @@ def check_scaled(x, phat, dtype):
 @pytest.mark.parametrize("name", list(CASES))
 def test_waiting_sweeps(name, bs):
     print(f"case {name} bs={bs}", flush=True)
-    rowptr, colidx, vals, b = CASES[name](bs)
+    make, level = CASES[name]
+    rowptr, colidx, vals, b = make(bs)
     n = len(rowptr) - 1
     g = fa.BicgstabSolver(bs, n, len(colidx))
     try:
         g.upload_bcsr(rowptr, colidx, vals)
-        g.analyse(True)
+        g.analyse(level)
         g.factor()
         perm = g.colouring()[1]
         sp = lambda v: v.reshape(n, bs)[perm].ravel()
@@ -95,7 +107,7 @@ def test_waiting_sweeps(name, bs):
 def test_nan_right_hand_side_ends():
     """NaN entries, the mark of an unwritten entry among them, are results like
     any other: the sweeps end and the run stops on the NaN."""
-    rowptr, colidx, vals, b = CASES["bands"](3)
+    rowptr, colidx, vals, b = bands(3)
     n = len(rowptr) - 1
     g = fa.BicgstabSolver(3, n, len(colidx))
     try:
