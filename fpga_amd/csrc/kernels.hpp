@@ -575,7 +575,7 @@ __global__ __launch_bounds__(256) void k_check_finite(int64_t n, const double *s
 // FP64 values one lane per two consecutive entries (one 16-byte load; 63
 // lanes per wave step for 3x3, 64 for 4x4); either way every wave load
 // instruction reads consecutive memory.  The tile's x entries are gathered
-// into LDS (column indices staged there first); a row lane adds its block
+// into LDS; a row lane adds its block
 // row's products left to right, pair lanes add theirs with the next lane's
 // in the same order through cross-lane shifts.  The per-block row partials
 // go to LDS.  Phase 2 gives
@@ -764,7 +764,7 @@ template <int RED> struct NRedOf { static constexpr int value = (RED & 1) + ((RE
 // carry a few blocks of padding for this): the compiler's wait-count
 // insertion falls back to waiting for every outstanding load at a branch,
 // which would serialise the memory round trips.  Column indices and row
-// pointers are issued first, so the first barrier waits for them and not
+// pointers are issued first, so the gathers wait for them and not
 // for the value stream issued after them.  A tile costs three dependent
 // memory round trips: descriptor; columns/values/row operands; x gathers.
 //
@@ -801,7 +801,6 @@ template <typename TX, int BS, int CAP>
 struct TileLds {
     double part[CAP * BS];
     TX sx[CAP * BS];
-    int32_t scol[(CAP + 64 * BS - 1) / (64 * BS) * 64 * BS];
     int32_t srow[64 * BS];
 };
 template <typename TX, int BS, int CAP>
@@ -814,6 +813,21 @@ __device__ inline double *tile_tv() {
     __shared__ double tv[N];
     return tv;
 }
+
+// Sweep launches of fewer than kPlainBelow tiles read FP32 matrix values and
+// column indices with plain loads instead of non-temporal ones (the merged
+// tail launch always does): their few MB then stay in the last-level cache
+// from one preconditioner application to the next, while the big launches'
+// non-temporal streams do not displace them.  On a 128x128x64 grid this
+// takes 0.5 us from the second lower colour, 0.4 us from the tall upper
+// colour 1 and 0.2 us from the tail per application.  FP64 sweeps keep
+// non-temporal loads: with FP64 vectors twice as large, keeping their matrix
+// data cached slowed the FP64 SpMV by 1.6 us.
+#ifndef BDA_PLAIN_BELOW
+#define BDA_PLAIN_BELOW 8192
+#endif
+constexpr int kPlainBelow = BDA_PLAIN_BELOW;
+template <typename TV> constexpr bool plain_small() { return std::is_same<TV, float>::value && kPlainBelow > 0; }
 
 // stream_tile is the work of one workgroup on the tile with descriptor d;
 // with KEEP it also leaves the tile's outputs (rounded to TX, (row - first
@@ -840,7 +854,7 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
     constexpr int VPW = BPW * BB;          // lanes carrying a value (63 or 64)
     constexpr int S = CAP / (NW * BPW);    // value slots per lane
     constexpr int CJ = (CAP + NT - 1) / NT;       // column loads per thread
-    constexpr int XV = (CAP + NT - 1) / NT;       // x gathers (whole blocks) per thread
+    constexpr int XV = CJ;                        // x gathers (whole blocks) per thread
     constexpr int NRED = (RED & 1) + ((RED >> 1) & 1);
     constexpr int RS = ROWS / 64;                 // epilogue rows per thread
     static_assert(ROWS == 64 || ROWS == 128, "tile rows");
@@ -854,7 +868,6 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
     TileLds<TX, BS, CAP> &lds = tile_lds<TX, BS, CAP>();
     double *part = lds.part;
     TX *sx = lds.sx;
-    int32_t *scol = lds.scol;
     int32_t *srow = lds.srow;
     double *tv = tile_tv<(MODE == SM_SUB_DINV || MODE == SM_SUB_Z) ? RS * NT : 1>();
     if constexpr (MODE == SM_SUB_SPMV) {
@@ -877,7 +890,7 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
     // 1. column indices and row pointers
     int ci[CJ];
 #pragma unroll
-    for (int j = 0; j < CJ; ++j) ci[j] = load_mat<PLAIN>(&a.colidx[b0 + min(t + j * NT, nblk)]);
+    for (int j = 0; j < CJ; ++j) ci[j] = load_mat<PLAIN>(&a.colidx[b0 + min(t + j * NT, max(nblk - 1, 0))]);
     const int rp = a.rowptr[r0 + min(t, nrow)];
 
     // 2. values.  Row lanes: slot u of thread t is block row j = u*NT + t of
@@ -962,13 +975,16 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
         }
     }
 
-#pragma unroll
-    for (int j = 0; j < CJ; ++j) scol[t + j * NT] = ci[j];
     srow[t] = rp - b0;
-    __syncthreads();
+    // Launches that fill the chip keep the barrier that staging the columns in
+    // LDS used to need: with it their waves issue their gathers together
+    // (without: precision form on 128x128x64 6.02 -> 6.10 ms).  The sweeps of
+    // smaller systems are shorter without it (64x64x32 FP64 forward and
+    // backward 3.87 -> 3.80 ms).
+    if constexpr (wide_tiles<MODE>() || (plain_small<TV>() && !PLAIN)) __syncthreads();
 
     // 4. x entries of the tile, one block (BS entries, one vector load) per
-    // lane, stored (block, component) like part[]; lanes past the last block
+    // lane, the lane that loaded the block's column index, stored (block, component) like part[]; lanes past the last block
     // repeat it (the same values to the same place).  A lane per entry needed
     // BS times the address work: the FP32 3x3 SpMV took 59.7 us instead of
     // 56.0 us with it (measured).
@@ -982,7 +998,7 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
 #pragma unroll
         for (int j = 0; j < XV; ++j) {
             xq[j] = min(t + j * NT, nblk > 0 ? nblk - 1 : 0);
-            const int cb = nblk > 0 ? scol[xq[j]] : 0;
+            const int cb = nblk > 0 ? ci[j] : 0;
             src[j] = (cb < a.split ? a.x_lo : a.x) + (size_t)cb * BS;
             ready[j] = false;
             free[j] = nblk == 0 || cb < a.split;
@@ -1023,7 +1039,7 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
         const int q = min(t + j * NT, nblk > 0 ? nblk - 1 : 0);
-        int cb = nblk > 0 ? scol[q] : 0;
+        int cb = nblk > 0 ? ci[j] : 0;
         xl[j] = -1;
         if constexpr (V == 2) {
             xl[j] = cb < 0 ? -1 - cb : -1;
@@ -1304,21 +1320,6 @@ struct TailArgs {
     const int32_t *dep;      // its rows that carry blocks (ndep <= 64)
     int32_t ndep;
 };
-
-// Sweep launches of fewer than kPlainBelow tiles read FP32 matrix values and
-// column indices with plain loads instead of non-temporal ones (the merged
-// tail launch always does): their few MB then stay in the last-level cache
-// from one preconditioner application to the next, while the big launches'
-// non-temporal streams do not displace them.  On a 128x128x64 grid this
-// takes 0.5 us from the second lower colour, 0.4 us from the tall upper
-// colour 1 and 0.2 us from the tail per application.  FP64 sweeps keep
-// non-temporal loads: with FP64 vectors twice as large, keeping their matrix
-// data cached slowed the FP64 SpMV by 1.6 us.
-#ifndef BDA_PLAIN_BELOW
-#define BDA_PLAIN_BELOW 8192
-#endif
-constexpr int kPlainBelow = BDA_PLAIN_BELOW;
-template <typename TV> constexpr bool plain_small() { return std::is_same<TV, float>::value && kPlainBelow > 0; }
 
 template <int BS, int MODEA, int MODEB, typename TV, typename TX>
 __global__ __launch_bounds__(64 * BS) void k_tail(StreamArgs<TV, TX> a, TailArgs<TV, TX> b) {
@@ -2022,8 +2023,11 @@ __global__ void k_gather_start(int n, int bs, const int32_t *perm, const double 
     const double vb = b[j], vx = x[j];
     bp[i] = vb;
     xp[i] = vx;
-    if (!(vx == 0.0) || (i == 0 && *nonfinite != 0))
-        __hip_atomic_store(&st->full_residual, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // one ordinary store per wave (they meet in the L2): agent-scope stores to
+    // one address are served one after the other, 417 us for 182k 4x4 rows
+    // with one from every lane that found an entry, 126 us with one per wave
+    const uint64_t found = __ballot(!(vx == 0.0) || (i == 0 && *nonfinite != 0));
+    if (found != 0 && (threadIdx.x & 63) == __builtin_ctzll(found)) st->full_residual = 1;
 }
 __global__ void k_scatter_rows(int n, int bs, const int32_t *perm, const double *in, double *out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
