@@ -61,7 +61,6 @@ struct SolverState {
     int32_t max_outer;
     int32_t adaptive;
     int32_t inner_h;        // sum of the inner runs' half iterations
-    int32_t full_residual;  // set by k_gather_start: the step-0 residual needs the product
     // watchdog (the counterpart of the reference kernel's abort cycle count,
     // param0): timeout in ticks of the device's constant-rate wall clock
     // (0 = off); the run's deadline is set on the device when its state is
@@ -290,14 +289,11 @@ __device__ inline void refine_step(SolverState *out, const SolverState *in) {
         signal_done(out);
 }
 
-// The factorisation's flags: cleared before it, and the bad row (INT32_MAX:
-// none) to mapped host memory after it.
-__global__ void k_factor_begin(int32_t *bad, int32_t *nonfinite) {
+// After a factorisation: its bad row (INT32_MAX: none) to mapped host memory,
+// and the flag cleared for the next (host_bad null: only that).
+__global__ void k_factor_end(int32_t *bad, int32_t *host_bad) {
+    if (host_bad) __hip_atomic_store(host_bad, *bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     *bad = INT32_MAX;
-    *nonfinite = 0;
-}
-__global__ void k_factor_end(const int32_t *bad, int32_t *host_bad) {
-    __hip_atomic_store(host_bad, *bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Sum over the 64 lanes of a wave as the butterfly v += v[lane ^ o] for
@@ -556,13 +552,14 @@ __global__ __launch_bounds__(kFinGroupThreads) void k_finalize_stage1(RedArgs ra
     }
 }
 
-// *nonfinite = 1 when one of n values is infinite or NaN.  Every writer stores
-// the same value.
-__global__ __launch_bounds__(256) void k_check_finite(int64_t n, const double *src, int32_t *nonfinite) {
+// *nonfinite = id when one of n values is infinite or NaN (id: the
+// factorisation's own, so that the flag never has to be cleared).  Every
+// writer stores the same value.
+__global__ __launch_bounds__(256) void k_check_finite(int64_t n, const double *src, int32_t *nonfinite, int32_t id) {
     bool bad = false;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         bad = bad || !finite(src[i]);
-    if (bad) __hip_atomic_store(nonfinite, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (bad) __hip_atomic_store(nonfinite, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---------------------------------------------------------------------------
@@ -632,6 +629,7 @@ struct StreamArgs {
     const int32_t *rowptr2 = nullptr;  // SUB_Z: the second sweep's row pointers
     TX *zout = nullptr;                // SUB_Z: z of the rows without second-sweep blocks
     const int32_t *rowmap = nullptr;   // dependency tiles (k_lower2): matrix row of each packed row
+    const int32_t *full = nullptr;     // step-0 residual: the id of a run that needs the product
     TX *reset = nullptr;               // waiting tiles: entries to mark as not written (see k_sweep_wait)
     int32_t *fail = nullptr;           // waiting tiles: a wait has run out; on the device, and for the host
     int32_t *host_fail = nullptr;
@@ -1289,7 +1287,7 @@ __global__ __launch_bounds__(64 * BS) void k_stream(StreamArgs<TV, TX> a) {
     const int slot = NRedOf<RED>::value > 0 ? a.slot[tile] : 0;
     static_assert(!ZX || ROWS == 64, "the zero-start path serves one row per thread");
     if constexpr (ZX) {
-        if (a.ra.st->full_residual == 0) {
+        if (*a.full != a.ra.st->run_id) {
             stream_rows_zero_x<BS, MODE, RED, TV, TX>(a, d, slot);
             return;
         }
@@ -2009,14 +2007,19 @@ __global__ void k_gather_rows(int n, int bs, const int32_t *perm, const double *
     const int64_t k = i / bs, c = i - k * bs;
     out[i] = in[(int64_t)perm[k] * bs + c];
 }
-// Start of a solve: the right-hand side and the start vector in one launch,
-// with the check before the step-0 residual: sets st->full_residual when an
-// entry of the start vector is not zero (a NaN counts as nonzero) or the
-// matrix holds a non-finite value (*nonfinite, recorded when it was
-// factorised).  Every writer stores the same value.
+// Start of a solve: its state (the watchdog's deadline counts from here), the
+// right-hand side and the start vector in one launch, with the check before
+// the step-0 residual: *full = the run's id when an entry of the start vector
+// is not zero (a NaN counts as nonzero) or the matrix holds a non-finite value
+// (*nonfinite, recorded when it was factorised as id).
 __global__ void k_gather_start(int n, int bs, const int32_t *perm, const double *b, double *bp, const double *x,
-                               double *xp, const int32_t *nonfinite, SolverState *st) {
+                               double *xp, const int32_t *nonfinite, int32_t id, int32_t *full, SolverState *st,
+                               SolverState start) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) {
+        if (start.timeout_ticks != 0) start.deadline = wall_clock64() + start.timeout_ticks;
+        *st = start;
+    }
     if (i >= (int64_t)n * bs) return;
     const int64_t k = i / bs, c = i - k * bs;
     const int64_t j = (int64_t)perm[k] * bs + c;
@@ -2026,8 +2029,8 @@ __global__ void k_gather_start(int n, int bs, const int32_t *perm, const double 
     // one ordinary store per wave (they meet in the L2): agent-scope stores to
     // one address are served one after the other, 417 us for 182k 4x4 rows
     // with one from every lane that found an entry, 126 us with one per wave
-    const uint64_t found = __ballot(!(vx == 0.0) || (i == 0 && *nonfinite != 0));
-    if (found != 0 && (threadIdx.x & 63) == __builtin_ctzll(found)) st->full_residual = 1;
+    const uint64_t found = __ballot(!(vx == 0.0) || (i == 0 && *nonfinite == id));
+    if (found != 0 && (threadIdx.x & 63) == __builtin_ctzll(found)) *full = start.run_id;
 }
 __global__ void k_scatter_rows(int n, int bs, const int32_t *perm, const double *in, double *out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2212,6 +2215,7 @@ struct IluArgs {
     double *l, *u, *dinv, *adiag;
     float *a32, *l32, *u32, *adiag32;
     int32_t *bad_row, *nonfinite;
+    int32_t id;                              // of the factorisation (nonfinite)
 };
 
 template <int BS>
@@ -2250,7 +2254,7 @@ __global__ __launch_bounds__(64 * BS) void k_ilu0_tile(IluArgs<BS> a) {
             if (a.a32) a.a32[(size_t)b0 * BB + e] = (float)v[u];
         }
     }
-    if (bad) __hip_atomic_store(a.nonfinite, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (bad) __hip_atomic_store(a.nonfinite, a.id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
 
     // where each block goes: L block index, -2 - U block index, -1 the diagonal

@@ -605,7 +605,9 @@ struct bda_handle_s {
     bda::DevMat A, L, U, At, Ut, Lt;
     bda::DBuf<int32_t> d_perm, d_blkrow, d_bad;
     bda::DBuf<int32_t> d_upd;  // what each L block updates in the factorisation (k_ilu0_updates)
-    bda::DBuf<int32_t> d_nonfinite;  // set by the factorisation when a matrix value is infinite or NaN
+    bda::DBuf<int32_t> d_nonfinite;  // the last factorisation (factor_id) that met an infinite or NaN value
+    bda::DBuf<int32_t> d_full;       // the last run (its id) whose step-0 residual needs the product
+    int32_t factor_id = 0;
     bda::DBuf<double> d_orig, A64, L64, U64, LU, Dinv, DinvT, At64, Ut64, Lt64;
     bda::DBuf<float> A32, L32, U32;
     bda::DBuf<double> A0d64;  // A's diagonal blocks of colour 0, packed (SM_SUB_SPMV)
@@ -832,8 +834,8 @@ int stream_dispatch(H &h, const StreamArgs<TV, TX> &a) {
 // --- streaming kernel launch over the tiles of one colour (or all) ---------
 // prof_kind >= 0: with profiling on, the streaming kernel alone (not its
 // finalize) is bracketed by an event pair of that kind.
-// ZX: a step-0 residual that takes the short path when k_gather_start left
-// the state's full_residual clear (zero start vector, finite matrix).
+// ZX: a step-0 residual that takes the short path unless k_gather_start left
+// the run's id in h.d_full (zero start vector, finite matrix).
 // colour kRestOfRows (the product only): every colour but the first, whose
 // rows' partial sums launch_sweep_spmv has left in their slots.
 constexpr int kRestOfRows = -2;
@@ -893,6 +895,7 @@ void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x
     a.ra = ra;
     a.rowptr2 = rowptr2;
     a.zout = zout;
+    a.full = h.d_full.p;
     if (!use_state) a.ra.st = h.st.p + kIdleState;
     if (MODE == SM_SUB_Z && (!rowptr2 || !zout || !dinv)) throw std::runtime_error("SUB_Z launch without z operands");
     if ((RED & SR_W0) && !w0) throw std::runtime_error("missing dot operand");
@@ -1418,9 +1421,11 @@ int32_t init_state(H &h, int idx, double tol, int maxit, bool abs_mode) {
 }
 
 // The start and the end of a solve on the caller's vectors.
-void gather_start(H &h, const double *d_b, double *bp, const double *d_x, double *xp, SolverState *st) {
+void gather_start(H &h, const double *d_b, double *bp, const double *d_x, double *xp, SolverState *st,
+                  const SolverState &start) {
     hipLaunchKernelGGL(k_gather_start, dim3(blocks_for((int64_t)h.N(), 256)), dim3(256), 0, h.stream, h.n, h.bs,
-                       h.d_perm.p, d_b, bp, d_x, xp, (const int32_t *)h.d_nonfinite.p, st);
+                       h.d_perm.p, d_b, bp, d_x, xp, (const int32_t *)h.d_nonfinite.p, h.factor_id, h.d_full.p, st,
+                       start);
     check_launch();
 }
 // x and the state (to h.h_st), complete on return
@@ -1459,8 +1464,9 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     } else {
         if constexpr (std::is_same<TX, double>::value) {
             // r = b - A x0; with x0 = 0 (and a finite matrix) this is b, without the product
-            run_id = init_state(h, 0, tol, maxit, abs_mode);
-            gather_start(h, d_b, h.bp.p, d_x, k.x.p, h.st.p);
+            const SolverState s = new_state(h, 0, tol, maxit, abs_mode);
+            run_id = s.run_id;
+            gather_start(h, d_b, h.bp.p, d_x, k.x.p, h.st.p, s);
             launch_stream<BS, SM_SUB, SR_SELF, TV, TX, true>(h, *op.A, op.Aval, -1, k.x.p, rhs, k.rt.p, nullptr,
                                                              nullptr, red(h, 0, FIN_INIT), true, k.r.p, k.p.p,
                                                              nullptr, 0, PK_SPMV);
@@ -1711,6 +1717,9 @@ void finish_analyse(H &h) {
     h.Dinv.ensure((size_t)h.n * bb);
     h.d_bad.ensure(1);
     h.d_nonfinite.ensure(1);
+    h.d_full.ensure(1);
+    hipLaunchKernelGGL(k_factor_end, dim3(1), dim3(1), 0, h.stream, h.d_bad.p, (int32_t *)nullptr);
+    check_launch();
     // reduction partials: one slot pair per workgroup of the largest reducing
     // launch, and room for the first stage of a two-stage sum
     const int cap = std::max({h.A.ntiles, h.At.ntiles, vec_blocks(h.N()), 1}) + kFinGroups;
@@ -1738,6 +1747,8 @@ void do_analyse(H &h, bool level) {
     analyse(h.pattern, level, h.an);
     finish_analyse(h);
 }
+
+int32_t next_factor_id(H &h) { return h.factor_id = h.factor_id == INT32_MAX ? 1 : h.factor_id + 1; }
 
 // The precision form's FP32 copies: their buffers, and those of L's packed
 // dependency rows (k_lower2) from the FP64 ones.
@@ -1771,8 +1782,6 @@ void do_factor(H &h) {
     constexpr int BB = BS * BS;
     const Analysis &an = h.an;
     const auto t0 = std::chrono::steady_clock::now();
-    hipLaunchKernelGGL(k_factor_begin, dim3(1), dim3(1), 0, h.stream, h.d_bad.p, h.d_nonfinite.p);
-    check_launch();
     const bool f32 = h.mixed_used;
     if (f32) mixed_buffers<BS>(h);
     if (an.ncolours > 1) h.A0d64.ensure((size_t)an.colour_ptr[1] * BB);
@@ -1793,6 +1802,7 @@ void do_factor(H &h) {
     a.u32 = f32 ? h.U32.p : nullptr;
     a.bad_row = h.d_bad.p;
     a.nonfinite = h.d_nonfinite.p;
+    a.id = next_factor_id(h);
     for (int c = 0; c < an.ncolours; ++c) {
         a.tile0 = h.A.colour_tile_wide[c];
         a.ntiles = h.A.colour_tile_wide[c + 1] - a.tile0;
@@ -1803,7 +1813,7 @@ void do_factor(H &h) {
     }
     gather_low2<BS>(h);
     if (f32) gather_low2_32<BS>(h);
-    hipLaunchKernelGGL(k_factor_end, dim3(1), dim3(1), 0, h.stream, (const int32_t *)h.d_bad.p, h.d_done + kBadRow);
+    hipLaunchKernelGGL(k_factor_end, dim3(1), dim3(1), 0, h.stream, h.d_bad.p, h.d_done + kBadRow);
     check_launch();
     HIP_CHECK(hipStreamSynchronize(h.stream));
     const int32_t bad = __atomic_load_n(h.h_done + kBadRow, __ATOMIC_ACQUIRE);
@@ -1826,12 +1836,10 @@ void do_factor(H &h) {
 template <int BS>
 void load_factors(H &h, const double *lu_values, const double *dinv) {
     constexpr int BB = BS * BS;
-    const int32_t zero = 0;
-    HIP_CHECK(hipMemcpyAsync(h.d_nonfinite.p, &zero, 4, hipMemcpyHostToDevice, h.stream));
     const int64_t nval = (int64_t)h.A.nnzb * BB;
     const int grid = (int)std::min<int64_t>(std::max<int64_t>(blocks_for(nval, 256), 1), 8192);
     hipLaunchKernelGGL(k_check_finite, dim3(grid), dim3(256), 0, h.stream, nval, (const double *)h.A64.p,
-                       h.d_nonfinite.p);
+                       h.d_nonfinite.p, next_factor_id(h));
     check_launch();
     h.LU.ensure((size_t)nval);
     HIP_CHECK(hipMemcpyAsync(h.LU.p, lu_values, (size_t)nval * 8, hipMemcpyHostToDevice, h.stream));
@@ -2017,9 +2025,7 @@ void solve_mixed_dev(H &h, const double *d_b, double *d_x, double tol, int max_o
     os.inner_tol = inner_tol;
     os.eta = h.refine_eta;
     os.adaptive = h.refine_adaptive;
-    hipLaunchKernelGGL(k_set_state, dim3(1), dim3(1), 0, h.stream, h.st.p + 1, os);
-    check_launch();
-    gather_start(h, d_b, h.bp.p, d_x, h.xo.p, h.st.p + 1);
+    gather_start(h, d_b, h.bp.p, d_x, h.xo.p, h.st.p + 1, os);
     bool aborted = false;
     for (int outer = 0;; ++outer) {
         // FP64 true residual ro = b - A x and the outer step's decisions; the
@@ -2415,7 +2421,7 @@ int bda_destroy(bda_handle h) {
     (void)hipSetDevice(h->device);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     for (DevMat *m : {&h->A, &h->L, &h->U, &h->At, &h->Ut, &h->Lt}) m->release();
-    for (DBuf<int32_t> *b : {&h->d_perm, &h->d_blkrow, &h->d_upd, &h->d_bad, &h->d_nonfinite, &h->d_sweep}) b->release();
+    for (DBuf<int32_t> *b : {&h->d_perm, &h->d_blkrow, &h->d_upd, &h->d_bad, &h->d_nonfinite, &h->d_full, &h->d_sweep}) b->release();
     for (DBuf<double> *b : {&h->d_orig, &h->A64, &h->L64, &h->U64, &h->LU, &h->Dinv, &h->DinvT, &h->At64, &h->Ut64,
                             &h->Lt64, &h->A0d64, &h->low2_v64, &h->bp, &h->xo, &h->ro, &h->vin, &h->vout, &h->vw, &h->gl, &h->gx, &h->ggrad,
                             &h->partials, &h->vparts})
