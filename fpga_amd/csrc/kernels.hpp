@@ -1690,8 +1690,8 @@ static_assert(sizeof(SolverState) % 8 == 0 && kStateWords <= kVecThreads, "a sta
 
 template <int NRED, int U>
 __device__ inline void fold_waves(const double *part, int cap, int n, double (*sred)[2]) {
-    constexpr int VW = kFinThreads / kVecThreads;   // waves of k_finalize one wave stands for
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NW = kVecThreads / 64, VW = kFinThreads / kVecThreads;  // this wave stands for VW of k_finalize's,
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;           // NW apart, so that few partials spread
     double v[VW][NRED][U];
 #pragma unroll
     for (int w = 0; w < VW; ++w)
@@ -1699,22 +1699,25 @@ __device__ inline void fold_waves(const double *part, int cap, int n, double (*s
         for (int j = 0; j < NRED; ++j)
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int i = u * kFinThreads + (wave * VW + w) * 64 + lane;
+                const int i = u * kFinThreads + (w * NW + wave) * 64 + lane;
                 v[w][j][u] = part[(size_t)j * cap + min(i, n - 1)];
             }
 #pragma unroll
-    for (int w = 0; w < VW; ++w)
+    for (int w = 0; w < VW; ++w) {
+        const int vw = w * NW + wave;
+        if (vw * 64 >= n) {  // no partials: the sum is +0.0
+            if (lane < NRED) sred[vw][lane] = 0.0;
+            continue;
+        }
 #pragma unroll
         for (int j = 0; j < NRED; ++j) {
             double t = 0.0;
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = u * kFinThreads + (wave * VW + w) * 64 + lane;
-                t += 0.0 + (i < n ? v[w][j][u] : 0.0);
-            }
+            for (int u = 0; u < U; ++u) t += 0.0 + (u * kFinThreads + vw * 64 + lane < n ? v[w][j][u] : 0.0);
             t = wave_sum(t);
-            if (lane == 0) sred[wave * VW + w][j] = t;
+            if (lane == 0) sred[vw][j] = t;
         }
+    }
 }
 // the wave sums of NRED reductions over n <= kFoldMax partials, for fold_total
 // after a barrier
