@@ -1675,7 +1675,9 @@ __device__ inline VecIdx vec_index(int64_t N) {
 // it.  A forward and backward solve of 64x64x32 to 1e-10 (20 iterations each)
 // 4.26 -> 3.96 ms, a 32x32x16 precision-form step 648 -> 608 us.  Every
 // workgroup repeats the sums, so their cost grows with the square of the
-// system: at 4,096 partials 288 workgroups read 19 MB from the L2.
+// system: us per FP64 / precision-form iteration, separate and folded, at
+// 3,502 partials 138 / 110 both ways, 4,597 (4x4) 174 / 130 -> 168 / 125,
+// 6,537 212 / 149 -> 206 / 145, 10,236 261 / 179 -> 269 / 189.
 struct FoldArgs {
     const double *part;      // the product's partials: reduction j at part + j * cap
     int32_t cap, n;
@@ -1684,7 +1686,8 @@ struct FoldArgs {
     const SolverState *in;
     SolverState *out;
 };
-constexpr int kFoldMax = 4 * kFinThreads;
+constexpr int kFoldStep = 4, kFoldMax = 8 * kFinThreads;
+static_assert(kFoldMax <= kFinThreads * kFinUnroll, "one pass of k_finalize: the same order of the sums");
 constexpr int kStateWords = sizeof(SolverState) / 8;
 static_assert(sizeof(SolverState) % 8 == 0 && kStateWords <= kVecThreads, "a state word per thread");
 
@@ -1692,16 +1695,30 @@ template <int NRED, int U>
 __device__ inline void fold_waves(const double *part, int cap, int n, double (*sred)[2]) {
     constexpr int NW = kVecThreads / 64, VW = kFinThreads / kVecThreads;  // this wave stands for VW of k_finalize's,
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;           // NW apart, so that few partials spread
-    double v[VW][NRED][U];
+    double t[VW][NRED];
 #pragma unroll
     for (int w = 0; w < VW; ++w)
 #pragma unroll
-        for (int j = 0; j < NRED; ++j)
+        for (int j = 0; j < NRED; ++j) t[w][j] = 0.0;
+    for (int u0 = 0; u0 == 0 || (U > 1 && u0 * kFinThreads < n); u0 += U) {
+        double v[VW][NRED][U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = u * kFinThreads + (w * NW + wave) * 64 + lane;
-                v[w][j][u] = part[(size_t)j * cap + min(i, n - 1)];
-            }
+        for (int w = 0; w < VW; ++w)
+#pragma unroll
+            for (int j = 0; j < NRED; ++j)
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int i = (u0 + u) * kFinThreads + (w * NW + wave) * 64 + lane;
+                    v[w][j][u] = part[(size_t)j * cap + min(i, n - 1)];
+                }
+#pragma unroll
+        for (int w = 0; w < VW; ++w)
+#pragma unroll
+            for (int j = 0; j < NRED; ++j)
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    t[w][j] += 0.0 + ((u0 + u) * kFinThreads + (w * NW + wave) * 64 + lane < n ? v[w][j][u] : 0.0);
+    }
 #pragma unroll
     for (int w = 0; w < VW; ++w) {
         const int vw = w * NW + wave;
@@ -1711,11 +1728,8 @@ __device__ inline void fold_waves(const double *part, int cap, int n, double (*s
         }
 #pragma unroll
         for (int j = 0; j < NRED; ++j) {
-            double t = 0.0;
-#pragma unroll
-            for (int u = 0; u < U; ++u) t += 0.0 + (u * kFinThreads + vw * 64 + lane < n ? v[w][j][u] : 0.0);
-            t = wave_sum(t);
-            if (lane == 0) sred[vw][j] = t;
+            const double s = wave_sum(t[w][j]);
+            if (lane == 0) sred[vw][j] = s;
         }
     }
 }
@@ -1724,7 +1738,7 @@ __device__ inline void fold_waves(const double *part, int cap, int n, double (*s
 template <int NRED>
 __device__ inline void fold_sums(const double *part, int cap, int n, double (*sred)[2]) {
     if (n <= kFinThreads) fold_waves<NRED, 1>(part, cap, n, sred);
-    else fold_waves<NRED, kFoldMax / kFinThreads>(part, cap, n, sred);
+    else fold_waves<NRED, kFoldStep>(part, cap, n, sred);
 }
 __device__ inline double fold_total(const double (*sred)[2], int j) {
     double t = sred[0][j];

@@ -1,7 +1,7 @@
 """Scalar steps folded into the vector updates (few reduction partials) against
 the CPU oracle and against themselves at the limits of the rule: one to a few
 hundred product tiles (one load per thread in the folded sums), above 1,024
-(four), and above 4,096 (launches of their own).  What has to hold on every
+(four), above 4,096 (four more), and above 8,192 (launches of their own).  What has to hold on every
 side: the iteration counts, flags and norms of the oracle's solve, the same
 bits when a solve is repeated, and the stops around the folded
 steps: an iteration cap (which stops after a first half), a convergence in the
@@ -16,7 +16,8 @@ import oracle
 pytestmark = pytest.mark.gpu
 
 # product tiles (3x3: 48 rows of 7 blocks each, 4x4: 36): below, at and above the lines
-SIZES = {"one_tile": (5, 3, 2), "few": (16, 15, 12), "over_1024": (48, 41, 31), "over_4096": (70, 64, 56)}
+SIZES = {"one_tile": (5, 3, 2), "few": (16, 15, 12), "over_1024": (48, 41, 31), "over_4096": (70, 64, 56),
+         "over_8192": (101, 80, 52)}
 
 
 @pytest.mark.parametrize("bs", [3, 4])
