@@ -552,6 +552,133 @@ __global__ __launch_bounds__(kFinGroupThreads) void k_finalize_stage1(RedArgs ra
     }
 }
 
+constexpr int kVecThreads = 256;
+
+// A vector update that forms the reduction results it needs itself ("folded"),
+// in place of a k_finalize launch before it.  Every workgroup adds up the
+// partials (in k_finalize's order, so to the same bits) and runs the scalar
+// step on its own copy of the state; workgroup 0 alone writes the new state,
+// to another slot than the one all of them read, and tells the host.  Up to
+// kFoldMax partials: a launch of its own takes about 3 us whatever it does;
+// folded, the sums run beside the update's own loads and add 1.0-1.5 us to
+// it.  A forward and backward solve of 64x64x32 to 1e-10 (20 iterations each)
+// 4.26 -> 3.96 ms, a 32x32x16 precision-form step 648 -> 608 us.  Every
+// workgroup repeats the sums, so their cost grows with the square of the
+// system: us per FP64 / precision-form iteration, separate and folded, at
+// 3,502 partials 138 / 110 both ways, 4,597 (4x4) 174 / 130 -> 168 / 125,
+// 6,537 212 / 149 -> 206 / 145, 10,236 261 / 179 -> 269 / 189.
+struct FoldArgs {
+    const double *part;      // the product's partials: reduction j at part + j * cap
+    int32_t cap, n;
+    const double *vpart;     // those of the vector update before it
+    int32_t vcap, vn;
+    const SolverState *in;
+    SolverState *out;
+};
+constexpr int kFoldStep = 4, kFoldMax = 8 * kFinThreads;
+static_assert(kFoldMax <= kFinThreads * kFinUnroll, "one pass of k_finalize: the same order of the sums");
+constexpr int kStateWords = sizeof(SolverState) / 8;
+static_assert(sizeof(SolverState) % 8 == 0 && kStateWords <= 192, "a state word per thread");
+
+template <int NRED, int U, int NT>
+__device__ inline void fold_waves(const double *part, int cap, int n, double (*sred)[2]) {
+    constexpr int NW = NT / 64, FW = kFinThreads / 64, VW = (FW + NW - 1) / NW;  // this wave stands for VW of
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;  // k_finalize's, NW apart, so that few partials spread
+    double t[VW][NRED];
+#pragma unroll
+    for (int w = 0; w < VW; ++w)
+#pragma unroll
+        for (int j = 0; j < NRED; ++j) t[w][j] = 0.0;
+    for (int u0 = 0; u0 == 0 || (U > 1 && u0 * kFinThreads < n); u0 += U) {
+        double v[VW][NRED][U];
+#pragma unroll
+        for (int w = 0; w < VW; ++w)
+#pragma unroll
+            for (int j = 0; j < NRED; ++j)
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int i = (u0 + u) * kFinThreads + (w * NW + wave) * 64 + lane;
+                    v[w][j][u] = part[(size_t)j * cap + min(i, n - 1)];
+                }
+#pragma unroll
+        for (int w = 0; w < VW; ++w)
+#pragma unroll
+            for (int j = 0; j < NRED; ++j)
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    t[w][j] += 0.0 + ((u0 + u) * kFinThreads + (w * NW + wave) * 64 + lane < n ? v[w][j][u] : 0.0);
+    }
+#pragma unroll
+    for (int w = 0; w < VW; ++w) {
+        const int vw = w * NW + wave;
+        if (vw >= FW) continue;
+        if (vw * 64 >= n) {  // no partials: the sum is +0.0
+            if (lane < NRED) sred[vw][lane] = 0.0;
+            continue;
+        }
+#pragma unroll
+        for (int j = 0; j < NRED; ++j) {
+            const double s = wave_sum(t[w][j]);
+            if (lane == 0) sred[vw][j] = s;
+        }
+    }
+}
+// the wave sums of NRED reductions over n <= kFoldMax partials, for fold_total
+// after a barrier
+template <int NRED, int NT = kVecThreads>
+__device__ inline void fold_sums(const double *part, int cap, int n, double (*sred)[2]) {
+    if (n <= kFinThreads) fold_waves<NRED, 1, NT>(part, cap, n, sred);
+    else fold_waves<NRED, kFoldStep, NT>(part, cap, n, sred);
+}
+__device__ inline double fold_total(const double (*sred)[2], int j) {
+    double t = sred[0][j];
+    for (int w = 1; w < kFinThreads / 64; ++w) t += sred[w][j];
+    return t;
+}
+// Whether a folded run is past its deadline (thread 0 of workgroup 0, whose
+// clock decides for all): it then stops with the launch after this one, whose
+// update is still complete.
+__device__ inline int fold_late(const SolverState *ss) {
+    return blockIdx.x == 0 && !ss->done && past_deadline(ss) ? 1 : 0;
+}
+// End of a folded scalar step (all threads, after the barrier that follows
+// it): the new state.
+__device__ inline void fold_store(const FoldArgs &f, const SolverState *ss, int late) {
+    if (blockIdx.x != 0) return;
+    const int t = threadIdx.x;
+    if (t < kStateWords) {
+        uint64_t w = reinterpret_cast<const uint64_t *>(ss)[t];
+        constexpr size_t od = offsetof(SolverState, done), oa = offsetof(SolverState, aborted);
+        if (late && t == (int)(od / 8)) w |= (uint64_t)1 << (od % 8 * 8);
+        if (late && t == (int)(oa / 8)) w |= (uint64_t)1 << (oa % 8 * 8);
+        reinterpret_cast<uint64_t *>(f.out)[t] = w;
+    }
+    if (t == 0 && late && ss->host_done)
+        __hip_atomic_store(ss->host_done, ss->run_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The ||s|| test (steps 7/8) of a folded run, one workgroup of NT threads.
+// Folded into the second half's k_update_xr the run learns of a convergence in
+// its first half only after the second half's product: 2% faster over 20
+// iterations, 2-8% slower over 2 to 5.  It is a launch of its own, or, where
+// the second half's first launch is a k_stream, an extra workgroup of that
+// (k_stream_half1): nothing in that sweep needs its result.  FEW: at most
+// kFinThreads partials.
+template <int NT, bool FEW>
+__device__ inline void half1_step(const FoldArgs &f) {
+    __shared__ SolverState ss;
+    __shared__ double sred[kFinThreads / 64][2];
+    if (threadIdx.x < kStateWords)
+        reinterpret_cast<uint64_t *>(&ss)[threadIdx.x] = reinterpret_cast<const uint64_t *>(f.in)[threadIdx.x];
+    if constexpr (FEW) fold_waves<1, 1, NT>(f.vpart, f.vcap, f.vn, sred);
+    else fold_sums<1, NT>(f.vpart, f.vcap, f.vn, sred);
+    __syncthreads();
+    if (threadIdx.x == 0 && !ss.done) scalar_step(&ss, FIN_HALF1, fold_total(sred, 0), 0.0, true);
+    __syncthreads();
+    fold_store(f, &ss, 0);
+}
+__global__ __launch_bounds__(kVecThreads) void k_fold_half1(FoldArgs f) { half1_step<kVecThreads, false>(f); }
+
 // *nonfinite = id when one of n values is infinite or NaN (id: the
 // factorisation's own, so that the flag never has to be cleared).  Every
 // writer stores the same value.
@@ -1295,6 +1422,21 @@ __global__ __launch_bounds__(64 * BS) void k_stream(StreamArgs<TV, TX> a) {
     stream_tile<BS, MODE, RED, TV, TX, ROWS, false, PLAIN>(a, d, nullptr, slot);
 }
 
+// A sweep launch with the ||s|| test of a folded run's first half in its first
+// workgroup, beside the tiles: a launch (2.8 us) less per iteration.  The
+// tiles may see the stop flag of before or after the test; if the run stops,
+// nothing reads what they write.
+template <int BS, int MODE, typename TV, typename TX, int ROWS, bool PLAIN>
+__global__ __launch_bounds__(64 * BS) void k_stream_half1(StreamArgs<TV, TX> a, FoldArgs f) {
+    if (blockIdx.x == 0) {
+        half1_step<64 * BS, true>(f);
+        return;
+    }
+    const int4 d = a.tile[a.tile0 + xcd_tile(blockIdx.x - 1, a.ntiles)];
+    if ((a.ra.st->done | ((d.x | d.y | d.z | d.w) < 0 ? 1 : 0)) != 0) return;
+    stream_tile<BS, MODE, SR_NONE, TV, TX, ROWS, false, PLAIN>(a, d, nullptr, 0);
+}
+
 // ---------------------------------------------------------------------------
 // The two sweep launches around the last colour C-1, merged.  When the
 // first sweep's last colour is one tile and at most 64 rows of colour C-2
@@ -1622,7 +1764,6 @@ __global__ __launch_bounds__(256) void k_sweep_reset(int64_t N, TX *y, int32_t *
 // the rest, never read by the matrix kernels and left out of every
 // reduction.  Loads and stores are therefore unconditional, and all loads of
 // a thread are in flight together.
-constexpr int kVecThreads = 256;
 constexpr int kVecPairsPerThread = 4;
 constexpr int kVecElemsPerBlock = kVecThreads * kVecPairsPerThread * 2;
 constexpr int kVecPad = 4;
@@ -1663,108 +1804,6 @@ __device__ inline VecIdx vec_index(int64_t N) {
         v.second[j] = 2 * p + 1 < N;
     }
     return v;
-}
-
-// A vector update that forms the reduction results it needs itself ("folded"),
-// in place of a k_finalize launch before it.  Every workgroup adds up the
-// partials (in k_finalize's order, so to the same bits) and runs the scalar
-// step on its own copy of the state; workgroup 0 alone writes the new state,
-// to another slot than the one all of them read, and tells the host.  Up to
-// kFoldMax partials: a launch of its own takes about 3 us whatever it does;
-// folded, the sums run beside the update's own loads and add 1.0-1.5 us to
-// it.  A forward and backward solve of 64x64x32 to 1e-10 (20 iterations each)
-// 4.26 -> 3.96 ms, a 32x32x16 precision-form step 648 -> 608 us.  Every
-// workgroup repeats the sums, so their cost grows with the square of the
-// system: us per FP64 / precision-form iteration, separate and folded, at
-// 3,502 partials 138 / 110 both ways, 4,597 (4x4) 174 / 130 -> 168 / 125,
-// 6,537 212 / 149 -> 206 / 145, 10,236 261 / 179 -> 269 / 189.
-struct FoldArgs {
-    const double *part;      // the product's partials: reduction j at part + j * cap
-    int32_t cap, n;
-    const double *vpart;     // those of the vector update before it
-    int32_t vcap, vn;
-    const SolverState *in;
-    SolverState *out;
-};
-constexpr int kFoldStep = 4, kFoldMax = 8 * kFinThreads;
-static_assert(kFoldMax <= kFinThreads * kFinUnroll, "one pass of k_finalize: the same order of the sums");
-constexpr int kStateWords = sizeof(SolverState) / 8;
-static_assert(sizeof(SolverState) % 8 == 0 && kStateWords <= kVecThreads, "a state word per thread");
-
-template <int NRED, int U>
-__device__ inline void fold_waves(const double *part, int cap, int n, double (*sred)[2]) {
-    constexpr int NW = kVecThreads / 64, VW = kFinThreads / kVecThreads;  // this wave stands for VW of k_finalize's,
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;           // NW apart, so that few partials spread
-    double t[VW][NRED];
-#pragma unroll
-    for (int w = 0; w < VW; ++w)
-#pragma unroll
-        for (int j = 0; j < NRED; ++j) t[w][j] = 0.0;
-    for (int u0 = 0; u0 == 0 || (U > 1 && u0 * kFinThreads < n); u0 += U) {
-        double v[VW][NRED][U];
-#pragma unroll
-        for (int w = 0; w < VW; ++w)
-#pragma unroll
-            for (int j = 0; j < NRED; ++j)
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int i = (u0 + u) * kFinThreads + (w * NW + wave) * 64 + lane;
-                    v[w][j][u] = part[(size_t)j * cap + min(i, n - 1)];
-                }
-#pragma unroll
-        for (int w = 0; w < VW; ++w)
-#pragma unroll
-            for (int j = 0; j < NRED; ++j)
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    t[w][j] += 0.0 + ((u0 + u) * kFinThreads + (w * NW + wave) * 64 + lane < n ? v[w][j][u] : 0.0);
-    }
-#pragma unroll
-    for (int w = 0; w < VW; ++w) {
-        const int vw = w * NW + wave;
-        if (vw * 64 >= n) {  // no partials: the sum is +0.0
-            if (lane < NRED) sred[vw][lane] = 0.0;
-            continue;
-        }
-#pragma unroll
-        for (int j = 0; j < NRED; ++j) {
-            const double s = wave_sum(t[w][j]);
-            if (lane == 0) sred[vw][j] = s;
-        }
-    }
-}
-// the wave sums of NRED reductions over n <= kFoldMax partials, for fold_total
-// after a barrier
-template <int NRED>
-__device__ inline void fold_sums(const double *part, int cap, int n, double (*sred)[2]) {
-    if (n <= kFinThreads) fold_waves<NRED, 1>(part, cap, n, sred);
-    else fold_waves<NRED, kFoldStep>(part, cap, n, sred);
-}
-__device__ inline double fold_total(const double (*sred)[2], int j) {
-    double t = sred[0][j];
-    for (int w = 1; w < kFinThreads / 64; ++w) t += sred[w][j];
-    return t;
-}
-// Whether a folded run is past its deadline (thread 0 of workgroup 0, whose
-// clock decides for all): it then stops with the launch after this one, whose
-// update is still complete.
-__device__ inline int fold_late(const SolverState *ss) {
-    return blockIdx.x == 0 && !ss->done && past_deadline(ss) ? 1 : 0;
-}
-// End of a folded scalar step (all threads, after the barrier that follows
-// it): the new state.
-__device__ inline void fold_store(const FoldArgs &f, const SolverState *ss, int late) {
-    if (blockIdx.x != 0) return;
-    const int t = threadIdx.x;
-    if (t < kStateWords) {
-        uint64_t w = reinterpret_cast<const uint64_t *>(ss)[t];
-        constexpr size_t od = offsetof(SolverState, done), oa = offsetof(SolverState, aborted);
-        if (late && t == (int)(od / 8)) w |= (uint64_t)1 << (od % 8 * 8);
-        if (late && t == (int)(oa / 8)) w |= (uint64_t)1 << (oa % 8 * 8);
-        reinterpret_cast<uint64_t *>(f.out)[t] = w;
-    }
-    if (t == 0 && late && ss->host_done)
-        __hip_atomic_store(ss->host_done, ss->run_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // steps 6-8 without the x update: s = r - alpha v; ||s||^2.  Step 6,
@@ -1814,22 +1853,6 @@ __global__ __launch_bounds__(kVecThreads) void k_update_s(int64_t N, const TX *r
     }
     double vv[1] = {acc};
     block_partials<kVecThreads, 1>(vv, ra, blockIdx.x);
-}
-
-// The ||s|| test (steps 7/8) of a folded run, one workgroup.  Folded into the
-// second half's k_update_xr the run learns of a convergence in its first half
-// only after the second half's product: 2% faster over 20 iterations, 2-8%
-// slower over 2 to 5.
-__global__ __launch_bounds__(kVecThreads) void k_fold_half1(FoldArgs f) {
-    __shared__ SolverState ss;
-    __shared__ double sred[kFinThreads / 64][2];
-    if (threadIdx.x < kStateWords)
-        reinterpret_cast<uint64_t *>(&ss)[threadIdx.x] = reinterpret_cast<const uint64_t *>(f.in)[threadIdx.x];
-    fold_sums<1>(f.vpart, f.vcap, f.vn, sred);
-    __syncthreads();
-    if (threadIdx.x == 0 && !ss.done) scalar_step(&ss, FIN_HALF1, fold_total(sred, 0), 0.0, true);
-    __syncthreads();
-    fold_store(f, &ss, 0);
 }
 
 // steps 6 and 11-14: x = (x + alpha phat) + omega shat, rounded to the type

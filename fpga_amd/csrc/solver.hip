@@ -824,8 +824,19 @@ void launch_finalize(H &h, int nred, const RedArgs &ra, int nparts) {
 
 // Launches the streaming kernel, one workgroup per tile; returns the number
 // of reduction partials written.
+// half1: the ||s|| test that a sweep's launch takes along (k_stream_half1),
+// else null.
 template <int BS, int MODE, int RED, typename TV, typename TX, int ROWS = kTileRows, bool ZX = false, bool PLAIN = false>
-int stream_dispatch(H &h, const StreamArgs<TV, TX> &a) {
+int stream_dispatch(H &h, const StreamArgs<TV, TX> &a, const FoldArgs *half1 = nullptr) {
+    if constexpr (RED == SR_NONE && !ZX && (MODE == SM_SUB || MODE == SM_SUB_DINV || MODE == SM_SUB_Z)) {
+        if (half1) {
+            hipLaunchKernelGGL((k_stream_half1<BS, MODE, TV, TX, ROWS, PLAIN>), dim3(a.ntiles + 1), dim3(64 * BS), 0,
+                               h.stream, a, *half1);
+            check_launch();
+            return a.ntiles;
+        }
+    }
+    if (half1) throw std::runtime_error("this launch takes no scalar step along");
     hipLaunchKernelGGL((k_stream<BS, MODE, RED, TV, TX, ROWS, ZX, PLAIN>), dim3(a.ntiles), dim3(64 * BS), 0, h.stream, a);
     check_launch();
     return a.ntiles;
@@ -845,7 +856,7 @@ template <int BS, int MODE, int RED, typename TV, typename TX, bool ZX = false>
 void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x, const TX *rhs, TX *out,
                    const double *dinv, const TX *w0, RedArgs ra, bool use_state, TX *out2 = nullptr,
                    TX *out3 = nullptr, const TX *x_lo = nullptr, int split = 0, int prof_kind = -1,
-                   const int32_t *rowptr2 = nullptr, TX *zout = nullptr) {
+                   const int32_t *rowptr2 = nullptr, TX *zout = nullptr, const FoldArgs *half1 = nullptr) {
     constexpr int nred = (RED & SR_W0 ? 1 : 0) + (RED & SR_SELF ? 1 : 0);
     StreamArgs<TV, TX> a;
     constexpr bool wide = wide_tiles<MODE>();
@@ -864,7 +875,10 @@ void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x
         a.tile0 = ct[colour];
         a.ntiles = ct[colour + 1] - ct[colour];
     }
-    if (a.ntiles <= 0) return;
+    if (a.ntiles <= 0) {
+        if (half1) throw std::runtime_error("no launch to take the scalar step along");
+        return;
+    }
     // a sweep colour with few blocks per row takes the tall tiling when that
     // saves a quarter of the workgroups or more
     bool tall = false;
@@ -907,14 +921,14 @@ void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x
         bool done = false;
         if constexpr (plain_small<TV>() && !ZX) {
             if (a.ntiles < kPlainBelow) {
-                if (tall) nparts = stream_dispatch<BS, MODE, RED, TV, TX, kTileRowsTall, false, true>(h, a);
-                else nparts = stream_dispatch<BS, MODE, RED, TV, TX, kTileRows, false, true>(h, a);
+                if (tall) nparts = stream_dispatch<BS, MODE, RED, TV, TX, kTileRowsTall, false, true>(h, a, half1);
+                else nparts = stream_dispatch<BS, MODE, RED, TV, TX, kTileRows, false, true>(h, a, half1);
                 done = true;
             }
         }
         if (!done) {
-            if (tall) nparts = stream_dispatch<BS, MODE, RED, TV, TX, kTileRowsTall>(h, a);
-            else nparts = stream_dispatch<BS, MODE, RED, TV, TX, kTileRows, ZX>(h, a);
+            if (tall) nparts = stream_dispatch<BS, MODE, RED, TV, TX, kTileRowsTall>(h, a, half1);
+            else nparts = stream_dispatch<BS, MODE, RED, TV, TX, kTileRows, ZX>(h, a, half1);
         }
     } else {
         nparts = stream_dispatch<BS, MODE, RED, TV, TX, kTileRows, ZX>(h, a);
@@ -979,14 +993,14 @@ int vec_blocks(size_t N) { return (int)((N + kVecElemsPerBlock - 1) / kVecElemsP
 
 template <int BS, typename TV, typename TX>
 void sweep_launch(H &h, const DevMat &m, const TV *val, int c, bool dinv_mode, const TX *x, const TX *x_lo, int split,
-                  const TX *rhs, TX *out, const double *dinv, int si) {
+                  const TX *rhs, TX *out, const double *dinv, int si, const FoldArgs *half1 = nullptr) {
     RedArgs ra = red(h, si, FIN_NONE);
     if (dinv_mode)
         launch_stream<BS, SM_SUB_DINV, SR_NONE, TV, TX>(h, m, val, c, x, rhs, out, dinv, nullptr, ra, true,
-                                                        nullptr, nullptr, x_lo, split);
+                                                        nullptr, nullptr, x_lo, split, -1, nullptr, (TX *)nullptr, half1);
     else
         launch_stream<BS, SM_SUB, SR_NONE, TV, TX>(h, m, val, c, x, rhs, out, nullptr, nullptr, ra, true, nullptr,
-                                                   nullptr, x_lo, split);
+                                                   nullptr, x_lo, split, -1, nullptr, (TX *)nullptr, half1);
 }
 
 // The first sweep's last colour C-1 and the second sweep's colour C-2 in one
@@ -1189,7 +1203,8 @@ template <> const float *low2_values<float>(H &h) { return h.low2_v32.p; }
 // skip_last: everything but the second sweep's colour 0 (launch_sweep_spmv
 // follows).
 template <int BS, typename TV, typename TX>
-void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si, bool skip_last = false) {
+void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si, bool skip_last = false,
+             const FoldArgs *half1 = nullptr) {
     const int nc = h.an.ncolours;
     if (op.s1_dinv && op.s2_dinv) throw std::runtime_error("at most one sweep may carry the diagonal inverse");
     const bool skip0 = !op.s1_dinv && nc > 1;
@@ -1200,7 +1215,18 @@ void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si, bool 
     // (with three colours the extended tail would cover colour 0)
     const bool merge3 = merge && h.tail3 && !op.s1_dinv && op.s2_dinv && op.S2->tail3_n >= 0 && !(skip_last && nc == 3);
     const bool low2 = h.low2 && skip0 && op.S1->low2_n >= 0 && nc >= 4 && op.S1 == &h.L;
+    // the first launch takes the ||s|| test along, unless it is k_lower2 (or
+    // has more partials to add up than the test in passing does)
+    auto take_half1 = [&] {
+        const FoldArgs *f = half1;
+        half1 = nullptr;
+        return f;
+    };
     prof_begin(h, PK_LOWER);
+    if (half1 && (h.profiling || (low2 && nc == 4) || half1->vn > kFinThreads)) {
+        hipLaunchKernelGGL(k_fold_half1, dim3(1), dim3(kVecThreads), 0, h.stream, *take_half1());
+        check_launch();
+    }
     for (int c = skip0 ? 1 : 0; c < nc - 1; ++c) {
         if (low2 && c == nc - 3) {
             lower2_launch<BS, TV, TX>(h, op, low2_values<TV>(h), p, y, lo, split, merge3 ? z : nullptr, si);
@@ -1208,13 +1234,13 @@ void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si, bool 
         } else if (merge3 && c == nc - 2)
             launch_stream<BS, SM_SUB_Z, SR_NONE, TV, TX>(h, *op.S1, op.S1val, c, y, p, y, op.dinv, nullptr,
                                                          red(h, si, FIN_NONE), true, nullptr, nullptr, lo, split,
-                                                         -1, op.S2->rowptr.p, z);
+                                                         -1, op.S2->rowptr.p, z, take_half1());
         else
-            sweep_launch<BS, TV, TX>(h, *op.S1, op.S1val, c, op.s1_dinv, y, lo, split, p, y, op.dinv, si);
+            sweep_launch<BS, TV, TX>(h, *op.S1, op.S1val, c, op.s1_dinv, y, lo, split, p, y, op.dinv, si, take_half1());
     }
     if (!merge)
         sweep_launch<BS, TV, TX>(h, *op.S1, op.S1val, nc - 1, op.s1_dinv || op.s2_dinv, y, lo, split, p, z, op.dinv,
-                                 si);
+                                 si, take_half1());
     prof_end(h);
     prof_begin(h, PK_UPPER);
     if (merge3) tail3_launch<BS, TV, TX>(h, op, y, lo, split, p, z, (nc - 3 == 0 && skip0) ? p : y, si);
@@ -1510,10 +1536,18 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     };
     double *spart = h.vparts.p, *xrpart = h.vparts.p + vb;
     // z = M^-1 p, and, fused, the colour-0 rows of v = A z with their dots
-    auto apply = [&](auto redc, const TX *p, TX *z, TX *v, const TX *w0) {
+    // (half1: the ||s|| test of a folded run, still to be made)
+    auto apply = [&](auto redc, const TX *p, TX *z, TX *v, const TX *w0, const FoldArgs *half1) {
         constexpr int RED = decltype(redc)::value;
-        if (wait) precond_wait<BS, TV, TX>(h, op, p, k.y.p, z, 0);
-        else precond<BS, TV, TX>(h, op, p, k.y.p, z, 0, fuse);
+        if (wait) {
+            if (half1) {
+                hipLaunchKernelGGL(k_fold_half1, dim3(1), dim3(kVecThreads), 0, h.stream, *half1);
+                check_launch();
+            }
+            precond_wait<BS, TV, TX>(h, op, p, k.y.p, z, 0);
+        } else {
+            precond<BS, TV, TX>(h, op, p, k.y.p, z, 0, fuse, half1);
+        }
         if (fuse) {
             prof_begin(h, PK_UPPER);
             launch_sweep_spmv<BS, RED, TV, TX>(h, op, p, z, v, w0, red(h, 0, FIN_NONE));
@@ -1547,7 +1581,7 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     const dim3 vg(vb), vt(kVecThreads);
     for (int it = 1; it <= maxit + 1 && !stop; ++it) {
         h.prof_tag = 2 * (it - 1);
-        apply(red_w0, k.p.p, k.phat.p, k.v.p, k.rt.p);
+        apply(red_w0, k.p.p, k.phat.p, k.v.p, k.rt.p, nullptr);
         throttle(2 * it - 1);
         if (stop) break;
         product(red_w0, k.phat.p, k.v.p, k.rt.p, FIN_ALPHA);
@@ -1555,8 +1589,6 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
         if (fold) {
             hipLaunchKernelGGL((k_update_s<TX, true>), vg, vt, 0, h.stream, (int64_t)N, k.r.p, k.v.p, k.s.p,
                                vec_red(FIN_NONE, spart), fold_args(0, kStateB, nullptr));
-            check_launch();
-            hipLaunchKernelGGL(k_fold_half1, dim3(1), vt, 0, h.stream, fold_args(kStateB, 0, spart));
             check_launch();
         } else {
             hipLaunchKernelGGL((k_update_s<TX, false>), vg, vt, 0, h.stream, (int64_t)N, k.r.p, k.v.p, k.s.p,
@@ -1566,7 +1598,8 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
         }
         prof_end(h);
         h.prof_tag = 2 * (it - 1) + 1;
-        apply(red_both, k.s.p, k.shat.p, k.t.p, k.s.p);
+        const FoldArgs half1 = fold_args(kStateB, 0, spart);
+        apply(red_both, k.s.p, k.shat.p, k.t.p, k.s.p, fold ? &half1 : nullptr);
         throttle(2 * it);
         if (stop) break;
         product(red_both, k.shat.p, k.t.p, k.s.p, FIN_OMEGA);
