@@ -10,7 +10,7 @@ form (FP32 matrix/factor values and inner vectors, FP64 sums, scalars,
 diagonal inverses and refinement).  ``value`` is the precision form's time
 per solve; the FP64 time, iteration counts, the error of each against a
 1e-12 FP64 solve, the roofline of the dominant kernel (the precision form's
-FP32 SpMV, timed inside a solve) and the CPU oracle baseline are in the same
+FP32 SpMV, launched back to back) and the CPU oracle baseline are in the same
 JSON line.
 
 Beside the headline the line carries, measured in the same run:
@@ -145,7 +145,9 @@ def main():
     err64 = (torch.linalg.vector_norm(x - x_ref).item() / nref)
 
     # one more FP64 solve, untimed, with every launch bracketed by HIP events
-    # on the solver's stream (per-kernel-class averages)
+    # on the solver's stream (per-kernel-class averages).  Where a solve merges
+    # colour 0's upper sweep with the product of its rows, that launch counts
+    # as an upper sweep and the SpMV's launches are those over the other rows
     g.set_profiling(True)
     run_fp64()
     spmv64_in = in_solve_avg(g.kernel_times(fa.KIND_SPMV))
@@ -174,9 +176,10 @@ def main():
     spmv32_bytes = g.algorithmic_bytes(fa.KIND_SPMV, True)
     # roofline of the dominant kernel of the timed solve, the precision
     # form's FP32 SpMV: 20 back-to-back launches between two HIP events on
-    # the solver's stream (per launch the same time as inside a solve in the
-    # kernel trace; the FP64 one gains a few percent back to back, part of
-    # its values staying in the 256 MB last-level cache between launches)
+    # the solver's stream, over all rows (per launch the same time as inside a
+    # solve with separate launches in the kernel trace; the FP64 one gains a
+    # few percent back to back, part of its values staying in the 256 MB
+    # last-level cache between launches)
     spmv_ms = g.time_spmv(20, False)
     spmv32_ms = g.time_spmv(20, True)
     # the roofline kernel is the SpMV instance with the fused v.rt sums: its
@@ -193,7 +196,9 @@ def main():
             traffic = t["fp32"]["read_bytes"] + t["fp32"]["write_bytes"]
     low_bytes, up_bytes = g.algorithmic_bytes(fa.KIND_LOWER), g.algorithmic_bytes(fa.KIND_UPPER)
     iters64 = r64.iterations
-    # algorithmic bytes per FP64 iteration: 2 SpMV + 2 (L + U) + 22 N vector passes
+    # algorithmic bytes per FP64 iteration: 2 SpMV + 2 (L + U) + 22 N vector passes,
+    # each as a pass of its own (a merged sweep and product reads colour 0's
+    # blocks once for both, so the rate counts them twice)
     it_bytes = 2 * spmv_bytes + 2 * (low_bytes + up_bytes) + 22 * s.N * 8
     solve_gbs = it_bytes * iters64 / t_fp64 / 1e9
     mixed_it_bytes = (2 * g.algorithmic_bytes(fa.KIND_SPMV, True)
@@ -302,9 +307,10 @@ def setup(fa, spec, torch):
 def level_block(fa, torch, dev, name, s, b, x_ref, tol, maxit, steps, coloured):
     """The same system and right-hand side with level scheduling instead of
     the colouring (the host API's level_scheduling flag,
-    fpga_functions_bicgstab.cpp:84): one level set per sweep launch, so the
-    preconditioner costs one launch per level and sweep, against fewer
-    iterations from the natural-order ILU0.  FP64 and precision-form solves
+    fpga_functions_bicgstab.cpp:84): fewer iterations from the natural-order
+    ILU0, but each sweep passes through the levels one after another (in a
+    solve as one launch whose workgroups wait for one another, in an
+    application by itself as one launch per level).  FP64 and precision-form solves
     to the same tolerance, their errors against the same 1e-12 solution, and
     one preconditioner application back to back in each form."""
     g = fa.BicgstabSolver(s.bs, s.n, s.nnzb)

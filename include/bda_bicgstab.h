@@ -289,7 +289,10 @@ int bda_spmv_perm_ex(bda_handle h, int32_t prec, const void *x, void *y, int32_t
 int bda_precond_apply_perm_ex(bda_handle h, int32_t prec, const void *p, void *z, int32_t transpose);
 /* Kernel launches one application of the preconditioner makes (transpose
  * != 0: of the adjoint's), after bda_analyse: one per colour and sweep, less
- * the launches the colouring lets the library merge.  No counterpart in the
+ * the launches the colouring lets the library merge.  These are the launches
+ * of an application by itself (bda_precond_apply_perm*, bda_time_precond); a
+ * solve may run the sweeps of many small colours as two launches, or the last
+ * launch together with the product of colour 0's rows.  No counterpart in the
  * reference, whose sweeps run colour by colour inside one kernel run
  * (rtl/bicgstab_solver_2r-3r3w/int_read_unit.vhd:287-302); for callers that
  * budget launch latency. */
@@ -414,7 +417,9 @@ int bda_get_kernel_stats(bda_handle h, int32_t kind, int64_t *launches, double *
 /* The individual durations (ms) of the launches counted above, in launch
  * order: up to capacity values go to ms, *count receives how many there
  * are.  Kind 0 brackets the streaming SpMV kernel alone (not the reduction
- * that follows it).  A diagnostic of this build; no counterpart in the
+ * that follows it); where a solve computes the product of colour 0's rows
+ * together with their upper sweep, that launch is of kind 2 and kind 0 is the
+ * launch over the other rows.  A diagnostic of this build; no counterpart in the
  * reference. */
 int bda_get_kernel_times(bda_handle h, int32_t kind, float *ms, int32_t capacity, int32_t *count);
 /* reps back-to-back launches of the solve's SpMV kernel (v = A phat with
