@@ -964,9 +964,7 @@ template <typename TV> constexpr bool plain_small() { return std::is_same<TV, fl
 // packed row's matrix row, for its right-hand side); its outputs only go to
 // keep[]; 2, a tile whose column indices below zero name a row of the
 // dependency tile: -1 - c is the row's place there, and its x comes from
-// ldsx[] (that tile's keep[]) instead of memory.  3, a tile of a waiting sweep
-// (k_sweep_wait): its x entries are waited for, its outputs are stored for
-// tiles that wait.
+// ldsx[] (that tile's keep[]) instead of memory.
 template <int BS, int MODE, int RED, typename TV, typename TX, int ROWS, bool KEEP, bool PLAIN = false, int V = 0>
 __device__ __attribute__((always_inline)) inline void stream_tile(const StreamArgs<TV, TX> &a, const int4 d, TX *keep,
                                                                    int slot, const TX *ldsx = nullptr) {
@@ -1116,51 +1114,6 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
     XVec<TX, BS> xg[XV];
     int xq[XV];
     int xl[XV];
-    if constexpr (V == 3) {
-        using Bits = typename NotYet<TX>::Bits;
-        const TX *src[XV];
-        bool ready[XV], free[XV], all = false;  // free: nothing to wait for
-#pragma unroll
-        for (int j = 0; j < XV; ++j) {
-            xq[j] = min(t + j * NT, nblk > 0 ? nblk - 1 : 0);
-            const int cb = nblk > 0 ? ci[j] : 0;
-            src[j] = (cb < a.split ? a.x_lo : a.x) + (size_t)cb * BS;
-            ready[j] = false;
-            free[j] = nblk == 0 || cb < a.split;
-        }
-        uint64_t since = 0;
-        for (uint32_t spin = 0; !all; ++spin) {
-            if (spin > 0) {
-                __builtin_amdgcn_s_sleep(1);
-                if ((spin & 255) == 0) {
-                    const uint64_t now = wall_clock64();
-                    if (since == 0) since = now;
-                    bool over = __hip_atomic_load(a.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-                    if (!over && now - since > kWaitTicks) {
-                        over = true;
-                        __hip_atomic_store(a.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        __hip_atomic_store(a.host_fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                    }
-                    if (over) break;
-                }
-            }
-            all = true;
-            Bits w[XV][BS];
-#pragma unroll
-            for (int j = 0; j < XV; ++j)
-#pragma unroll
-                for (int c = 0; c < BS; ++c) w[j][c] = load_entry(src[j] + c);
-#pragma unroll
-            for (int j = 0; j < XV; ++j) {
-                bool r = true;
-#pragma unroll
-                for (int c = 0; c < BS; ++c) r = r && w[j][c] != NotYet<TX>::mark;
-                if (!ready[j]) __builtin_memcpy(&xg[j], w[j], sizeof(xg[j]));
-                ready[j] = ready[j] || r || free[j];
-                all = all && ready[j];
-            }
-        }
-    } else
 #pragma unroll
     for (int j = 0; j < XV; ++j) {
         const int q = min(t + j * NT, nblk > 0 ? nblk - 1 : 0);
@@ -1343,10 +1296,7 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
         const TX o = from_double<TX>(res[s]);
         if constexpr (KEEP) keep[t] = o;
         if constexpr (MODE == SM_SUB_SPMV) a.vout[gi[s]] = o;
-        else if constexpr (V == 3) {
-            store_entry(&a.out[gi[s]], o);
-            if (a.reset) mark_entry(&a.reset[gi[s]]);
-        } else if constexpr (V != 1) {
+        else if constexpr (V != 1) {
             a.out[gi[s]] = o;
             if (a.out2) a.out2[gi[s]] = o;
             if (a.out3) a.out3[gi[s]] = o;
@@ -1700,20 +1650,32 @@ __global__ __launch_bounds__(64 * BS) void k_lower2(StreamArgs<TV, TX> a, Stream
 // depend on other tiles, then waits for the x entries it reads, entry by
 // entry (NotYet): the hop from one level to the next is one store and one
 // load instead of a launch.  Every tile waits only for tiles of earlier
-// tickets, each held by a workgroup that runs and itself waits only for
+// tickets, each held by a workgroup that runs, takes its tiles in ticket order
+// (it fetches the next ticket while it works on one) and waits only for
 // earlier ones, so the first unfinished tile never waits and the sweep ends
 // however few workgroups are resident; ticket numbers are bounded, so every
 // workgroup ends.
+//
+// A quad of lanes serves a row, lane r its component r; each wave 16 rows, by
+// itself.  The chain is what counts here: lane r polls component r of the
+// row's x blocks (the quad's loads are one access) and hands it to the quad's
+// other lanes by DPP, so between the load that brings the last entry and the
+// row's store there is only arithmetic, no LDS and no barrier.
 //
 // The first sweep writes y, except that the last level (which has no blocks
 // in the second sweep) goes to z with the diagonal inverse, as when launched
 // by itself; it marks the other z entries as not written, the second sweep
 // the y entries, and each clears the other's ticket counter: y and the
 // counters only have to be prepared once per run (k_sweep_reset).  The
-// arithmetic is k_stream's.  It is bound by the chain: 1.1 us from level to
-// level (store, poll, the tile's LDS exchanges) against 2.8 us for a launch
-// per level; the 48x48x24 level-scheduled FP64 step 33.6 -> 14.6 ms, 128x128x64
-// 150 -> 49 ms.
+// arithmetic and its order are k_stream's.  It is bound by the chain, about
+// 1.0 us from level to level (the store on its way to memory, the poll, two
+// dozen dependent FP64 operations) against 2.8 us for a launch per level: the
+// 48x48x24 level-scheduled FP64 step 33.6 -> 11.6 ms, 96x96x48 30.7 ms,
+// 128x128x64 150 -> 43 ms (with k_stream's tile, three barriers and LDS
+// exchanges a hop, 1.3 us: 14.6, 37.5 and 48.9).  Every load of a poll costs time (a
+// fixed four per lane instead of the wave's need: 12.5, 32.8 and 46.5), and
+// so do two polls in flight (k_stream's tile: 14.1 -> 16.5) and longer sleeps
+// between polls (64 clocks 14.1, 128 14.3, 256 14.5, 640 15.4).
 template <typename TX>
 struct WaitArgs {
     int32_t *ticket, *other;   // this sweep's ticket counter and the other's
@@ -1725,27 +1687,134 @@ struct WaitArgs {
     TX *z;
 };
 
+// v of the quad's lane C (DPP)
+template <int C> __device__ inline int quad_lane(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, C * 0x55 /* quad_perm:[C,C,C,C] */, 0xF, 0xF, true);
+}
+template <int C> __device__ inline double quad_lane(double v) {
+    return __hiloint2double(quad_lane<C>(__double2hiint(v)), quad_lane<C>(__double2loint(v)));
+}
+template <int C> __device__ inline float quad_lane(float v) { return __int_as_float(quad_lane<C>(__float_as_int(v))); }
+template <int BS, typename T> __device__ inline void quad_all(T v, T (&o)[BS]) {
+    o[0] = quad_lane<0>(v);
+    o[1] = quad_lane<1>(v);
+    o[2] = quad_lane<2>(v);
+    if constexpr (BS == 4) o[3] = quad_lane<3>(v);
+}
+
+constexpr int kWaitThreads = 256, kWaitBlocks = 4;  // rows of a tile * 4; blocks of a row at a time
 template <int BS, int MODE, typename TV, typename TX>
-__global__ __launch_bounds__(64 * BS) void k_sweep_wait(StreamArgs<TV, TX> a, WaitArgs<TX> w) {
+__global__ __launch_bounds__(kWaitThreads) void k_sweep_wait(StreamArgs<TV, TX> a, WaitArgs<TX> w) {
     if (a.ra.st->done) return;
-    __shared__ int tk;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *w.other = 0;
-    for (;;) {
-        if (threadIdx.x == 0) tk = __hip_atomic_fetch_add(w.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        const int k = tk;
-        if (k >= w.ntiles) return;
-        const int4 d = a.tile[a.tile0 + (w.reverse ? w.ntiles - 1 - k : k)];
-        StreamArgs<TV, TX> b = a;
-        if (d.x < w.rhs_split) b.rhs = w.rhs_lo;
-        if (d.x >= w.last_row0) {
-            b.out = w.z;
-            b.reset = nullptr;
-            stream_tile<BS, SM_SUB_DINV, SR_NONE, TV, TX, 64, false, plain_small<TV>(), 3>(b, d, nullptr, 0);
-        } else {
-            stream_tile<BS, MODE, SR_NONE, TV, TX, 64, false, plain_small<TV>(), 3>(b, d, nullptr, 0);
+    using Bits = typename NotYet<TX>::Bits;
+    constexpr int MB = kWaitBlocks, BB = BS * BS;
+    static_assert(MB == 4);
+    constexpr bool PLAIN = plain_small<TV>();
+    __shared__ int tk[2];
+    const int t = threadIdx.x, k = t >> 2, r = min(t & 3, BS - 1);
+    if (blockIdx.x == 0 && t == 0) *w.other = 0;
+    auto take = [&] { return __hip_atomic_fetch_add(w.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    if (t == 0) tk[0] = take();
+    __syncthreads();
+    for (int p = 0;; p ^= 1) {
+        const int ticket = tk[p];
+        if (ticket >= w.ntiles) return;
+        const int4 d = a.tile[a.tile0 + (w.reverse ? w.ntiles - 1 - ticket : ticket)];
+        const int nrow = d.z - d.x;
+        int next = 0;
+        if (t == 0) next = take();
+        if ((t >> 6) * 16 < nrow) {  // this wave has rows
+            const bool last = d.x >= w.last_row0;
+            const bool inv = MODE == SM_SUB_DINV || last;
+            const int i = d.x + min(k, nrow - 1);
+            const size_t gi = (size_t)i * BS + r;
+            const int q0 = a.rowptr[i], q1 = a.rowptr[i + 1];
+            const double rhs = (double)(d.x < w.rhs_split ? w.rhs_lo : a.rhs)[gi];
+            double dv[BS];
+            if (inv)
+#pragma unroll
+                for (int c = 0; c < BS; ++c) dv[c] = a.dinv[gi * BS + c];
+            double sum = 0.0;
+            // M blocks of the row from q on (clamped to its last one), M as the
+            // wave's rows need
+            auto blocks = [&](auto m, int q) {
+                constexpr int M = decltype(m)::value;
+                int cb[M];
+                TV av[M][BS];
+#pragma unroll
+                for (int j = 0; j < M; ++j) {
+                    const int qj = min(q + j, q1 - 1);
+                    cb[j] = load_mat<PLAIN>(&a.colidx[qj]);
+#pragma unroll
+                    for (int c = 0; c < BS; ++c) av[j][c] = load_mat<PLAIN>(&a.val[(size_t)qj * BB + r * BS + c]);
+                }
+                const TX *src[M];
+                TX got[M];
+                bool ready[M], free[M], all = false;  // free: nothing to wait for
+#pragma unroll
+                for (int j = 0; j < M; ++j) {
+                    src[j] = (cb[j] < a.split ? a.x_lo : a.x) + (size_t)cb[j] * BS + r;
+                    ready[j] = false;
+                    free[j] = cb[j] < a.split;
+                }
+                uint64_t since = 0;
+                for (uint32_t spin = 0; !all; ++spin) {
+                    if (spin > 0) {
+                        __builtin_amdgcn_s_sleep(1);
+                        if ((spin & 255) == 0) {
+                            const uint64_t now = wall_clock64();
+                            if (since == 0) since = now;
+                            bool over = __hip_atomic_load(a.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+                            if (!over && now - since > kWaitTicks) {
+                                over = true;
+                                __hip_atomic_store(a.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                __hip_atomic_store(a.host_fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                            }
+                            if (over) break;
+                        }
+                    }
+                    all = true;
+                    Bits e[M];
+#pragma unroll
+                    for (int j = 0; j < M; ++j) e[j] = load_entry(src[j]);
+#pragma unroll
+                    for (int j = 0; j < M; ++j) {
+                        if (!ready[j]) __builtin_memcpy(&got[j], &e[j], sizeof(TX));
+                        ready[j] = ready[j] || free[j] || e[j] != NotYet<TX>::mark;
+                        all = all && ready[j];
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < M; ++j) {
+                    TX xs[BS];
+                    quad_all<BS>(got[j], xs);
+                    double sm = prod<TV, TX>(av[j][0], xs[0]);
+#pragma unroll
+                    for (int c = 1; c < BS; ++c) sm = sm + prod<TV, TX>(av[j][c], xs[c]);
+                    if (q + j < q1) sum += sm;
+                }
+            };
+            for (int q = q0; q < q1; q += MB) {  // (a quad's lanes stay together)
+                if (__ballot(q + 3 < q1)) blocks(std::integral_constant<int, MB>{}, q);
+                else if (__ballot(q + 2 < q1)) blocks(std::integral_constant<int, 3>{}, q);
+                else if (__ballot(q + 1 < q1)) blocks(std::integral_constant<int, 2>{}, q);
+                else blocks(std::integral_constant<int, 1>{}, q);
+            }
+            double res = rhs - sum;
+            if (inv) {
+                double tv[BS], z = 0.0;
+                quad_all<BS>(res, tv);
+#pragma unroll
+                for (int c = 0; c < BS; ++c) z += dv[c] * tv[c];
+                res = z;
+            }
+            if (k < nrow && (t & 3) < BS) {
+                store_entry(&(last ? w.z : a.out)[gi], from_double<TX>(res));
+                if (!last) mark_entry(&a.reset[gi]);
+            }
         }
-        __syncthreads();  // the tile's LDS, and tk
+        if (t == 0) tk[p ^ 1] = next;
+        __syncthreads();
     }
 }
 

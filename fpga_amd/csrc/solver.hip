@@ -1254,9 +1254,11 @@ void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si, bool 
 // Workgroups of a waiting sweep: enough for kWaitLevelsAhead of its widest
 // levels, so that a level's tiles have loaded their operands when their turn
 // comes, and few enough that those waiting do not crowd the memory system
-// (128x128x64 by level sets, FP64 step by levels ahead: 1: 57.1 ms, 2: 49.0,
-// 4: 50.9, 6: 53.0, 12: 60.3; 48x48x24: 17.9, 14.6, 14.7, 14.7, 14.8).
-constexpr int kWaitLevelsAhead = 2;
+// (FP64 step by levels ahead: 48x48x24 by level sets with 2, 3, 4: 13.3, 12.4,
+// 12.1 ms; with 4, 6, 8: 12.5, 12.3, 12.3, 96x96x48 32.9, 33.0, 34.5, 128x128x64
+// 46.5, 48.0, 51.0; after the loads of a poll were cut to the wave's need, 3 and
+// 4: 11.9 and 11.6, 31.4 and 30.7, 41.8 and 43.2).
+constexpr int kWaitLevelsAhead = 4;
 int wait_grid(const DevMat &m, int c0, int c1) {
     int widest = 1;
     for (int c = c0; c < c1; ++c) widest = std::max(widest, m.colour_tile[c + 1] - m.colour_tile[c]);
@@ -1297,7 +1299,7 @@ void precond_wait(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si) 
     w.last_row0 = h.an.colour_ptr[nc - 1];
     w.z = z;
     prof_begin(h, PK_LOWER);
-    const dim3 g1(wait_grid(m1, c0, nc)), b(64 * BS);
+    const dim3 g1(wait_grid(m1, c0, nc)), b(kWaitThreads);
     if (op.s1_dinv) hipLaunchKernelGGL((k_sweep_wait<BS, SM_SUB_DINV, TV, TX>), g1, b, 0, h.stream, a, w);
     else hipLaunchKernelGGL((k_sweep_wait<BS, SM_SUB, TV, TX>), g1, b, 0, h.stream, a, w);
     check_launch();
@@ -1363,22 +1365,22 @@ bool fuse_sweep_spmv(const H &h, const OpSet<TV> &op) {
 }
 
 // Whether a solve runs its sweeps as two launches whose tiles wait for one
-// another (k_sweep_wait).  A launch of a small colour or level costs 2.8 us, a
-// waiting sweep's about 4.2, and its tiles about 10 ns each more than
-// k_stream's (their gathers go past the L2): it pays from four launches on
-// and up to kWaitTilesPerLaunch tiles for each launch above three.  us per
-// FP64 iteration, launches / waiting: 4 colours of 110 to 3 rows, forward (3
-// launches) 59.8 / 58.8, adjoint (6) 74.3 / 61.4; of 811 to 15 rows (4) 68.6 /
-// 59.9; 5 colours of 12116 to 1 rows, 5 launches 87.3 / 97.1, 8 launches 108 /
-// 106; 2 colours of 8192 51.9 / 70.4; 16 levels of 2000 rows 295 / 156; of
-// 20000 rows 406 / 420.
-constexpr int kWaitTilesPerLaunch = 280;
+// another (k_sweep_wait).  A launch of a small colour or level costs 2.8 us;
+// two waiting sweeps cost about as much as six, and their tiles 13 to 19 ns
+// each more than k_stream's (their gathers go past the L2).  us per FP64
+// iteration, launches / waiting: 4 colours of 811 to 15 rows, 4 launches 56.3 /
+// 60.5, the adjoint's 6 61.3 / 60.4 (4x4 61.6 / 64.8); 5 colours of 12116 to 1
+// rows, 8 launches 83.8 / 121.7; level sets, 7 of 27 rows in all 102 / 58, 6 of
+// 2,000 each 111 / 81 and of 20,000 154 / 245, 10 of 2,000 177 / 103 and of
+// 20,000 253 / 332, 16 of 2,000 301 / 133 and of 20,000 364 / 484: even at
+// about 1,200 tiles with 10 launches, 3,400 with 18, 6,700 with 30.
+constexpr int kWaitLaunches = 6, kWaitTilesPerLaunch = 270;
 template <typename TV>
 bool sweeps_wait(const H &h, const OpSet<TV> &op) {
     if (!h.wait) return false;
     const int launches = precond_launches(h, op);
     const int64_t tiles = (int64_t)op.S1->ntiles + op.S2->ntiles;
-    return launches >= 4 && tiles < (int64_t)kWaitTilesPerLaunch * (launches - 3);
+    return launches > kWaitLaunches && tiles < (int64_t)kWaitTilesPerLaunch * (launches - kWaitLaunches);
 }
 
 struct RunOut {
