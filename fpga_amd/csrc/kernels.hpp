@@ -756,13 +756,21 @@ struct StreamArgs {
     const int32_t *rowptr2 = nullptr;  // SUB_Z: the second sweep's row pointers
     TX *zout = nullptr;                // SUB_Z: z of the rows without second-sweep blocks
     const int32_t *rowmap = nullptr;   // dependency tiles (k_lower2): matrix row of each packed row
-    const int32_t *full = nullptr;     // step-0 residual: the id of a run that needs the product
-    TX *reset = nullptr;               // waiting tiles: entries to mark as not written (see k_sweep_wait)
-    int32_t *fail = nullptr;           // waiting tiles: a wait has run out; on the device, and for the host
-    int32_t *host_fail = nullptr;
-    const TV *adiag = nullptr;         // SUB_SPMV: A's diagonal blocks of colour 0
-    TX *vout = nullptr;                // SUB_SPMV: v = A out of the tile's rows
 };
+// What one launch form alone needs comes behind these, so that the others'
+// arguments do not grow with it.
+template <typename TV, typename TX>
+struct StartArgs : StreamArgs<TV, TX> {  // ZX
+    const int32_t *full;  // the id of the last run that needs the step-0 product
+};
+template <typename TV, typename TX>
+struct SweepSpmvArgs : StreamArgs<TV, TX> {  // SM_SUB_SPMV
+    const TV *adiag;  // A's diagonal blocks of colour 0
+    TX *vout;         // v = A out of the tile's rows
+};
+template <int MODE, bool ZX, typename TV, typename TX>
+using ArgsOf = std::conditional_t<MODE == SM_SUB_SPMV, SweepSpmvArgs<TV, TX>,
+                                  std::conditional_t<ZX, StartArgs<TV, TX>, StreamArgs<TV, TX>>>;
 
 template <typename TV, typename TX>
 __device__ inline double prod(TV a, TX x);
@@ -1057,6 +1065,14 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
         }
     }
 
+    // The product by itself starts on an idle chip: its gathers' arguments come
+    // from a line of the argument block that no cache holds yet, so their load
+    // is kept behind the values' (ahead of them it held them up: 33x32x16 FP32
+    // 3.72 -> 3.90 us, the call 14.5 -> 14.9 us).  In a solve that line is warm
+    // and the compiler's order is the faster one (FP64 with a dot 4.8 us, 5.1
+    // with the values first).
+    if constexpr (MODE == SM_SPMV && RED == SR_NONE) __builtin_amdgcn_sched_barrier(0);
+
     // 3. per-row operands of the epilogue: thread t serves scalar row r of
     // block rows k0 and (ROWS = 128) k0 + 64
     const int k0 = t / BS, r = t - k0 * BS;
@@ -1085,7 +1101,7 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
         if constexpr ((RED & SR_W0) != 0) w_v[s] = (double)a.w0[gi[s]];
         if constexpr (MODE == SM_SUB_SPMV) {
 #pragma unroll
-            for (int c = 0; c < BS; ++c) dg[c] = a.adiag[gi[s] * BS + c];
+            for (int c = 0; c < BS; ++c) dg[c] = static_cast<const SweepSpmvArgs<TV, TX> &>(a).adiag[gi[s] * BS + c];
         }
         if constexpr (MODE == SM_SUB_DINV || MODE == SM_SUB_Z || MODE == SM_SUB_SPMV) {
             const double *D = a.dinv + gi[s] * BS;
@@ -1099,11 +1115,12 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
     }
 
     srow[t] = rp - b0;
-    // Launches that fill the chip keep the barrier that staging the columns in
-    // LDS used to need: with it their waves issue their gathers together
-    // (without: precision form on 128x128x64 6.02 -> 6.10 ms).  The sweeps of
-    // smaller systems are shorter without it (64x64x32 FP64 forward and
-    // backward 3.87 -> 3.80 ms).
+    // The products and the FP32 sweeps of many tiles keep the barrier that
+    // staging the columns in LDS used to need: with it their waves issue their
+    // gathers together (without: precision form on 128x128x64 6.02 -> 6.10 ms;
+    // the FP64 product by itself on 96x96x48 48.3 -> 49.3 us, and even on 12x11x5
+    // no faster).  The FP64 sweeps and the small FP32 ones are shorter without it
+    // (64x64x32 FP64 forward and backward 3.87 -> 3.80 ms).
     if constexpr (wide_tiles<MODE>() || (plain_small<TV>() && !PLAIN)) __syncthreads();
 
     // 4. x entries of the tile, one block (BS entries, one vector load) per
@@ -1295,7 +1312,7 @@ __device__ __attribute__((always_inline)) inline void stream_tile(const StreamAr
         if (!has_row[s]) continue;
         const TX o = from_double<TX>(res[s]);
         if constexpr (KEEP) keep[t] = o;
-        if constexpr (MODE == SM_SUB_SPMV) a.vout[gi[s]] = o;
+        if constexpr (MODE == SM_SUB_SPMV) static_cast<const SweepSpmvArgs<TV, TX> &>(a).vout[gi[s]] = o;
         else if constexpr (V != 1) {
             a.out[gi[s]] = o;
             if (a.out2) a.out2[gi[s]] = o;
@@ -1351,7 +1368,7 @@ __device__ inline void stream_rows_zero_x(const StreamArgs<TV, TX> &a, const int
 }
 
 template <int BS, int MODE, int RED, typename TV, typename TX, int ROWS = kTileRows, bool ZX = false, bool PLAIN = false>
-__global__ __launch_bounds__(64 * BS) void k_stream(StreamArgs<TV, TX> a) {
+__global__ __launch_bounds__(64 * BS) void k_stream(ArgsOf<MODE, ZX, TV, TX> a) {
     // the stop flag and the tile descriptor are loaded together (one scalar
     // round trip instead of two before the first vector load): the exit test
     // also reads the descriptor (a negative entry never occurs), so the
@@ -1685,6 +1702,9 @@ struct WaitArgs {
     int32_t rhs_split;
     int32_t last_row0;         // rows from here on: z = D^-1 (rhs - S1 y) (first sweep)
     TX *z;
+    TX *reset;                 // entries to mark as not written
+    int32_t *fail;             // a wait has run out; on the device, and for the host
+    int32_t *host_fail;
 };
 
 // v of the quad's lane C (DPP)
@@ -1764,11 +1784,11 @@ __global__ __launch_bounds__(kWaitThreads) void k_sweep_wait(StreamArgs<TV, TX> 
                         if ((spin & 255) == 0) {
                             const uint64_t now = wall_clock64();
                             if (since == 0) since = now;
-                            bool over = __hip_atomic_load(a.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+                            bool over = __hip_atomic_load(w.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
                             if (!over && now - since > kWaitTicks) {
                                 over = true;
-                                __hip_atomic_store(a.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                __hip_atomic_store(a.host_fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                                __hip_atomic_store(w.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                __hip_atomic_store(w.host_fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                             }
                             if (over) break;
                         }
@@ -1810,7 +1830,7 @@ __global__ __launch_bounds__(kWaitThreads) void k_sweep_wait(StreamArgs<TV, TX> 
             }
             if (k < nrow && (t & 3) < BS) {
                 store_entry(&(last ? w.z : a.out)[gi], from_double<TX>(res));
-                if (!last) mark_entry(&a.reset[gi]);
+                if (!last) mark_entry(&w.reset[gi]);
             }
         }
         if (t == 0) tk[p ^ 1] = next;

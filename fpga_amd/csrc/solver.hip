@@ -827,7 +827,7 @@ void launch_finalize(H &h, int nred, const RedArgs &ra, int nparts) {
 // half1: the ||s|| test that a sweep's launch takes along (k_stream_half1),
 // else null.
 template <int BS, int MODE, int RED, typename TV, typename TX, int ROWS = kTileRows, bool ZX = false, bool PLAIN = false>
-int stream_dispatch(H &h, const StreamArgs<TV, TX> &a, const FoldArgs *half1 = nullptr) {
+int stream_dispatch(H &h, const ArgsOf<MODE, ZX, TV, TX> &a, const FoldArgs *half1 = nullptr) {
     if constexpr (RED == SR_NONE && !ZX && (MODE == SM_SUB || MODE == SM_SUB_DINV || MODE == SM_SUB_Z)) {
         if (half1) {
             hipLaunchKernelGGL((k_stream_half1<BS, MODE, TV, TX, ROWS, PLAIN>), dim3(a.ntiles + 1), dim3(64 * BS), 0,
@@ -858,7 +858,7 @@ void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x
                    TX *out3 = nullptr, const TX *x_lo = nullptr, int split = 0, int prof_kind = -1,
                    const int32_t *rowptr2 = nullptr, TX *zout = nullptr, const FoldArgs *half1 = nullptr) {
     constexpr int nred = (RED & SR_W0 ? 1 : 0) + (RED & SR_SELF ? 1 : 0);
-    StreamArgs<TV, TX> a;
+    ArgsOf<MODE, ZX, TV, TX> a;
     constexpr bool wide = wide_tiles<MODE>();
     const std::vector<int32_t> &ct = wide ? m.colour_tile_wide : m.colour_tile;
     a.tile = colour < 0 ? (wide ? m.tile_wide_sp.p : m.tile_sp.p) : (wide ? m.tile_wide.p : m.tile.p);
@@ -909,7 +909,7 @@ void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x
     a.ra = ra;
     a.rowptr2 = rowptr2;
     a.zout = zout;
-    a.full = h.d_full.p;
+    if constexpr (ZX) a.full = h.d_full.p;
     if (!use_state) a.ra.st = h.st.p + kIdleState;
     if (MODE == SM_SUB_Z && (!rowptr2 || !zout || !dinv)) throw std::runtime_error("SUB_Z launch without z operands");
     if ((RED & SR_W0) && !w0) throw std::runtime_error("missing dot operand");
@@ -944,7 +944,7 @@ void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x
 template <int BS, int RED, typename TV, typename TX>
 void launch_sweep_spmv(H &h, const OpSet<TV> &op, const TX *rhs, TX *z, TX *v, const TX *w0, RedArgs ra) {
     const DevMat &m = *op.A;
-    StreamArgs<TV, TX> a;
+    SweepSpmvArgs<TV, TX> a;
     std::memset(&a, 0, sizeof(a));
     a.tile = m.tile_wide_sweep.p;
     a.slot = m.slot_wide.p;
@@ -1284,10 +1284,7 @@ void precond_wait(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si) 
     a.split = skip0 ? h.an.colour_ptr[1] : 0;
     a.rhs = p;
     a.out = y;
-    a.reset = z;
     a.dinv = op.dinv;
-    a.fail = h.d_sweep.p + 2;
-    a.host_fail = h.d_done + kSweepFail;
     a.ra = red(h, si, FIN_NONE);
     WaitArgs<TX> w;
     w.ticket = h.d_sweep.p;
@@ -1298,6 +1295,9 @@ void precond_wait(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si) 
     w.rhs_split = 0;
     w.last_row0 = h.an.colour_ptr[nc - 1];
     w.z = z;
+    w.reset = z;
+    w.fail = h.d_sweep.p + 2;
+    w.host_fail = h.d_done + kSweepFail;
     prof_begin(h, PK_LOWER);
     const dim3 g1(wait_grid(m1, c0, nc)), b(kWaitThreads);
     if (op.s1_dinv) hipLaunchKernelGGL((k_sweep_wait<BS, SM_SUB_DINV, TV, TX>), g1, b, 0, h.stream, a, w);
@@ -1313,7 +1313,7 @@ void precond_wait(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si) 
     a.split = 0;
     a.rhs = y;
     a.out = z;
-    a.reset = y;
+    w.reset = y;
     w.ticket = h.d_sweep.p + 1;
     w.other = h.d_sweep.p;
     w.ntiles = m2.colour_tile[nc - 1];
