@@ -26,6 +26,8 @@
 
 #include <type_traits>
 
+#include "wait_bound.hpp"
+
 #include "bda_host.hpp"  // kTileRows
 
 namespace bda {
@@ -812,10 +814,6 @@ template <typename T> __device__ inline void store_entry(T *p, T v) {
 template <typename T> __device__ inline void mark_entry(T *p) {
     *reinterpret_cast<typename NotYet<T>::Bits *>(p) = NotYet<T>::mark;
 }
-// Ticks of the wall clock (100 MHz) after which a wait is given up: 2 s, far
-// beyond any sweep.  Nothing waits that long (see k_sweep_wait); it bounds
-// the loop whatever happens.
-constexpr uint64_t kWaitTicks = 200000000;
 
 // Map workgroups to tiles so that each XCD (workgroups are dispatched to the
 // 8 XCDs round-robin) works on one contiguous range of tiles and the x
@@ -1777,15 +1775,15 @@ __global__ __launch_bounds__(kWaitThreads) void k_sweep_wait(StreamArgs<TV, TX> 
                     ready[j] = false;
                     free[j] = cb[j] < a.split;
                 }
-                uint64_t since = 0;
+                WaitCount count;
                 for (uint32_t spin = 0; !all; ++spin) {
                     if (spin > 0) {
                         __builtin_amdgcn_s_sleep(1);
-                        if ((spin & 255) == 0) {
-                            const uint64_t now = wall_clock64();
-                            if (since == 0) since = now;
+                        if ((spin & (kWaitLook - 1)) == 0) {
                             bool over = __hip_atomic_load(w.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-                            if (!over && now - since > kWaitTicks) {
+                            const int32_t tickets =
+                                __hip_atomic_load(w.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            if (!over && wait_over(count, tickets, kWaitPatience)) {
                                 over = true;
                                 __hip_atomic_store(w.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                                 __hip_atomic_store(w.host_fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
