@@ -95,6 +95,7 @@ SIGNATURES = {
     "bda_factor": (i32, [vp]),
     "bda_prepare_mixed": (i32, [vp]),
     "bda_set_options": (i32, [vp, f64, i32, i32]),
+    "bda_set_wait_limit": (i32, [vp, C.c_uint32]),
     "bda_solve": (i32, [vp, vp, vp, f64, i32, C.POINTER(BdaResult)]),
     "bda_solve_dev": (i32, [vp, vp, vp, f64, i32, C.POINTER(BdaResult)]),
     "bda_get_residual": (i32, [vp, vp]),

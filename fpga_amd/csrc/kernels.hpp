@@ -70,6 +70,7 @@ struct SolverState {
     uint64_t timeout_ticks;
     uint64_t deadline;
     int32_t aborted;
+    int32_t failed;         // a waiting sweep gave up: no result, the caller's x stays as it was
 };
 
 enum Fin : int32_t {
@@ -287,7 +288,8 @@ __device__ inline void refine_step(SolverState *out, const SolverState *in) {
         out->nan_flag = in->nan_flag;
     }
     if (in->aborted) out->aborted = 1;
-    if (in->no_results || in->aborted || ((in->breakdown || in->nan_flag) && in->h == 0 && in->last_half == 0))
+    if (in->failed) out->failed = 1;
+    if (in->no_results || in->aborted || in->failed || ((in->breakdown || in->nan_flag) && in->h == 0 && in->last_half == 0))
         signal_done(out);
 }
 
@@ -1701,8 +1703,8 @@ struct WaitArgs {
     int32_t last_row0;         // rows from here on: z = D^-1 (rhs - S1 y) (first sweep)
     TX *z;
     TX *reset;                 // entries to mark as not written
-    int32_t *fail;             // a wait has run out; on the device, and for the host
-    int32_t *host_fail;
+    int32_t *fail;             // a wait has run out
+    WaitLimit limit;
 };
 
 // v of the quad's lane C (DPP)
@@ -1718,6 +1720,14 @@ template <int BS, typename T> __device__ inline void quad_all(T v, T (&o)[BS]) {
     o[1] = quad_lane<1>(v);
     o[2] = quad_lane<2>(v);
     if constexpr (BS == 4) o[3] = quad_lane<3>(v);
+}
+
+// A wait has run out: the other waits end at their next look and the run stops
+// as failed, since what its sweeps have written is no preconditioner's output.
+__device__ inline void wait_failed(SolverState *st, int32_t *fail) {
+    __hip_atomic_store(fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    st->failed = 1;
+    signal_done(st);
 }
 
 constexpr int kWaitThreads = 256, kWaitBlocks = 4;  // rows of a tile * 4; blocks of a row at a time
@@ -1779,14 +1789,13 @@ __global__ __launch_bounds__(kWaitThreads) void k_sweep_wait(StreamArgs<TV, TX> 
                 for (uint32_t spin = 0; !all; ++spin) {
                     if (spin > 0) {
                         __builtin_amdgcn_s_sleep(1);
-                        if ((spin & (kWaitLook - 1)) == 0) {
+                        if ((spin & w.limit.mask) == 0) {
                             bool over = __hip_atomic_load(w.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
                             const int32_t tickets =
                                 __hip_atomic_load(w.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            if (!over && wait_over(count, tickets, kWaitPatience)) {
+                            if (!over && wait_over(count, tickets, w.limit.patience)) {
                                 over = true;
-                                __hip_atomic_store(w.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                                __hip_atomic_store(w.host_fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                                wait_failed(a.ra.st, w.fail);
                             }
                             if (over) break;
                         }
@@ -2167,7 +2176,8 @@ __global__ void k_scatter_rows(int n, int bs, const int32_t *perm, const double 
 }
 // End of a solve: x (finished with phat, when given) to the caller's order,
 // and the state to mapped host memory, so that the host waits once, for this
-// launch (an 8-byte copy and its wait took 21 us).
+// launch (an 8-byte copy and its wait took 21 us).  Out is left alone when the
+// run has failed.
 __global__ __launch_bounds__(256) void k_scatter_end(int n, int bs, const int32_t *perm, const double *x,
                                                      const double *phat, double *out, const SolverState *st,
                                                      SolverState *host) {
@@ -2176,9 +2186,10 @@ __global__ __launch_bounds__(256) void k_scatter_end(int n, int bs, const int32_
                            reinterpret_cast<const uint64_t *>(st)[threadIdx.x], __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_SYSTEM);
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)n * bs) return;
+    const int32_t failed = st->failed, half = st->last_half;  // (one round trip: half is never negative)
+    if (i >= (int64_t)n * bs || (failed | (half < 0 ? 1 : 0)) != 0) return;
     const int64_t k = i / bs, c = i - k * bs;
-    out[(int64_t)perm[k] * bs + c] = finished_x(x, phat, i, phat && st->last_half == 1, st->alpha);
+    out[(int64_t)perm[k] * bs + c] = finished_x(x, phat, i, phat && half == 1, st->alpha);
 }
 
 // dst block k = src block idx[k] (idx null: identity), optionally transposed

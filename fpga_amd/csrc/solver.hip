@@ -630,6 +630,7 @@ struct bda_handle_s {
     // bda_factor, not known of a caller's own (bda_upload_factored)
     bool u0_is_a = false;
     bool wait = BDA_WAIT != 0;    // sweeps of many levels in one launch each (k_sweep_wait)
+    bda::WaitLimit wait_limit;    // (bda_set_wait_limit)
     bool fold = BDA_FOLD != 0;    // scalar steps folded into the vector updates (small systems)
     bool fuse0 = BDA_FUSE0 != 0;  // the second sweep of colour 0 with the product's (SM_SUB_SPMV)
 
@@ -648,7 +649,7 @@ struct bda_handle_s {
     bda::SolverState *h_st = nullptr;  // pinned
     bda::SolverState *d_host_st = nullptr;  // its device address
     int32_t *h_done = nullptr;          // mapped host flags, one per state: the id of the run that stopped;
-                                        // then kBadRow and kSweepFail
+                                        // then kBadRow
     bda::DBuf<int32_t> d_sweep;         // waiting sweeps: two ticket counters, and whether a wait ran out
     int32_t *d_done = nullptr;          // their device address
     uint64_t *h_prog = nullptr;         // mapped progress words, one per state (run id << 32 | count)
@@ -783,7 +784,7 @@ void check_launch() { HIP_CHECK(hipGetLastError()); }
 // with folded scalar steps takes its state to kStateB after alpha and after
 // omega, and back to slot 0 after the ||s|| test and after beta.
 constexpr int kIdleState = 2, kStateB = 3, kStates = 4;
-constexpr int kBadRow = 2, kSweepFail = 3, kFlags = 4;  // places among the mapped flags
+constexpr int kBadRow = 2, kFlags = 3;  // places among the mapped flags
 
 RedArgs red(H &h, int state_idx, int fin) {
     RedArgs ra;
@@ -1297,7 +1298,7 @@ void precond_wait(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si) 
     w.z = z;
     w.reset = z;
     w.fail = h.d_sweep.p + 2;
-    w.host_fail = h.d_done + kSweepFail;
+    w.limit = h.wait_limit;
     prof_begin(h, PK_LOWER);
     const dim3 g1(wait_grid(m1, c0, nc)), b(kWaitThreads);
     if (op.s1_dinv) hipLaunchKernelGGL((k_sweep_wait<BS, SM_SUB_DINV, TV, TX>), g1, b, 0, h.stream, a, w);
@@ -1462,8 +1463,10 @@ void scatter_end(H &h, const double *x, const double *phat, double *d_x, const S
                        h.d_perm.p, x, phat, d_x, st, h.d_host_st);
     check_launch();
     HIP_CHECK(hipStreamSynchronize(h.stream));
-    if (__atomic_exchange_n(h.h_done + kSweepFail, 0, __ATOMIC_ACQ_REL) != 0)
-        throw std::runtime_error("a sweep's wait did not end");
+    if (h.h_st->failed) {
+        h.ev_used = 0;
+        throw std::runtime_error("a sweep's wait did not end: the solve was given up");
+    }
 }
 
 // One BiCGSTAB run following the reference microprogram (solver_pkg.vhd:120-141).
@@ -2626,6 +2629,10 @@ int bda_set_options(bda_handle h, double timeout_s, int32_t abs_tol, int32_t pol
         h->abs_tol = abs_tol != 0;
         h->poll_iters = poll_iters > 0 ? poll_iters : 1;
     });
+}
+
+int bda_set_wait_limit(bda_handle h, uint32_t polls) {
+    return guarded(h, [&] { h->wait_limit = polls ? bda::wait_limit(polls) : bda::WaitLimit{}; });
 }
 
 int bda_set_refinement(bda_handle h, int32_t adaptive, double eta) {

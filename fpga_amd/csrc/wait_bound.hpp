@@ -17,6 +17,18 @@ namespace bda {
 // polls, seconds in which no tile of the sweep was started.
 constexpr uint32_t kWaitLook = 256, kWaitPatience = 1u << 14;
 
+// Polls between two looks (less one) and equal looks to give up after, for a
+// limit in polls; a limit below kWaitLook looks after every poll.
+struct WaitLimit {
+    uint32_t mask = kWaitLook - 1, patience = kWaitPatience;
+};
+constexpr WaitLimit wait_limit(uint32_t polls) {
+    WaitLimit l;
+    l.mask = polls < kWaitLook ? 0 : kWaitLook - 1;
+    l.patience = polls < kWaitLook ? polls : polls / kWaitLook;
+    return l;
+}
+
 struct WaitCount {
     int32_t tickets = -1;  // at the last look
     uint32_t looks = 0;    // without a change

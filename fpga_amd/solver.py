@@ -268,6 +268,10 @@ class BicgstabSolver:
     def set_options(self, timeout_s: float = 0.0, abs_tol: bool = False, poll_iters: int = 1):
         self._check(lib.bda_set_options(self._h, timeout_s, int(abs_tol), poll_iters), "bda_set_options")
 
+    def set_wait_limit(self, polls: int = 0):
+        """Polls without progress after which a waiting sweep gives a solve up (0: the default)."""
+        self._check(lib.bda_set_wait_limit(self._h, polls), "bda_set_wait_limit")
+
     # -- solves (original ordering) ----------------------------------------
     def solve(self, b, x0=None, tol: float = 1e-6, maxit: int = 1000):
         b = _f64(b)

@@ -206,6 +206,15 @@ int bda_prepare_mixed(bda_handle h);
  * half-iterations are unfinished. */
 int bda_set_options(bda_handle h, double timeout_s, int32_t abs_tol, int32_t poll_iters);
 
+/* Where a solve runs the sweeps of many levels as two launches whose tiles
+ * wait for one another: the polls a tile makes, with no tile of the sweep
+ * started anywhere meanwhile, before the solve is given up with an error (x
+ * stays as it was); 0 = the default, 4 million (seconds without any progress).
+ * A bound against waiting for ever, which no healthy solve comes near; for
+ * callers with a bound of their own, and for tests of the error.  No
+ * counterpart in the reference. */
+int bda_set_wait_limit(bda_handle h, uint32_t polls);
+
 /* Plain FP64 ILU0-BiCGSTAB, the reference's microprogram
  * (solver_pkg.vhd:120-141): x holds x0 on entry and the solution on exit.
  * maxit follows the kernel's max_iter parameter: maxit full iterations are
