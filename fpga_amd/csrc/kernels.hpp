@@ -2331,10 +2331,10 @@ __global__ __launch_bounds__(256) void k_ilu0_updates(int64_t nnzb, const int32_
 // the tile's blocks are read once, in order, into LDS; lane (row, r) owns
 // component row r of every block of its row, so the whole elimination needs
 // no exchange between lanes; one lane per row inverts the diagonal block; and
-// L, U, D^-1, and the FP32 copies where the precision form is in use (the
-// float pointers, else null), are written from LDS, again in order.  On the
-// way it records non-finite values of A and copies colour 0's diagonal
-// blocks (adiag).  One thread per row instead, in place on a copy of A that
+// L, U, D^-1, and the FP32 copies where those of the factorisation before
+// were asked for (the float pointers, else null), are written from LDS, again
+// in order.  On the way it records non-finite values of A and copies colour
+// 0's diagonal blocks (adiag).  One thread per row instead, in place on a copy of A that
 // was gathered into L and U afterwards, read and wrote each 72- or 128-byte
 // block from one lane (64 cache lines per load) with a chain of dependent
 // loads per block: on a 128x128x64 3x3 grid copy 147 us, elimination 766,

@@ -615,10 +615,10 @@ struct bda_handle_s {
     bda::DBuf<double> low2_v64;  // values of L's packed dependency rows (k_lower2)
     bda::DBuf<float> low2_v32;
     bda::DBuf<float> At32, Ut32, Lt32;  // FP32 transposes (component access only)
-    // the precision form has been used: the factorisation then writes its FP32
-    // copies beside the FP64 values (copies_gen: the factorisation whose
-    // values they hold; mixed_gen: the one they were last asked for)
-    bool mixed_used = false;
+    // The precision form's FP32 copies: a factorisation writes them beside the
+    // FP64 values if those of the one before were asked for (copies_gen: the
+    // factorisation whose values they hold; mixed_gen: the one they were last
+    // asked for), else the first call that needs them makes them
     uint64_t copies_gen = UINT64_MAX;
     uint64_t factor_gen = 0, mixed_gen = UINT64_MAX, adj_gen = UINT64_MAX, adj32_gen = UINT64_MAX;
     uint64_t values_gen = 0;  // changes with every upload, value update and factorisation
@@ -1820,7 +1820,7 @@ void do_factor(H &h) {
     constexpr int BB = BS * BS;
     const Analysis &an = h.an;
     const auto t0 = std::chrono::steady_clock::now();
-    const bool f32 = h.mixed_used;
+    const bool f32 = h.mixed_gen == h.factor_gen;
     if (f32) mixed_buffers<BS>(h);
     if (an.ncolours > 1) h.A0d64.ensure((size_t)an.colour_ptr[1] * BB);
     IluArgs<BS> a;
@@ -1896,7 +1896,6 @@ template <int BS>
 void ensure_mixed(H &h) {
     require_factored(h);
     if (h.mixed_gen == h.factor_gen) return;
-    h.mixed_used = true;
     if (h.copies_gen == h.factor_gen) {  // written by the factorisation
         h.mixed_gen = h.factor_gen;
         return;
