@@ -1820,6 +1820,7 @@ void do_factor(H &h) {
     constexpr int BB = BS * BS;
     const Analysis &an = h.an;
     const auto t0 = std::chrono::steady_clock::now();
+    h.factored = false;  // until it succeeds: the factors are written in place
     const bool f32 = h.mixed_gen == h.factor_gen;
     if (f32) mixed_buffers<BS>(h);
     if (an.ncolours > 1) h.A0d64.ensure((size_t)an.colour_ptr[1] * BB);
