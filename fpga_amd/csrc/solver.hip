@@ -992,6 +992,12 @@ void launch_stream_timed(H &h, const TV *val, const TX *x, TX *y, const TX *w0, 
 
 int vec_blocks(size_t N) { return (int)((N + kVecElemsPerBlock - 1) / kVecElemsPerBlock); }
 
+// The ||s|| test of a folded run as a launch of its own.
+void fold_half1(H &h, const FoldArgs &f) {
+    hipLaunchKernelGGL(k_fold_half1, dim3(1), dim3(kVecThreads), 0, h.stream, f);
+    check_launch();
+}
+
 template <int BS, typename TV, typename TX>
 void sweep_launch(H &h, const DevMat &m, const TV *val, int c, bool dinv_mode, const TX *x, const TX *x_lo, int split,
                   const TX *rhs, TX *out, const double *dinv, int si, const FoldArgs *half1 = nullptr) {
@@ -1223,11 +1229,8 @@ void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si, bool 
         half1 = nullptr;
         return f;
     };
+    if (half1 && ((low2 && nc == 4) || half1->vn > kFinThreads)) fold_half1(h, *take_half1());
     prof_begin(h, PK_LOWER);
-    if (half1 && (h.profiling || (low2 && nc == 4) || half1->vn > kFinThreads)) {
-        hipLaunchKernelGGL(k_fold_half1, dim3(1), dim3(kVecThreads), 0, h.stream, *take_half1());
-        check_launch();
-    }
     for (int c = skip0 ? 1 : 0; c < nc - 1; ++c) {
         if (low2 && c == nc - 3) {
             lower2_launch<BS, TV, TX>(h, op, low2_values<TV>(h), p, y, lo, split, merge3 ? z : nullptr, si);
@@ -1544,15 +1547,8 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     // (half1: the ||s|| test of a folded run, still to be made)
     auto apply = [&](auto redc, const TX *p, TX *z, TX *v, const TX *w0, const FoldArgs *half1) {
         constexpr int RED = decltype(redc)::value;
-        if (wait) {
-            if (half1) {
-                hipLaunchKernelGGL(k_fold_half1, dim3(1), dim3(kVecThreads), 0, h.stream, *half1);
-                check_launch();
-            }
-            precond_wait<BS, TV, TX>(h, op, p, k.y.p, z, 0);
-        } else {
-            precond<BS, TV, TX>(h, op, p, k.y.p, z, 0, fuse, half1);
-        }
+        if (wait) precond_wait<BS, TV, TX>(h, op, p, k.y.p, z, 0);
+        else precond<BS, TV, TX>(h, op, p, k.y.p, z, 0, fuse, half1);
         if (fuse) {
             prof_begin(h, PK_UPPER);
             launch_sweep_spmv<BS, RED, TV, TX>(h, op, p, z, v, w0, red(h, 0, FIN_NONE));
@@ -1584,7 +1580,11 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
         }
     };
     const dim3 vg(vb), vt(kVecThreads);
+    // no sweep takes the ||s|| test along: the waiting ones cannot, and while
+    // launches are timed it counts with the vector updates
+    const bool half1_alone = fold && (wait || h.profiling);
     for (int it = 1; it <= maxit + 1 && !stop; ++it) {
+        const FoldArgs half1 = fold_args(kStateB, 0, spart);
         h.prof_tag = 2 * (it - 1);
         apply(red_w0, k.p.p, k.phat.p, k.v.p, k.rt.p, nullptr);
         throttle(2 * it - 1);
@@ -1595,6 +1595,7 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
             hipLaunchKernelGGL((k_update_s<TX, true>), vg, vt, 0, h.stream, (int64_t)N, k.r.p, k.v.p, k.s.p,
                                vec_red(FIN_NONE, spart), fold_args(0, kStateB, nullptr));
             check_launch();
+            if (half1_alone) fold_half1(h, half1);
         } else {
             hipLaunchKernelGGL((k_update_s<TX, false>), vg, vt, 0, h.stream, (int64_t)N, k.r.p, k.v.p, k.s.p,
                                red(h, 0, FIN_HALF1), FoldArgs{});
@@ -1603,8 +1604,7 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
         }
         prof_end(h);
         h.prof_tag = 2 * (it - 1) + 1;
-        const FoldArgs half1 = fold_args(kStateB, 0, spart);
-        apply(red_both, k.s.p, k.shat.p, k.t.p, k.s.p, fold ? &half1 : nullptr);
+        apply(red_both, k.s.p, k.shat.p, k.t.p, k.s.p, fold && !half1_alone ? &half1 : nullptr);
         throttle(2 * it);
         if (stop) break;
         product(red_both, k.shat.p, k.t.p, k.s.p, FIN_OMEGA);
