@@ -154,6 +154,7 @@ def main():
     n_low, ms_low = g.kernel_stats(fa.KIND_LOWER)
     n_up, ms_up = g.kernel_stats(fa.KIND_UPPER)
     n_vec, ms_vec = g.kernel_stats(fa.KIND_VEC)
+    merged64 = merged_sweeps(g, fa)
     g.set_profiling(False)
 
     torch.cuda.synchronize()
@@ -170,6 +171,7 @@ def main():
     g.set_profiling(True)
     run_mixed()
     spmv32_in = in_solve_avg(g.kernel_times(fa.KIND_SPMV))
+    merged32 = merged_sweeps(g, fa)
     g.set_profiling(False)
 
     spmv_bytes = g.algorithmic_bytes(fa.KIND_SPMV)
@@ -194,16 +196,9 @@ def main():
         t = json.loads(tfile.read_text())
         if "fp32" in t:
             traffic = t["fp32"]["read_bytes"] + t["fp32"]["write_bytes"]
-    low_bytes, up_bytes = g.algorithmic_bytes(fa.KIND_LOWER), g.algorithmic_bytes(fa.KIND_UPPER)
     iters64 = r64.iterations
-    # algorithmic bytes per FP64 iteration: 2 SpMV + 2 (L + U) + 22 N vector passes,
-    # each as a pass of its own (a merged sweep and product reads colour 0's
-    # blocks once for both, so the rate counts them twice)
-    it_bytes = 2 * spmv_bytes + 2 * (low_bytes + up_bytes) + 22 * s.N * 8
-    solve_gbs = it_bytes * iters64 / t_fp64 / 1e9
-    mixed_it_bytes = (2 * g.algorithmic_bytes(fa.KIND_SPMV, True)
-                      + 2 * (g.algorithmic_bytes(fa.KIND_LOWER, True) + g.algorithmic_bytes(fa.KIND_UPPER, True))
-                      + 22 * s.N * 4)
+    solve_gbs = iteration_bytes(g, fa, s, False, merged64) * iters64 / t_fp64 / 1e9
+    mixed_it_bytes = iteration_bytes(g, fa, s, True, merged32)
     # one preconditioner application (L then U sweep) back to back, both forms
     trisolve = {}
     for fp32 in (False, True):
@@ -274,13 +269,27 @@ def main():
     return 0
 
 
-def iteration_bytes(g, fa, s, fp32):
+def merged_sweeps(g, fa):
+    """Whether the profiled solve ran colour 0's upper sweep and the product of
+    its rows as one launch: there are two upper-sweep brackets per lower one
+    then (profiling is on; call before it is switched off)."""
+    return g.kernel_stats(fa.KIND_UPPER)[0] >= 2 * g.kernel_stats(fa.KIND_LOWER)[0] > 0
+
+
+def iteration_bytes(g, fa, s, fp32, merged):
     """Algorithmic bytes of one BiCGSTAB iteration: 2 SpMV + 2 (L + U) + 22 N
-    vector element passes (the same for the transposed operators)."""
-    sx = 4 if fp32 else 8
-    return (2 * g.algorithmic_bytes(fa.KIND_SPMV, fp32)
-            + 2 * (g.algorithmic_bytes(fa.KIND_LOWER, fp32) + g.algorithmic_bytes(fa.KIND_UPPER, fp32))
-            + 22 * s.N * sx)
+    vector element passes (the same for the transposed operators).  merged: the
+    blocks that colour 0's rows of U share with A (all but the diagonal) are
+    read once for both passes, in each half-iteration."""
+    sv = sx = 4 if fp32 else 8
+    by = (2 * g.algorithmic_bytes(fa.KIND_SPMV, fp32)
+          + 2 * (g.algorithmic_bytes(fa.KIND_LOWER, fp32) + g.algorithmic_bytes(fa.KIND_UPPER, fp32))
+          + 22 * s.N * sx)
+    if merged:
+        _, perm, cptr = g.colouring()
+        shared = int((np.diff(s.rowptr)[perm[:cptr[1]]] - 1).sum())
+        by -= 2 * shared * (s.bs * s.bs * sv + 4)
+    return by
 
 
 def grad_bytes(s):
@@ -381,7 +390,7 @@ def adjoint_block(fa, torch, dev, steps):
         torch.cuda.synchronize()
         times.append(time.perf_counter() - t0)
     t = float(np.median(times))
-    by = iteration_bytes(g, fa, s, False) * ra.iterations + grad_bytes(s)
+    by = iteration_bytes(g, fa, s, False, False) * ra.iterations + grad_bytes(s)
     lam_ref = lam.clone()
     nref = torch.linalg.vector_norm(lam_ref).item()
     g.adjoint_solve_mixed_dev(w.data_ptr(), lam.data_ptr(), 1e-10)   # builds the FP32 transposes
@@ -439,6 +448,16 @@ def big_block(fa, torch, dev, steps):
     e64 = torch.linalg.vector_norm(x - x_ref).item() / nref
     tmx, rmx = timed(lambda: g.solve_mixed_dev(b.data_ptr(), x.data_ptr(), 1e-6, 20, 1e-4, 1000, True))
     emx = torch.linalg.vector_norm(x - x_ref).item() / nref
+    # the bytes of an iteration of each: one more solve, untimed, to see its launches
+    it_adj, it_fwd = iteration_bytes(g, fa, s, False, False), []
+    for fp32, run in ((False, lambda: g.solve_dev(b.data_ptr(), x.data_ptr(), 1e-6, 1000)),
+                      (True, lambda: g.solve_mixed_dev(b.data_ptr(), x.data_ptr(), 1e-6, 20, 1e-4, 1000, True))):
+        x.zero_()
+        g.set_profiling(True)
+        run()
+        merged = merged_sweeps(g, fa)
+        g.set_profiling(False)
+        it_fwd.append(iteration_bytes(g, fa, s, fp32, merged))
     w = torch.from_numpy(np.random.default_rng(0).standard_normal(s.N)).to(dev)
     lam = torch.zeros_like(w)
     grad = torch.empty((s.nnzb, s.bs, s.bs), dtype=torch.float64, device=dev)
@@ -461,16 +480,15 @@ def big_block(fa, torch, dev, steps):
 
     tam, ram = timed(adj_mixed)
     eam = torch.linalg.vector_norm(lam - lam_ref).item() / nlam
-    it64, it32 = iteration_bytes(g, fa, s, False), iteration_bytes(g, fa, s, True)
     out = {"workload": "grid256x256x64", "block": s.bs, "block_rows": s.n, "blocks": s.nnzb, "unknowns": s.N,
            "colours": g.num_colours, "setup_s": st, "steps": steps,
            "fp64": {"time_s": t64, "iterations": r64.iterations, "x_rel_err_vs_1e-10": e64,
-                    "GBs_algorithmic": it64 * r64.iterations / t64 / 1e9},
+                    "GBs_algorithmic": it_fwd[0] * r64.iterations / t64 / 1e9},
            "mixed": {"time_s": tmx, "outer": rmx.outer_iterations, "inner_iterations": rmx.iterations,
                      "x_rel_err_vs_1e-10": emx, "speedup_vs_fp64": t64 / tmx,
-                     "GBs_algorithmic_approx": it32 * rmx.iterations / tmx / 1e9},
+                     "GBs_algorithmic_approx": it_fwd[1] * rmx.iterations / tmx / 1e9},
            "adjoint": {"time_s": tad, "tol": 1e-10, "iterations": rad.iterations, "converged": rad.converged,
-                       "GBs_algorithmic": (it64 * rad.iterations + grad_bytes(s)) / tad / 1e9},
+                       "GBs_algorithmic": (it_adj * rad.iterations + grad_bytes(s)) / tad / 1e9},
            "adjoint_mixed": {"time_s": tam, "tol": 1e-10, "outer": ram.outer_iterations,
                              "inner_iterations": ram.iterations, "converged": ram.converged,
                              "lambda_rel_diff_vs_fp64": eam, "speedup_vs_fp64_adjoint": tad / tam}}
