@@ -574,7 +574,7 @@ constexpr int kVecThreads = 256;
 struct FoldArgs {
     const double *part;      // the product's partials: reduction j at part + j * cap
     int32_t cap, n;
-    const double *vpart;     // those of the vector update before it
+    const double *vpart;     // those of the vector update before it (at most kFinThreads)
     int32_t vcap, vn;
     const SolverState *in;
     SolverState *out;
@@ -627,12 +627,13 @@ __device__ inline void fold_waves(const double *part, int cap, int n, double (*s
         }
     }
 }
-// the wave sums of NRED reductions over n <= kFoldMax partials, for fold_total
-// after a barrier
-template <int NRED, int NT = kVecThreads>
+// the wave sums of NRED reductions over the product's n <= kFoldMax partials,
+// for fold_total after a barrier (a vector update's are at most kFinThreads
+// then, see the rule: one load per thread)
+template <int NRED>
 __device__ inline void fold_sums(const double *part, int cap, int n, double (*sred)[2]) {
-    if (n <= kFinThreads) fold_waves<NRED, 1, NT>(part, cap, n, sred);
-    else fold_waves<NRED, kFoldStep, NT>(part, cap, n, sred);
+    if (n <= kFinThreads) fold_waves<NRED, 1, kVecThreads>(part, cap, n, sred);
+    else fold_waves<NRED, kFoldStep, kVecThreads>(part, cap, n, sred);
 }
 __device__ inline double fold_total(const double (*sred)[2], int j) {
     double t = sred[0][j];
@@ -666,22 +667,20 @@ __device__ inline void fold_store(const FoldArgs &f, const SolverState *ss, int 
 // its first half only after the second half's product: 2% faster over 20
 // iterations, 2-8% slower over 2 to 5.  It is a launch of its own, or, where
 // the second half's first launch is a k_stream, an extra workgroup of that
-// (k_stream_half1): nothing in that sweep needs its result.  FEW: at most
-// kFinThreads partials.
-template <int NT, bool FEW>
+// (k_stream_half1): nothing in that sweep needs its result.
+template <int NT>
 __device__ inline void half1_step(const FoldArgs &f) {
     __shared__ SolverState ss;
     __shared__ double sred[kFinThreads / 64][2];
     if (threadIdx.x < kStateWords)
         reinterpret_cast<uint64_t *>(&ss)[threadIdx.x] = reinterpret_cast<const uint64_t *>(f.in)[threadIdx.x];
-    if constexpr (FEW) fold_waves<1, 1, NT>(f.vpart, f.vcap, f.vn, sred);
-    else fold_sums<1, NT>(f.vpart, f.vcap, f.vn, sred);
+    fold_waves<1, 1, NT>(f.vpart, f.vcap, f.vn, sred);
     __syncthreads();
     if (threadIdx.x == 0 && !ss.done) scalar_step(&ss, FIN_HALF1, fold_total(sred, 0), 0.0, true);
     __syncthreads();
     fold_store(f, &ss, 0);
 }
-__global__ __launch_bounds__(kVecThreads) void k_fold_half1(FoldArgs f) { half1_step<kVecThreads, false>(f); }
+__global__ __launch_bounds__(kVecThreads) void k_fold_half1(FoldArgs f) { half1_step<kVecThreads>(f); }
 
 // *nonfinite = id when one of n values is infinite or NaN (id: the
 // factorisation's own, so that the flag never has to be cleared).  Every
@@ -1396,7 +1395,7 @@ __global__ __launch_bounds__(64 * BS) void k_stream(ArgsOf<MODE, ZX, TV, TX> a) 
 template <int BS, int MODE, typename TV, typename TX, int ROWS, bool PLAIN>
 __global__ __launch_bounds__(64 * BS) void k_stream_half1(StreamArgs<TV, TX> a, FoldArgs f) {
     if (blockIdx.x == 0) {
-        half1_step<64 * BS, true>(f);
+        half1_step<64 * BS>(f);
         return;
     }
     const int4 d = a.tile[a.tile0 + xcd_tile(blockIdx.x - 1, a.ntiles)];
@@ -2032,7 +2031,7 @@ __global__ __launch_bounds__(kVecThreads) void k_update_p(int64_t N, TX *p, cons
         __shared__ int late;
         if (threadIdx.x < kStateWords)
             reinterpret_cast<uint64_t *>(&ss)[threadIdx.x] = reinterpret_cast<const uint64_t *>(f.in)[threadIdx.x];
-        fold_sums<2>(f.vpart, f.vcap, f.vn, sred);
+        fold_waves<2, 1, kVecThreads>(f.vpart, f.vcap, f.vn, sred);
         __syncthreads();
         if (threadIdx.x == 0) {
             if (!ss.done) scalar_step(&ss, FIN_HALF2, fold_total(sred, 0), fold_total(sred, 1), blockIdx.x == 0);

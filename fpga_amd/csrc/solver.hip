@@ -1222,14 +1222,13 @@ void precond(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si, bool 
     // (with three colours the extended tail would cover colour 0)
     const bool merge3 = merge && h.tail3 && !op.s1_dinv && op.s2_dinv && op.S2->tail3_n >= 0 && !(skip_last && nc == 3);
     const bool low2 = h.low2 && skip0 && op.S1->low2_n >= 0 && nc >= 4 && op.S1 == &h.L;
-    // the first launch takes the ||s|| test along, unless it is k_lower2 (or
-    // has more partials to add up than the test in passing does)
+    // the first launch takes the ||s|| test along, unless it is k_lower2
     auto take_half1 = [&] {
         const FoldArgs *f = half1;
         half1 = nullptr;
         return f;
     };
-    if (half1 && ((low2 && nc == 4) || half1->vn > kFinThreads)) fold_half1(h, *take_half1());
+    if (half1 && low2 && nc == 4) fold_half1(h, *take_half1());
     prof_begin(h, PK_LOWER);
     for (int c = skip0 ? 1 : 0; c < nc - 1; ++c) {
         if (low2 && c == nc - 3) {
@@ -1529,7 +1528,9 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
         check_launch();
     }
     const int nparts = op.A->ntiles_wide;  // of the product
-    const bool fold = h.fold && nparts <= kFoldMax && vb <= kFoldMax;
+    const bool fold = h.fold && nparts <= kFoldMax;
+    static_assert((int64_t)kFoldMax * kTileRows * 4 <= (int64_t)kFinThreads * kVecElemsPerBlock,
+                  "folded runs: the vector updates' partials are one load per thread");
     auto fin_of = [&](int fin) { return fold ? (int)FIN_NONE : fin; };
     auto fold_args = [&](int in, int out, const double *vpart) {
         return FoldArgs{h.partials.p, h.partial_cap, nparts, vpart, vb, vb, h.st.p + in, h.st.p + out};
