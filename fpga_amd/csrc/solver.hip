@@ -603,10 +603,8 @@ struct bda_handle_s {
 
     // device matrices
     bda::DevMat A, L, U, At, Ut, Lt;
-    bda::DBuf<int32_t> d_perm, d_blkrow, d_bad;
+    bda::DBuf<int32_t> d_perm, d_blkrow;
     bda::DBuf<int32_t> d_upd;  // what each L block updates in the factorisation (k_ilu0_updates)
-    bda::DBuf<int32_t> d_nonfinite;  // the last factorisation (factor_id) that met an infinite or NaN value
-    bda::DBuf<int32_t> d_full;       // the last run (its id) whose step-0 residual needs the product
     int32_t factor_id = 0;
     bda::DBuf<double> d_orig, A64, L64, U64, LU, Dinv, DinvT, At64, Ut64, Lt64;
     bda::DBuf<float> A32, L32, U32;
@@ -643,14 +641,14 @@ struct bda_handle_s {
 
     // reductions and scalar state (0 = solve, 1 = outer loop or auxiliary, 2 = idle)
     bda::DBuf<double> partials;
-    bda::DBuf<double> vparts;  // folded runs: those of k_update_s, then the two of k_update_xr
+    double *vparts = nullptr;  // behind them, for folded runs: those of k_update_s, then the two of k_update_xr
     int32_t partial_cap = 0;
     bda::DBuf<bda::SolverState> st;
     bda::SolverState *h_st = nullptr;  // pinned
     bda::SolverState *d_host_st = nullptr;  // its device address
     int32_t *h_done = nullptr;          // mapped host flags, one per state: the id of the run that stopped;
                                         // then kBadRow
-    bda::DBuf<int32_t> d_sweep;         // waiting sweeps: two ticket counters, and whether a wait ran out
+    bda::DBuf<int32_t> d_words;         // single words (Word)
     int32_t *d_done = nullptr;          // their device address
     uint64_t *h_prog = nullptr;         // mapped progress words, one per state (run id << 32 | count)
     uint64_t *d_prog = nullptr;
@@ -786,6 +784,17 @@ void check_launch() { HIP_CHECK(hipGetLastError()); }
 constexpr int kIdleState = 2, kStateB = 3, kStates = 4;
 constexpr int kBadRow = 2, kFlags = 3;  // places among the mapped flags
 
+// Places in the handle's array of single words (one allocation, made with the
+// handle: an allocation and its zero fill take 10 us or more each).
+enum Word : int {
+    WD_TICKET = 0,     // waiting sweeps: two ticket counters, and whether a wait ran out (k_sweep_reset)
+    WD_FAIL = 2,
+    WD_BAD = 3,        // a factorisation's first bad row
+    WD_NONFINITE = 4,  // the last factorisation (factor_id) that met an infinite or NaN value
+    WD_FULL = 5,       // the last run (its id) whose step-0 residual needs the product
+    WD_N = 6
+};
+
 RedArgs red(H &h, int state_idx, int fin) {
     RedArgs ra;
     ra.partials = h.partials.p;
@@ -847,7 +856,7 @@ int stream_dispatch(H &h, const ArgsOf<MODE, ZX, TV, TX> &a, const FoldArgs *hal
 // prof_kind >= 0: with profiling on, the streaming kernel alone (not its
 // finalize) is bracketed by an event pair of that kind.
 // ZX: a step-0 residual that takes the short path unless k_gather_start left
-// the run's id in h.d_full (zero start vector, finite matrix).
+// the run's id in WD_FULL (zero start vector, finite matrix).
 // colour kRestOfRows (the product only): every colour but the first, whose
 // rows' partial sums launch_sweep_spmv has left in their slots.
 constexpr int kRestOfRows = -2;
@@ -910,7 +919,7 @@ void launch_stream(H &h, const DevMat &m, const TV *val, int colour, const TX *x
     a.ra = ra;
     a.rowptr2 = rowptr2;
     a.zout = zout;
-    if constexpr (ZX) a.full = h.d_full.p;
+    if constexpr (ZX) a.full = h.d_words.p + WD_FULL;
     if (!use_state) a.ra.st = h.st.p + kIdleState;
     if (MODE == SM_SUB_Z && (!rowptr2 || !zout || !dinv)) throw std::runtime_error("SUB_Z launch without z operands");
     if ((RED & SR_W0) && !w0) throw std::runtime_error("missing dot operand");
@@ -1290,8 +1299,8 @@ void precond_wait(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si) 
     a.dinv = op.dinv;
     a.ra = red(h, si, FIN_NONE);
     WaitArgs<TX> w;
-    w.ticket = h.d_sweep.p;
-    w.other = h.d_sweep.p + 1;
+    w.ticket = h.d_words.p + WD_TICKET;
+    w.other = h.d_words.p + WD_TICKET + 1;
     w.ntiles = m1.colour_tile[nc] - m1.colour_tile[c0];
     w.reverse = 0;
     w.rhs_lo = nullptr;
@@ -1299,7 +1308,7 @@ void precond_wait(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si) 
     w.last_row0 = h.an.colour_ptr[nc - 1];
     w.z = z;
     w.reset = z;
-    w.fail = h.d_sweep.p + 2;
+    w.fail = h.d_words.p + WD_FAIL;
     w.limit = h.wait_limit;
     prof_begin(h, PK_LOWER);
     const dim3 g1(wait_grid(m1, c0, nc)), b(kWaitThreads);
@@ -1317,8 +1326,8 @@ void precond_wait(H &h, const OpSet<TV> &op, const TX *p, TX *y, TX *z, int si) 
     a.rhs = y;
     a.out = z;
     w.reset = y;
-    w.ticket = h.d_sweep.p + 1;
-    w.other = h.d_sweep.p;
+    w.ticket = h.d_words.p + WD_TICKET + 1;
+    w.other = h.d_words.p + WD_TICKET;
     w.ntiles = m2.colour_tile[nc - 1];
     w.reverse = 1;
     w.rhs_lo = p;
@@ -1361,10 +1370,14 @@ int precond_launches(const H &h, const OpSet<TV> &op) {
 // (1365), 192 / 173 (2666); 4x4: 71.4 / 71.5, 95.9 / 93.7, 150.7 / 136.9,
 // 248 / 213.
 constexpr int kFuseFrom = 640;
+// what the ordering decides of it: only then are the merged launch's tile
+// lists and diagonal blocks made
+bool fuse_ordered(const H &h) {
+    return h.fuse0 && h.an.ncolours > 1 && h.an.A.colour_tile_wide[1] >= kFuseFrom;
+}
 template <typename TV>
 bool fuse_sweep_spmv(const H &h, const OpSet<TV> &op) {
-    return h.fuse0 && h.u0_is_a && op.A == &h.A && op.S2 == &h.U && !op.s1_dinv && op.s2_dinv && h.an.ncolours > 1 &&
-           op.A->colour_tile_wide[1] >= kFuseFrom;
+    return h.u0_is_a && op.A == &h.A && op.S2 == &h.U && !op.s1_dinv && op.s2_dinv && fuse_ordered(h);
 }
 
 // Whether a solve runs its sweeps as two launches whose tiles wait for one
@@ -1455,7 +1468,7 @@ int32_t init_state(H &h, int idx, double tol, int maxit, bool abs_mode) {
 void gather_start(H &h, const double *d_b, double *bp, const double *d_x, double *xp, SolverState *st,
                   const SolverState &start) {
     hipLaunchKernelGGL(k_gather_start, dim3(blocks_for((int64_t)h.N(), 256)), dim3(256), 0, h.stream, h.n, h.bs,
-                       h.d_perm.p, d_b, bp, d_x, xp, (const int32_t *)h.d_nonfinite.p, h.factor_id, h.d_full.p, st,
+                       h.d_perm.p, d_b, bp, d_x, xp, (const int32_t *)(h.d_words.p + WD_NONFINITE), h.factor_id, h.d_words.p + WD_FULL, st,
                        start);
     check_launch();
 }
@@ -1524,7 +1537,7 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
     const bool fuse = !wait && fuse_sweep_spmv(h, op);
     if (wait) {
         hipLaunchKernelGGL((k_sweep_reset<TX>), dim3(blocks_for((int64_t)std::max<size_t>(N, 3), 256)), dim3(256), 0,
-                           h.stream, (int64_t)N, k.y.p, h.d_sweep.p);
+                           h.stream, (int64_t)N, k.y.p, h.d_words.p + WD_TICKET);
         check_launch();
     }
     const int nparts = op.A->ntiles_wide;  // of the product
@@ -1543,7 +1556,7 @@ RunOut run_bicgstab(H &h, const OpSet<TV> &op, Krylov<TX> &k, const double *rhs,
         }
         return ra;
     };
-    double *spart = h.vparts.p, *xrpart = h.vparts.p + vb;
+    double *spart = h.vparts, *xrpart = h.vparts + vb;
     // z = M^-1 p, and, fused, the colour-0 rows of v = A z with their dots
     // (half1: the ||s|| test of a folded run, still to be made)
     auto apply = [&](auto redc, const TX *p, TX *z, TX *v, const TX *w0, const FoldArgs *half1) {
@@ -1725,7 +1738,7 @@ void finish_analyse(H &h) {
         else restore_values<4>(h);
     }
     const int64_t span = DevMat::coupling_span(an.A, an.perm);
-    h.A.upload(an.A, h.stream, &an.perm, span, &an.U);
+    h.A.upload(an.A, h.stream, &an.perm, span, fuse_ordered(h) ? &an.U : nullptr);
     h.L.upload(an.L, h.stream, &an.perm, span);
     h.U.upload(an.U, h.stream, &an.perm, span);
     h.At.upload(an.At, h.stream, &an.perm, span);
@@ -1754,17 +1767,14 @@ void finish_analyse(H &h) {
     h.L64.ensure((an.L.nnzb() + kPadBlocks) * bb);
     h.U64.ensure((an.U.nnzb() + kPadBlocks) * bb);
     h.Dinv.ensure((size_t)h.n * bb);
-    h.d_bad.ensure(1);
-    h.d_nonfinite.ensure(1);
-    h.d_full.ensure(1);
-    hipLaunchKernelGGL(k_factor_end, dim3(1), dim3(1), 0, h.stream, h.d_bad.p, (int32_t *)nullptr);
+    hipLaunchKernelGGL(k_factor_end, dim3(1), dim3(1), 0, h.stream, h.d_words.p + WD_BAD, (int32_t *)nullptr);
     check_launch();
     // reduction partials: one slot pair per workgroup of the largest reducing
     // launch, and room for the first stage of a two-stage sum
     const int cap = std::max({h.A.ntiles, h.At.ntiles, vec_blocks(h.N()), 1}) + kFinGroups;
     h.partial_cap = cap;
-    h.partials.ensure((size_t)2 * cap);
-    h.vparts.ensure((size_t)3 * vec_blocks(h.N()));
+    h.partials.ensure((size_t)2 * cap + (size_t)3 * vec_blocks(h.N()));
+    h.vparts = h.partials.p + (size_t)2 * cap;
     h.k64.ensure(h.Npad());
     h.bp.ensure(h.Npad());
     h.xo.ensure(h.Npad());
@@ -1797,7 +1807,7 @@ void mixed_buffers(H &h) {
     h.A32.ensure((h.A.nnzb + kPadBlocks) * bb);
     h.L32.ensure((h.L.nnzb + kPadBlocks) * bb);
     h.U32.ensure((h.U.nnzb + kPadBlocks) * bb);
-    if (h.an.ncolours > 1) h.A0d32.ensure((size_t)h.an.colour_ptr[1] * bb);
+    if (fuse_ordered(h)) h.A0d32.ensure((size_t)h.an.colour_ptr[1] * bb);
     if (h.L.low2_n >= 0) h.low2_v32.ensure((h.L.low2_nvblk + kPadBlocks) * bb);
 }
 template <int BS>
@@ -1824,7 +1834,7 @@ void do_factor(H &h) {
     h.factored = false;  // until it succeeds: the factors are written in place
     const bool f32 = h.mixed_gen == h.factor_gen;
     if (f32) mixed_buffers<BS>(h);
-    if (an.ncolours > 1) h.A0d64.ensure((size_t)an.colour_ptr[1] * BB);
+    if (fuse_ordered(h)) h.A0d64.ensure((size_t)an.colour_ptr[1] * BB);
     IluArgs<BS> a;
     a.tile = h.A.tile_wide.p;
     a.rowptr = h.A.rowptr.p;
@@ -1840,20 +1850,20 @@ void do_factor(H &h) {
     a.a32 = f32 ? h.A32.p : nullptr;
     a.l32 = f32 ? h.L32.p : nullptr;
     a.u32 = f32 ? h.U32.p : nullptr;
-    a.bad_row = h.d_bad.p;
-    a.nonfinite = h.d_nonfinite.p;
+    a.bad_row = h.d_words.p + WD_BAD;
+    a.nonfinite = h.d_words.p + WD_NONFINITE;
     a.id = next_factor_id(h);
     for (int c = 0; c < an.ncolours; ++c) {
         a.tile0 = h.A.colour_tile_wide[c];
         a.ntiles = h.A.colour_tile_wide[c + 1] - a.tile0;
-        a.adiag = c == 0 && an.ncolours > 1 ? h.A0d64.p : nullptr;
+        a.adiag = c == 0 && fuse_ordered(h) ? h.A0d64.p : nullptr;
         a.adiag32 = a.adiag && f32 ? h.A0d32.p : nullptr;
         hipLaunchKernelGGL((k_ilu0_tile<BS>), dim3(a.ntiles), dim3(64 * BS), 0, h.stream, a);
         check_launch();
     }
     gather_low2<BS>(h);
     if (f32) gather_low2_32<BS>(h);
-    hipLaunchKernelGGL(k_factor_end, dim3(1), dim3(1), 0, h.stream, h.d_bad.p, h.d_done + kBadRow);
+    hipLaunchKernelGGL(k_factor_end, dim3(1), dim3(1), 0, h.stream, h.d_words.p + WD_BAD, h.d_done + kBadRow);
     check_launch();
     HIP_CHECK(hipStreamSynchronize(h.stream));
     const int32_t bad = __atomic_load_n(h.h_done + kBadRow, __ATOMIC_ACQUIRE);
@@ -1879,7 +1889,7 @@ void load_factors(H &h, const double *lu_values, const double *dinv) {
     const int64_t nval = (int64_t)h.A.nnzb * BB;
     const int grid = (int)std::min<int64_t>(std::max<int64_t>(blocks_for(nval, 256), 1), 8192);
     hipLaunchKernelGGL(k_check_finite, dim3(grid), dim3(256), 0, h.stream, nval, (const double *)h.A64.p,
-                       h.d_nonfinite.p, next_factor_id(h));
+                       h.d_words.p + WD_NONFINITE, next_factor_id(h));
     check_launch();
     h.LU.ensure((size_t)nval);
     HIP_CHECK(hipMemcpyAsync(h.LU.p, lu_values, (size_t)nval * 8, hipMemcpyHostToDevice, h.stream));
@@ -1907,7 +1917,7 @@ void ensure_mixed(H &h) {
     gather_blocks<BS, float>(h, h.L.nnzb, nullptr, h.L64.p, h.L32.p, 0);
     gather_blocks<BS, float>(h, h.U.nnzb, nullptr, h.U64.p, h.U32.p, 0);
     gather_low2_32<BS>(h);
-    if (h.u0_is_a && h.an.ncolours > 1)
+    if (h.u0_is_a && fuse_ordered(h))
         gather_blocks<BS, float>(h, h.an.colour_ptr[1], nullptr, h.A0d64.p, h.A0d32.p, 0);
     HIP_CHECK(hipStreamSynchronize(h.stream));
     h.copies_gen = h.mixed_gen = h.factor_gen;
@@ -2438,7 +2448,7 @@ int bda_create(int32_t bs, int32_t n, int32_t nnzb_max, bda_handle *out) {
         HIP_CHECK(hipHostGetDevicePointer((void **)&h->d_host_st, h->h_st, 0));
         HIP_CHECK(hipHostMalloc((void **)&h->h_done, kFlags * sizeof(int32_t), hipHostMallocMapped));
         std::memset(h->h_done, 0, kFlags * sizeof(int32_t));
-        h->d_sweep.ensure(3);
+        h->d_words.ensure(WD_N);
         HIP_CHECK(hipHostGetDevicePointer((void **)&h->d_done, h->h_done, 0));
         HIP_CHECK(hipHostMalloc((void **)&h->h_prog, 2 * sizeof(uint64_t), hipHostMallocMapped));
         h->h_prog[0] = h->h_prog[1] = 0;
@@ -2460,10 +2470,10 @@ int bda_destroy(bda_handle h) {
     (void)hipSetDevice(h->device);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     for (DevMat *m : {&h->A, &h->L, &h->U, &h->At, &h->Ut, &h->Lt}) m->release();
-    for (DBuf<int32_t> *b : {&h->d_perm, &h->d_blkrow, &h->d_upd, &h->d_bad, &h->d_nonfinite, &h->d_full, &h->d_sweep}) b->release();
+    for (DBuf<int32_t> *b : {&h->d_perm, &h->d_blkrow, &h->d_upd, &h->d_words}) b->release();
     for (DBuf<double> *b : {&h->d_orig, &h->A64, &h->L64, &h->U64, &h->LU, &h->Dinv, &h->DinvT, &h->At64, &h->Ut64,
                             &h->Lt64, &h->A0d64, &h->low2_v64, &h->bp, &h->xo, &h->ro, &h->vin, &h->vout, &h->vw, &h->gl, &h->gx, &h->ggrad,
-                            &h->partials, &h->vparts})
+                            &h->partials})
         b->release();
     for (DBuf<float> *b : {&h->A32, &h->L32, &h->U32, &h->A0d32, &h->low2_v32, &h->At32, &h->Ut32, &h->Lt32}) b->release();
     h->k64.release();
