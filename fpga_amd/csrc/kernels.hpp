@@ -2192,17 +2192,20 @@ __global__ __launch_bounds__(256) void k_scatter_end(int n, int bs, const int32_
 }
 
 // dst block k = src block idx[k] (idx null: identity), optionally transposed
-// and converted (K17 demotion when TD = float).  A workgroup writes
-// kGatherUnroll * 256 consecutive entries, each thread entries 256 apart: all
-// its index loads are in flight together, then all its value loads.  With one
-// entry per thread and a 64-bit division for each, 6.0M 3x3 blocks took 211 us
-// (4.1 TB/s) and 24M 4x4 blocks 1520 us, the two dependent loads leaving too
-// few bytes in flight; now 171 (5.1 TB/s) and 1150 us (5.4 TB/s).
-constexpr int kGatherUnroll = 8;
-template <int BS, typename TD>
+// and converted (K17 demotion when TD = float).  A workgroup writes U * 256
+// consecutive entries, each thread entries 256 apart: all its index loads are
+// in flight together, then all its value loads.  With one entry per thread and
+// a 64-bit division for each, 6.0M 3x3 blocks took 211 us (4.1 TB/s) and 24M
+// 4x4 blocks 1520 us, the two dependent loads leaving too few bytes in flight;
+// with eight 171 (5.1 TB/s) and 1150 us (5.4 TB/s).  Below kGatherFrom entries
+// that leaves too few workgroups (3x3, one entry with the 64-bit division /
+// two / eight: 30k entries 4.6 / 4.4 / 5.6 us, 345k (4x4) 4.9 / 5.0 / 5.8, 0.9M
+// (4x4) 7.3 / 7.2 / 7.5, 1.0M 7.8 / 7.5 / 8.2, 1.8M 11.9 / 11.5 / 11.4): two there.
+constexpr int64_t kGatherFrom = 1 << 20;
+template <int BS, typename TD, int U>
 __global__ __launch_bounds__(256) void k_gather_blocks(int64_t nblk, const int32_t *idx, const double *src, TD *dst,
                                                        int trans) {
-    constexpr int BB = BS * BS, U = kGatherUnroll;
+    constexpr int BB = BS * BS;
     const int64_t i0 = (int64_t)blockIdx.x * (256 * U);
     const int64_t k0 = i0 / BB;
     const int rem = (int)(i0 - k0 * BB) + threadIdx.x;

@@ -1690,8 +1690,13 @@ template <int BS, typename TD>
 void gather_blocks(H &h, int64_t nblk, const int32_t *idx, const double *src, TD *dst, int trans) {
     if (nblk <= 0) return;
     const int64_t work = nblk * BS * BS;
-    hipLaunchKernelGGL((k_gather_blocks<BS, TD>), dim3(blocks_for(work, 256 * kGatherUnroll)), dim3(256), 0, h.stream, nblk, idx,
-                       src, dst, trans);
+    auto launch = [&](auto u) {
+        constexpr int U = decltype(u)::value;
+        hipLaunchKernelGGL((k_gather_blocks<BS, TD, U>), dim3(blocks_for(work, 256 * U)), dim3(256), 0, h.stream, nblk,
+                           idx, src, dst, trans);
+    };
+    if (work < kGatherFrom) launch(std::integral_constant<int, 2>{});
+    else launch(std::integral_constant<int, 8>{});
     check_launch();
 }
 
