@@ -1480,6 +1480,7 @@ void scatter_end(H &h, const double *x, const double *phat, double *d_x, const S
     HIP_CHECK(hipStreamSynchronize(h.stream));
     if (h.h_st->failed) {
         h.ev_used = 0;
+        h.last_solve_valid = false;  // (its residual and history are of no use)
         throw std::runtime_error("a sweep's wait did not end: the solve was given up");
     }
 }

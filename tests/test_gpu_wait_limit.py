@@ -43,6 +43,8 @@ def test_given_up_sweep(kind, bs):
         with pytest.raises(BdaError, match="wait did not end"):
             KINDS[kind](g, db.data_ptr(), dx.data_ptr())
         np.testing.assert_array_equal(dx.cpu().numpy(), x0)
+        with pytest.raises(BdaError, match="no solve has run"):
+            g.residual()
         with pytest.raises(BdaError, match="wait did not end"):
             getattr(g, kind.replace("_x64", ""))(b, x0, tol=1e-8)
         g.set_wait_limit()
